@@ -1438,7 +1438,7 @@ __device__ inline void repair_group_reg(const Rsi16Dev &T, uint16_t *m, uint16_t
     constexpr uint32_t PF = C >= 4 ? 1 : 4;
     PR<E> syn;
     const uint32_t nb = T.n / E;
-    if constexpr (SIN) {  // syndromes computed ahead (rsi16_synd_mfma_kernel)
+    if constexpr (SIN) {  // syndromes computed ahead (rsi16_contract_kernel)
 #pragma unroll
         for (int h = 0; h < C; ++h)
             syn.v[h] = syn_in[L.gl + (uint32_t)h * G];
@@ -1820,142 +1820,248 @@ __global__ __launch_bounds__(64) void rsi16_repair_known_kernel(uint16_t *__rest
         *status = FFRS_RSI16_REPAIR_OK;
 }
 
-// ---------------------------------------------------------------- encode as an int8 MFMA contraction
+// ---------------------------------------------------------------- linear maps as int8 MFMA contractions
 
 // The parity of a message is a fixed linear map of it mod p: parity_j = sum_m v_m G[m][j] mod p,
 // then & 0xFFFF (pyrsi16.hpp:128-140), with G[m] the encode of the unit message at m (the residue
 // NTT, mix and GS butterfly of rsi16v_impl.hpp:93-119 are linear). That holds for the scalar
 // words always, and for the SIMD words wherever no mix constant is 65536 (there a zero residue
-// reduces to p, and p * 65536 wraps to 65536 in 32 bits). This kernel evaluates the map exactly
-// on the 16x16x64 int8 matrix cores:
-//  - symbol v = v0 + 256 v1; the limbs enter as int8 v_a - 128 (the byte XOR 0x80);
-//  - G entry g = g0 + 128 g1 + 16384 g2 (g0, g1 < 128, g2 <= 4), three non-negative int8 limbs;
-//  - P_ab = sum_m (v_a[m] - 128) g_b[m][j] accumulates in int32 (|P| <= 128 * 127 * k);
-//  - value_j = sum_ab 256^a 128^b P_ab + K_j mod p, where K_j = 128 * 257 * sum_b 128^b C_b[j]
-//    (C_b[j] = sum_m g_b[m][j]) puts the offsets back; with 2^16 = -1 mod p every partial sum
-//    is folded as lo16 - hi16 before it can overflow.
-// One wave takes 16 codewords: B operand lane l = codeword l % 16, symbols 16 (l / 16) .. +16 of a
-// 64-symbol chunk; A operand = the matching G limbs of 16 parity rows; the C tile holds parity
-// rows 4 (l / 16) .. +4 of codeword l % 16. Symbols past k meet zero rows of G.
+// reduces to p, and p * 65536 wraps to 65536 in 32 bits). The syndromes of NTT::pntt
+// (ntt.hpp:133-152), S_j = sum over the n symbols of c_m w^(j rbo(m)) mod p, are another such map.
+// Both are evaluated exactly on the 16x16x64 int8 matrix cores:
+//  - symbol v = 256 v1 + v0; the bytes enter as int8, y_a = v_a - 128 (the byte XOR 0x80);
+//  - a matrix entry g = 256 g1 + g0 with two int8 limbs. They reach every residue mod p but one
+//    (32640: 256 * 127 + 127 = 32639, -256 * 128 - 128 = 32641 - p), so every output row j is
+//    scaled by an s_j for which s_j g meets that residue nowhere, and its sums by 1 / s_j;
+//  - with 2^16 = -1 mod p and -y1 = (y1 XOR 0xFF) + 1,
+//      v g = y0 g0 + (y1 XOR 0xFF) g1 + 256 (y1 g0 + y0 g1) + g1 + 128 * 257 g   (mod p),
+//    two int32 sums per output (P0 the first two products, P1 the bracket; |P| <= 2^15 k) and a
+//    constant K_j = sum_m (g1 + 128 * 257 g)[m][j], which P0 starts from;
+//  - value_j = (P0 + 256 P1) / s_j mod p, every step folded as lo16 - hi16 before it can overflow.
+// Operands of one MFMA: B lane l = codeword l % 16, symbols 16 (l / 16) .. +16 of a 64-symbol
+// chunk; A the matching limbs of 16 output rows; the C tile holds rows 4 (l / 16) .. +4 of codeword
+// l % 16. Symbols past the end of a chunked part meet zero rows of the matrix.
 typedef int v4i_t __attribute__((ext_vector_type(4)));
 
+struct MfmaTab {
+    const uint4 *pack;  // ((t nq + q) 2 + limb) 64 + lane: A operand of output tile t, chunk q
+    const int2 *row;    // {K_j, 1 / s_j (in [-32767, 32767])}
+    uint32_t nq, nq_m;  // 64-symbol chunks in all, of the message
+};
+
 // x - 65536 floor(x / 65536) - floor(x / 65536) = x mod p (up to a multiple of p), small enough
-// for the next step
+// for the next step; twice gives [-1, 65536]
 __device__ inline int32_t fold16(int32_t x) { return (x & 0xffff) - (x >> 16); }
 
-//
-// SYN: the same contraction gives the syndromes of NTT::pntt (ntt.hpp:133-152), S_j = sum over the
-// n symbols of c_m w^(j rbo(m)) mod p, with the chunks of the message (msgs, k per codeword)
-// followed by those of the parity (eccs, E per codeword, ecc_bytes in the buffer) against the
-// matching rows of that matrix (nq_m message chunks); the canonical values go to syn (u32).
-template <int CT, bool SYN>
-__device__ inline void mfma_contract(const uint16_t *__restrict__ msgs, uint32_t msg_bytes, uint32_t count,
-                                     uint16_t *__restrict__ out, const uint4 *__restrict__ gpack,
-                                     const uint32_t *__restrict__ kconst, uint32_t k, uint32_t E, uint32_t nq,
-                                     const uint16_t *__restrict__ eccs, uint32_t ecc_bytes, uint32_t nq_m,
-                                     uint32_t *__restrict__ syn)
+// (p0 + 256 p1) sinv mod p, canonical; |p0| < 2^30, |p1| < 2^30
+__device__ inline uint32_t contract_value(int32_t p0, int32_t p1, int32_t sinv)
 {
+    const int32_t f = fold16(fold16(p0 + 256 * fold16(p1)));
+    const int32_t r = fold16(fold16(f * sinv));  // |f sinv| <= 65536 * 32767
+    return (uint32_t)(r + ((r >> 31) & (int32_t)P16));
+}
+
+// The byte limbs of 16 symbols as B operands: low bytes and high bytes, XOR 0x80
+__device__ inline void contract_limbs(const uint4 &x0, const uint4 &x1, v4i_t &lo, v4i_t &hi)
+{
+    const uint32_t w[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        lo[i] = (int)(__builtin_amdgcn_perm(w[2 * i + 1], w[2 * i], 0x06040200u) ^ 0x80808080u);
+        hi[i] = (int)(__builtin_amdgcn_perm(w[2 * i + 1], w[2 * i], 0x07050301u) ^ 0x80808080u);
+    }
+}
+
+// acc[0] += lo g0 + ~hi g1, acc[1] += hi g0 + lo g1
+__device__ inline void contract_step(v4i_t acc[2], const v4i_t &g0, const v4i_t &g1, const v4i_t &lo, const v4i_t &hi,
+                                     const v4i_t &nhi)
+{
+    acc[0] = __builtin_amdgcn_mfma_i32_16x16x64_i8(g0, lo, acc[0], 0, 0, 0);
+    acc[1] = __builtin_amdgcn_mfma_i32_16x16x64_i8(g0, hi, acc[1], 0, 0, 0);
+    acc[0] = __builtin_amdgcn_mfma_i32_16x16x64_i8(g1, nhi, acc[0], 0, 0, 0);
+    acc[1] = __builtin_amdgcn_mfma_i32_16x16x64_i8(g1, lo, acc[1], 0, 0, 0);
+}
+
+__device__ inline v4i_t as_v4i(const uint4 &v) { return v4i_t{(int)v.x, (int)v.y, (int)v.z, (int)v.w}; }
+
+struct ContractIn {  // `count` codewords: message rows of k symbols and (syndromes) parity rows of E
+    __amdgpu_buffer_rsrc_t msg, ecc;
+    uint32_t k, E, nq_m;
+    // symbols 16 h .. +16 of chunk q of codeword cw: 32-byte aligned reads, wholly inside or wholly
+    // past the buffer
+    template <bool SYN>
+    __device__ void load(uint32_t cw, uint32_t q, uint32_t h, uint4 &x0, uint4 &x1) const
+    {
+        if (!SYN || q < nq_m) {
+            const uint32_t off = cw * k * 2 + (64 * q + 16 * h) * 2;
+            x0 = buf_load_u32x4(msg, off);
+            x1 = buf_load_u32x4(msg, off + 16);
+        } else {
+            const uint32_t off = cw * E * 2 + (64 * (q - nq_m) + 16 * h) * 2;
+            x0 = buf_load_u32x4(ecc, off);
+            x1 = buf_load_u32x4(ecc, off + 16);
+        }
+    }
+};
+
+// Output rows 16 t + 4 h .. +4 of codeword cw: parity symbols, or canonical syndromes (u32)
+template <bool SYN>
+__device__ inline void contract_store(const v4i_t acc[2], const MfmaTab &M, uint32_t t, uint32_t h, uint32_t cw,
+                                      uint32_t E, uint16_t *out, uint32_t *syn)
+{
+    const uint32_t j = 16 * t + 4 * h;
+    uint32_t v[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        v[i] = contract_value(acc[0][i], acc[1][i], M.row[j + i].y);
+    if constexpr (SYN)
+        *reinterpret_cast<uint4 *>(syn + (size_t)cw * E + j) = make_uint4(v[0], v[1], v[2], v[3]);
+    else
+        *reinterpret_cast<uint2 *>(out + (size_t)cw * E + j) =
+            make_uint2((v[0] & 0xffffu) | (v[1] << 16), (v[2] & 0xffffu) | (v[3] << 16));
+}
+
+// ecc_len 16 and 32: a wave takes CG groups of 16 codewords and every output tile; the matrix
+// (a few KB per chunk) comes from the caches. Bound by the codewords' HBM reads (rows of a few
+// hundred bytes): 262,144 RSi16(256,32) parities in 36 us (3.7 TB/s), 39 with three 7-bit limbs.
+template <int T, int CG, bool SYN>
+__global__ __launch_bounds__(256) void rsi16_contract_wave_kernel(const uint16_t *__restrict__ msgs, uint32_t msg_bytes,
+                                                                  const uint16_t *__restrict__ eccs, uint32_t ecc_bytes,
+                                                                  uint32_t count, MfmaTab M, uint32_t k,
+                                                                  uint16_t *__restrict__ out,
+                                                                  uint32_t *__restrict__ syn)
+{
+    constexpr uint32_t E = 16 * T;
     const uint32_t lane = threadIdx.x & 63, c = lane & 15, h = lane >> 4;
     const uint32_t wave = blockIdx.x * 4 + (threadIdx.x >> 6), waves = gridDim.x * 4;
-    const __amdgpu_buffer_rsrc_t rsrc = make_rsrc(msgs, msg_bytes);
-    const __amdgpu_buffer_rsrc_t rsrc_e = make_rsrc(SYN ? eccs : msgs, SYN ? ecc_bytes : msg_bytes);
-    const uint32_t T = E / 16;
-    for (uint32_t grp = wave; grp * 16 < count; grp += waves) {
-        const uint32_t cw = grp * 16 + c;
-        const bool valid = cw < count;
-        const uint32_t row = cw * k * 2;  // byte offset of the codeword's message (< 2^32: launches are split)
-        const uint32_t erow = cw * E * 2;
-        for (uint32_t t0 = 0; t0 < T; t0 += CT) {
-            v4i_t acc[CT][2][3];
+    const ContractIn in{make_rsrc(msgs, msg_bytes), make_rsrc(SYN ? eccs : msgs, SYN ? ecc_bytes : 0), k, E, M.nq_m};
+    for (uint32_t grp = wave; grp * 16 * CG < count; grp += waves) {
+        v4i_t acc[T][CG][2];
 #pragma unroll
-            for (int tt = 0; tt < CT; ++tt)
+        for (int t = 0; t < T; ++t)
 #pragma unroll
-                for (int a = 0; a < 2; ++a)
+            for (int g = 0; g < CG; ++g) {
 #pragma unroll
-                    for (int b = 0; b < 3; ++b)
-                        acc[tt][a][b] = v4i_t{0, 0, 0, 0};
-            for (uint32_t q = 0; q < nq; ++q) {
-                uint4 x0 = make_uint4(0, 0, 0, 0), x1 = x0;
-                if (valid) {  // 32-byte aligned reads, wholly inside or wholly past the buffer
-                    if (!SYN || q < nq_m) {
-                        const uint32_t off = row + (64 * q + 16 * h) * 2;
-                        x0 = buf_load_u32x4(rsrc, off);
-                        x1 = buf_load_u32x4(rsrc, off + 16);
-                    } else {
-                        const uint32_t off = erow + (64 * (q - nq_m) + 16 * h) * 2;
-                        x0 = buf_load_u32x4(rsrc_e, off);
-                        x1 = buf_load_u32x4(rsrc_e, off + 16);
-                    }
-                }
-                const v4i_t lo = {(int)(__builtin_amdgcn_perm(x0.y, x0.x, 0x06040200u) ^ 0x80808080u),
-                                  (int)(__builtin_amdgcn_perm(x0.w, x0.z, 0x06040200u) ^ 0x80808080u),
-                                  (int)(__builtin_amdgcn_perm(x1.y, x1.x, 0x06040200u) ^ 0x80808080u),
-                                  (int)(__builtin_amdgcn_perm(x1.w, x1.z, 0x06040200u) ^ 0x80808080u)};
-                const v4i_t hi = {(int)(__builtin_amdgcn_perm(x0.y, x0.x, 0x07050301u) ^ 0x80808080u),
-                                  (int)(__builtin_amdgcn_perm(x0.w, x0.z, 0x07050301u) ^ 0x80808080u),
-                                  (int)(__builtin_amdgcn_perm(x1.y, x1.x, 0x07050301u) ^ 0x80808080u),
-                                  (int)(__builtin_amdgcn_perm(x1.w, x1.z, 0x07050301u) ^ 0x80808080u)};
+                for (int i = 0; i < 4; ++i)
+                    acc[t][g][0][i] = M.row[16 * t + 4 * h + i].x;
+                acc[t][g][1] = v4i_t{0, 0, 0, 0};
+            }
+#pragma unroll 2
+        for (uint32_t q = 0; q < M.nq; ++q) {
+            uint4 x0[CG], x1[CG], a[T][2];
 #pragma unroll
-                for (int tt = 0; tt < CT; ++tt) {
-                    const uint32_t t = t0 + tt;
-#pragma unroll
-                    for (int b = 0; b < 3; ++b) {
-                        const uint4 g = gpack[((size_t)(b * T + t) * nq + q) * 64 + lane];
-                        const v4i_t A = {(int)g.x, (int)g.y, (int)g.z, (int)g.w};
-                        acc[tt][0][b] = __builtin_amdgcn_mfma_i32_16x16x64_i8(A, lo, acc[tt][0][b], 0, 0, 0);
-                        acc[tt][1][b] = __builtin_amdgcn_mfma_i32_16x16x64_i8(A, hi, acc[tt][1][b], 0, 0, 0);
-                    }
-                }
+            for (int g = 0; g < CG; ++g) {
+                const uint32_t cw = (grp * CG + g) * 16 + c;
+                in.load<SYN>(cw < count ? cw : count - 1, q, h, x0[g], x1[g]);
             }
 #pragma unroll
-            for (int tt = 0; tt < CT; ++tt) {
-                const uint32_t t = t0 + tt;
-                uint32_t v[4];
+            for (int t = 0; t < T; ++t)
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const uint32_t j = 16 * t + 4 * h + i;
-                    int32_t z[3];
+                for (int b = 0; b < 2; ++b)
+                    a[t][b] = M.pack[((t * M.nq + q) * 2 + b) * 64 + lane];
 #pragma unroll
-                    for (int b = 0; b < 3; ++b)
-                        z[b] = fold16(fold16(acc[tt][0][b][i]) + 256 * fold16(acc[tt][1][b][i]));
-                    int32_t f = fold16(z[0] + 128 * z[1] + 16384 * z[2] + (int32_t)kconst[j]);
-                    f = f < 0 ? f + (int32_t)P16 : f;
-                    f = f >= (int32_t)P16 ? f - (int32_t)P16 : f;
-                    v[i] = SYN ? (uint32_t)f : (uint32_t)f & 0xffffu;
-                }
-                if (valid) {
-                    if constexpr (SYN)
-                        *reinterpret_cast<uint4 *>(syn + (size_t)cw * E + 16 * t + 4 * h) =
-                            make_uint4(v[0], v[1], v[2], v[3]);
-                    else
-                        *reinterpret_cast<uint2 *>(out + (size_t)cw * E + 16 * t + 4 * h) =
-                            make_uint2(v[0] | (v[1] << 16), v[2] | (v[3] << 16));
-                }
+            for (int g = 0; g < CG; ++g) {
+                v4i_t lo, hi;
+                contract_limbs(x0[g], x1[g], lo, hi);
+                const v4i_t nhi = ~hi;
+#pragma unroll
+                for (int t = 0; t < T; ++t)
+                    contract_step(acc[t][g], as_v4i(a[t][0]), as_v4i(a[t][1]), lo, hi, nhi);
             }
+        }
+#pragma unroll
+        for (int g = 0; g < CG; ++g) {
+            const uint32_t cw = (grp * CG + g) * 16 + c;
+            if (cw < count)
+#pragma unroll
+                for (int t = 0; t < T; ++t)
+                    contract_store<SYN>(acc[t][g], M, t, h, cw, E, out, syn);
         }
     }
 }
 
-template <int CT>
-__global__ __launch_bounds__(256) void rsi16_encode_mfma_kernel(const uint16_t *__restrict__ msgs, uint32_t msg_bytes,
-                                                                uint32_t count, uint16_t *__restrict__ out,
-                                                                const uint4 *__restrict__ gpack,
-                                                                const uint32_t *__restrict__ kconst, uint32_t k,
-                                                                uint32_t E, uint32_t nq)
+// ecc_len 64 to 256: a workgroup of NW waves takes CG groups of 16 codewords and every output tile,
+// TPW of them per wave, so that the matrix is read once per 16 CG codewords; the codewords' limbs
+// go through LDS (double buffered, one barrier per chunk), loaded D chunks ahead by the first CG
+// waves, the matrix limbs D chunks ahead by the wave that uses them. 64 codewords per workgroup
+// (CG = 4) where that gives every CU one, 16 below. 16,384 RSi16(4096,256) parities in 72 us
+// (1.9 TB/s; the matrix cores need 26 at their peak), 168 with the butterflies in registers, 623
+// with the matrix read once per 16 codewords.
+template <int NW, int TPW, int CG, int D, bool SYN>
+__global__ __launch_bounds__(NW * 64) void rsi16_contract_kernel(const uint16_t *__restrict__ msgs, uint32_t msg_bytes,
+                                                                 const uint16_t *__restrict__ eccs, uint32_t ecc_bytes,
+                                                                 uint32_t count, MfmaTab M, uint32_t k,
+                                                                 uint16_t *__restrict__ out, uint32_t *__restrict__ syn)
 {
-    mfma_contract<CT, false>(msgs, msg_bytes, count, out, gpack, kconst, k, E, nq, nullptr, 0, 0, nullptr);
-}
-
-// The syndromes of NTT::pntt (ntt.hpp:133-152) as the same contraction (mfma_contract, SYN).
-template <int CT>
-__global__ __launch_bounds__(256) void rsi16_synd_mfma_kernel(const uint16_t *__restrict__ msgs, uint32_t msg_bytes,
-                                                              const uint16_t *__restrict__ eccs, uint32_t ecc_bytes,
-                                                              uint32_t count, const uint4 *__restrict__ vpack,
-                                                              const uint32_t *__restrict__ vconst, uint32_t k,
-                                                              uint32_t E, uint32_t nq, uint32_t nq_m,
-                                                              uint32_t *__restrict__ syn)
-{
-    mfma_contract<CT, true>(msgs, msg_bytes, count, nullptr, vpack, vconst, k, E, nq, eccs, ecc_bytes, nq_m, syn);
+    static_assert(CG <= NW, "one loading wave per group");
+    constexpr uint32_t E = 16 * NW * TPW;
+    __shared__ uint4 s_x[2][CG][2][64];
+    const uint32_t lane = threadIdx.x & 63, c = lane & 15, h = lane >> 4, wave = threadIdx.x >> 6;
+    const uint32_t cw0 = blockIdx.x * 16 * CG;
+    const ContractIn in{make_rsrc(msgs, msg_bytes), make_rsrc(SYN ? eccs : msgs, SYN ? ecc_bytes : 0), k, E, M.nq_m};
+    const bool loader = wave < CG;
+    const uint32_t mine = min(cw0 + wave * 16 + c, count - 1);
+    v4i_t acc[TPW][CG][2];
+#pragma unroll
+    for (int t = 0; t < TPW; ++t)
+#pragma unroll
+        for (int g = 0; g < CG; ++g) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                acc[t][g][0][i] = M.row[16 * (wave * TPW + t) + 4 * h + i].x;
+            acc[t][g][1] = v4i_t{0, 0, 0, 0};
+        }
+    uint4 a[D][TPW][2], x[D][2];
+    auto fetch = [&](int d, uint32_t q) {
+        if (q >= M.nq)
+            return;
+#pragma unroll
+        for (int t = 0; t < TPW; ++t)
+#pragma unroll
+            for (int b = 0; b < 2; ++b)
+                a[d][t][b] = M.pack[(((wave * TPW + t) * M.nq + q) * 2 + b) * 64 + lane];
+        if (loader)
+            in.load<SYN>(mine, q, h, x[d][0], x[d][1]);
+    };
+    auto stage = [&](int d, uint32_t q) {
+        if (loader && q < M.nq) {
+            v4i_t lo, hi;
+            contract_limbs(x[d][0], x[d][1], lo, hi);
+            s_x[q & 1][wave][0][lane] = make_uint4((uint32_t)lo[0], (uint32_t)lo[1], (uint32_t)lo[2], (uint32_t)lo[3]);
+            s_x[q & 1][wave][1][lane] = make_uint4((uint32_t)hi[0], (uint32_t)hi[1], (uint32_t)hi[2], (uint32_t)hi[3]);
+        }
+    };
+#pragma unroll
+    for (int d = 0; d < D; ++d)
+        fetch(d, d);
+    stage(0, 0);
+    __syncthreads();
+    for (uint32_t q0 = 0; q0 < M.nq; q0 += D) {
+#pragma unroll
+        for (int d = 0; d < D; ++d) {
+            const uint32_t q = q0 + d;
+            if (q >= M.nq)
+                break;
+            stage((d + 1) % D, q + 1);
+#pragma unroll
+            for (int g = 0; g < CG; ++g) {
+                const v4i_t lo = as_v4i(s_x[q & 1][g][0][lane]), hi = as_v4i(s_x[q & 1][g][1][lane]), nhi = ~hi;
+#pragma unroll
+                for (int t = 0; t < TPW; ++t)
+                    contract_step(acc[t][g], as_v4i(a[d][t][0]), as_v4i(a[d][t][1]), lo, hi, nhi);
+            }
+            fetch(d, q + D);
+            __syncthreads();
+        }
+    }
+#pragma unroll
+    for (int g = 0; g < CG; ++g) {
+        const uint32_t cw = cw0 + g * 16 + c;
+        if (cw < count)
+#pragma unroll
+            for (int t = 0; t < TPW; ++t)
+                contract_store<SYN>(acc[t][g], M, wave * TPW + t, h, cw, E, out, syn);
+    }
 }
 
 // ---------------------------------------------------------------- interleaved repair, SIMD words
@@ -2746,6 +2852,12 @@ __global__ __launch_bounds__(64) void rsi16_plan_kernel(uint16_t *__restrict__ m
 
 using namespace ffrs;
 
+// Tables of one contraction on the device (nq = 0: not built).
+struct ContractTab {
+    void *d = nullptr;
+    MfmaTab dev{};
+};
+
 struct ffrs_rsi16 {
     ffrs_ctx *ctx = nullptr;
     uint32_t n = 0, k = 0, E = 0, N = 0, nbits = 0, primitive = 0, root = 0;
@@ -2754,16 +2866,9 @@ struct ffrs_rsi16 {
     uint32_t g_enc = 0, g_rep = 0;  // lanes per codeword of the encode and repair kernels
     void *d_work = nullptr;          // workspace of the SIMD-word interleaved repair
     size_t work_size = 0;
-    // the encode as an int8 MFMA contraction (rsi16_encode_mfma_kernel), where it applies
-    uint4 *d_gpack = nullptr;        // G limbs in the A-operand lane layout
-    uint32_t *d_kconst = nullptr;    // K_j
-    uint32_t mfma_nq = 0;            // 64-symbol chunks of the message (0: no MFMA encode)
+    ContractTab enc, synd;           // the encode and the syndromes as int8 MFMA contractions
     bool mix_minus_one = false;      // a mix constant is 65536: the SIMD words are not the linear map
     int encode_mode = 0;             // 0 automatic, 1 butterflies, 2 MFMA wherever it applies
-    // the syndromes as the same contraction (rsi16_synd_mfma_kernel) ahead of the repair
-    uint4 *d_vpack = nullptr;        // limbs of w^(j rbo(m)), m < n, in the A-operand lane layout
-    uint32_t *d_vconst = nullptr;    // their offset constants
-    uint32_t synd_nq = 0, synd_nqm = 0;  // chunks in all, message chunks (0: not built)
     uint32_t *d_syn = nullptr;       // syndromes of the last repair launch
     size_t syn_size = 0;
     int repair_synd = 0;             // 0 automatic, 1 in the repair kernel, 2 MFMA ahead of it
@@ -2838,22 +2943,51 @@ int launch_encode_reg(ffrs_rsi16 *rs, const uint16_t *d_msg, size_t count, uint1
     return FFRS_OK;
 }
 
-// The MFMA contraction over `count` codewords, in launches of < 2^31 message bytes.
+// Codewords per launch of a contraction: < 2^31 message bytes, a multiple of 64.
+size_t contract_step_count(const ffrs_rsi16 *rs)
+{
+    return std::max<size_t>(64, (((size_t)1 << 31) / (rs->k * 2)) & ~(size_t)63);
+}
+
+// One launch of a contraction (count <= contract_step_count) for ecc_len E.
+template <int E, bool SYN>
+int launch_contract(ffrs_rsi16 *rs, const MfmaTab &M, const uint16_t *d_msg, const uint16_t *d_ecc, size_t count,
+                    uint16_t *d_out, uint32_t *d_syn)
+{
+    const uint32_t mb = (uint32_t)(count * rs->k * 2), eb = (uint32_t)(count * E * 2);
+    if constexpr (E <= 32) {
+        const size_t groups = (count + 15) / 16;
+        hipLaunchKernelGGL((rsi16_contract_wave_kernel<E / 16, 1, SYN>),
+                           dim3(persistent_grid(rs->ctx, 8, (groups + 3) / 4)), dim3(256), 0, rs->ctx->stream, d_msg,
+                           mb, d_ecc, eb, (uint32_t)count, M, rs->k, d_out, d_syn);
+    } else {
+        constexpr int NW = E == 64 ? 4 : 8, TPW = E / 16 / NW;
+        if ((count + 63) / 64 >= (size_t)rs->ctx->cu_count)
+            hipLaunchKernelGGL((rsi16_contract_kernel<NW, TPW, 4, 3, SYN>), dim3((unsigned)((count + 63) / 64)),
+                               dim3(NW * 64), 0, rs->ctx->stream, d_msg, mb, d_ecc, eb, (uint32_t)count, M, rs->k, d_out,
+                               d_syn);
+        else
+            hipLaunchKernelGGL((rsi16_contract_kernel<NW, TPW, 1, 4, SYN>), dim3((unsigned)((count + 15) / 16)),
+                               dim3(NW * 64), 0, rs->ctx->stream, d_msg, mb, d_ecc, eb, (uint32_t)count, M, rs->k, d_out,
+                               d_syn);
+    }
+    FFRS_HIP(hipGetLastError());
+    return FFRS_OK;
+}
+
+// The encode as a contraction, in launches of < 2^31 message bytes.
 int launch_encode_mfma(ffrs_rsi16 *rs, const uint16_t *d_msg, size_t count, uint16_t *d_ecc)
 {
-    const size_t k = rs->k, E = rs->E;
-    const size_t step = std::max<size_t>(16, (((size_t)1 << 31) / (k * 2)) & ~(size_t)15);
-    auto *kern = E == 16 ? rsi16_encode_mfma_kernel<1> : E == 32 ? rsi16_encode_mfma_kernel<2>
-                                                                 : rsi16_encode_mfma_kernel<4>;
-    for (size_t b = 0; b < count; b += step) {
-        const size_t c = std::min(step, count - b);
-        const size_t groups = (c + 15) / 16;
-        const int grid = persistent_grid(rs->ctx, 8, (groups + 3) / 4);
-        hipLaunchKernelGGL(kern, dim3(grid), dim3(256), 0, rs->ctx->stream, d_msg + b * k, (uint32_t)(c * k * 2),
-                           (uint32_t)c, d_ecc + b * E, (const uint4 *)rs->d_gpack, (const uint32_t *)rs->d_kconst,
-                           (uint32_t)k, (uint32_t)E, rs->mfma_nq);
-        FFRS_HIP(hipGetLastError());
-    }
+    const size_t step = contract_step_count(rs);
+    auto *f = rs->E == 16    ? launch_contract<16, false>
+              : rs->E == 32  ? launch_contract<32, false>
+              : rs->E == 64  ? launch_contract<64, false>
+              : rs->E == 128 ? launch_contract<128, false>
+                             : launch_contract<256, false>;
+    for (size_t b = 0; b < count; b += step)
+        if (int r = f(rs, rs->enc.dev, d_msg + b * rs->k, nullptr, std::min(step, count - b), d_ecc + b * rs->E,
+                      nullptr))
+            return r;
     mark_kernel(rs->ctx);
     return FFRS_OK;
 }
@@ -2863,9 +2997,8 @@ int launch_encode(ffrs_rsi16 *rs, const uint16_t *d_msg, size_t count, uint16_t 
     marks_begin(rs->ctx);
     if (count == 0)
         return FFRS_OK;
-    // the linear map on the matrix cores where it is the encode of the words asked for (and,
-    // automatically, where it is measured faster than the butterflies: ecc_len <= 32)
-    if (rs->mfma_nq && I == 1 && rs->encode_mode != 1 && (rs->encode_mode == 2 || rs->E <= 32) &&
+    // the linear map on the matrix cores where it is the encode of the words asked for
+    if (rs->enc.dev.nq && I == 1 && rs->encode_mode != 1 &&
         !(vec && rs->mix_minus_one) && (((uintptr_t)d_msg | (uintptr_t)d_ecc) & 15) == 0)
         return launch_encode_mfma(rs, d_msg, count, d_ecc);
     // one lane per codeword (g = 1): the register kernel for ecc_len <= 32, plain layout
@@ -2916,10 +3049,10 @@ int launch_repair_reg(ffrs_rsi16 *rs, uint16_t *d_msg, uint16_t *d_ecc, size_t c
 {
     constexpr uint32_t cpw = 64 / RegShape<E>::G;
     const size_t lds = (size_t)cpw * REG_WORDS * E * 4;
-    // the syndromes on the matrix cores first, where their tables exist (ecc 16, 32, 64)
-    const bool msyn = rs->synd_nq && rs->repair_synd != 1 && (((uintptr_t)d_msg | (uintptr_t)d_ecc) & 15) == 0;
+    // the syndromes on the matrix cores first, where their tables exist
+    const bool msyn = rs->synd.dev.nq && rs->repair_synd != 1 && (((uintptr_t)d_msg | (uintptr_t)d_ecc) & 15) == 0;
     if (msyn) {
-        const size_t step = std::max<size_t>(16, (((size_t)1 << 31) / (rs->k * 2)) & ~(size_t)15);
+        const size_t step = contract_step_count(rs);
         const size_t need = std::min(count, step) * E * 4;
         if (rs->syn_size < need) {
             if (rs->d_syn)
@@ -2931,19 +3064,14 @@ int launch_repair_reg(ffrs_rsi16 *rs, uint16_t *d_msg, uint16_t *d_ecc, size_t c
                 return fail(FFRS_ERR_NOMEM, "syndrome workspace of %zu bytes: %s", need, hipGetErrorString(e));
             rs->syn_size = need;
         }
-        constexpr int CT = E >= 16 && E <= 64 ? E / 16 : 1;  // every tile in one pass (tables: ecc 16 .. 64)
-        auto *ks = rsi16_synd_mfma_kernel<CT>;
         if (int r = allow_lds(rsi16_repair_reg_kernel<E, true>, lds))
             return r;
         for (size_t b = 0; b < count; b += step) {
             const size_t c = std::min(step, count - b);
-            const size_t groups = (c + 15) / 16;
-            hipLaunchKernelGGL(ks, dim3(persistent_grid(rs->ctx, 8, (groups + 3) / 4)), dim3(256), 0, rs->ctx->stream,
-                               (const uint16_t *)(d_msg + b * rs->k), (uint32_t)(c * rs->k * 2),
-                               (const uint16_t *)(d_ecc + b * E), (uint32_t)(c * E * 2), (uint32_t)c,
-                               (const uint4 *)rs->d_vpack, (const uint32_t *)rs->d_vconst, rs->k, (uint32_t)E,
-                               rs->synd_nq, rs->synd_nqm, rs->d_syn);
-            FFRS_HIP(hipGetLastError());
+            if constexpr (E >= 16)
+                if (int r = launch_contract<E, true>(rs, rs->synd.dev, d_msg + b * rs->k, d_ecc + b * E, c, nullptr,
+                                                     rs->d_syn))
+                    return r;
             mark_kernel(rs->ctx);
             hipLaunchKernelGGL((rsi16_repair_reg_kernel<E, true>), dim3((unsigned)((c + cpw - 1) / cpw)), dim3(64), lds,
                                rs->ctx->stream, d_msg + b * rs->k, d_ecc + b * E, (uint32_t)c, d_status + b, rs->dev,
@@ -3015,114 +3143,99 @@ void gs_host(const std::vector<uint32_t> &roots, uint32_t *x, uint32_t len)
             }
 }
 
-// The tables of rsi16_encode_mfma_kernel: G[m] = the parity of the unit message at m, i.e. the GS
-// butterfly of mix_i X_m^i with X_m = w^rbo(m) (the message residue of rsi16v_impl.hpp:93-97 is
-// sum_m v_m X_m^i, then :108-119), split into three 7-bit limbs and packed in the A-operand
-// lane order, and K_j. Shapes with ecc_len not a multiple of 16, above 256, or message_len above
-// 16384 keep the butterfly kernels.
+// Uploads a contraction's tables: `mat` holds its nq * 64 rows of E canonical entries (zero rows
+// where no symbol enters), nq_m chunks of them for the message.
+int build_contract(ContractTab *tab, const std::vector<uint32_t> &mat, uint32_t E, uint32_t nq, uint32_t nq_m)
+{
+    const uint32_t T = E / 16, rows = nq * 64;
+    std::vector<uint8_t> pack((size_t)T * nq * 2 * 64 * 16);
+    std::vector<int32_t> row((size_t)E * 2);
+    std::vector<uint8_t> seen(P16);
+    const uint32_t third = s_pow(3, 65535);
+    for (uint32_t j = 0; j < E; ++j) {
+        std::fill(seen.begin(), seen.end(), 0);
+        for (uint32_t m = 0; m < rows; ++m)
+            seen[mat[(size_t)m * E + j]] = 1;
+        // the first power of 3 that moves no entry onto 32640 and whose inverse is not +-32768
+        uint32_t s = 1, si = 1, tries = 0;
+        while (seen[S::mul(32640, si)] || si == 32768 || si == P16 - 32768) {
+            if (++tries == 65536)
+                return FFRS_OK;  // no such scale: the butterflies stay
+            s = S::mul(s, 3);
+            si = S::mul(si, third);
+        }
+        uint64_t K = 0;
+        for (uint32_t m = 0; m < rows; ++m) {
+            const uint32_t g = S::mul(s, mat[(size_t)m * E + j]);
+            const int32_t v = g > 32639 ? (int32_t)g - (int32_t)P16 : (int32_t)g;
+            const int32_t lo = ((v + 128) & 255) - 128, hi = (v - lo) >> 8;
+            K += (uint64_t)((int64_t)g * 32896 + hi + (int64_t)P16);
+            const uint32_t q = m / 64, lane = j % 16 + 16 * (m % 64 / 16), bt = m % 16;
+            uint8_t *p = &pack[((((size_t)(j / 16) * nq + q) * 2) * 64 + lane) * 16 + bt];
+            p[0] = (uint8_t)lo;
+            p[64 * 16] = (uint8_t)hi;
+        }
+        row[2 * j] = (int32_t)(K % P16);
+        row[2 * j + 1] = si > 32768 ? (int32_t)si - (int32_t)P16 : (int32_t)si;
+    }
+    char *d = nullptr;
+    hipError_t e = hipMalloc(&d, pack.size() + row.size() * 4);
+    if (e == hipSuccess) {
+        tab->d = d;
+        e = hipMemcpy(d, pack.data(), pack.size(), hipMemcpyHostToDevice);
+    }
+    if (e == hipSuccess)
+        e = hipMemcpy(d + pack.size(), row.data(), row.size() * 4, hipMemcpyHostToDevice);
+    if (e != hipSuccess)
+        return fail(FFRS_ERR_DEVICE, "MFMA contraction tables: %s", hipGetErrorString(e));
+    tab->dev = MfmaTab{(const uint4 *)d, (const int2 *)(d + pack.size()), nq, nq_m};
+    return FFRS_OK;
+}
+
+// The encode's matrix: G[m] = the parity of the unit message at m, i.e. the GS butterfly of
+// mix_i X_m^i with X_m = w^rbo(m) (the message residue of rsi16v_impl.hpp:93-97 is
+// sum_m v_m X_m^i, then :108-119). Shapes with ecc_len not a multiple of 16, above 256, or
+// message_len above 16384 keep the butterfly kernels.
 int build_mfma_encode(ffrs_rsi16 *rs, const std::vector<uint32_t> &mix, const std::vector<uint32_t> &roots_i_ecc,
                       const std::vector<uint32_t> &roots_ntt)
 {
     const uint32_t k = rs->k, E = rs->E;
     if (E % 16 || E > 256 || k > 16384)
         return FFRS_OK;
-    const uint32_t nq = (k + 63) / 64, T = E / 16, kp = nq * 64;
-    std::vector<uint8_t> limb((size_t)3 * kp * E, 0);  // [b][m][j]
-    std::vector<uint64_t> C((size_t)3 * E, 0);
-    std::vector<uint32_t> row(E);
+    const uint32_t nq = (k + 63) / 64;
+    std::vector<uint32_t> mat((size_t)nq * 64 * E, 0);
     for (uint32_t m = 0; m < k; ++m) {
         const uint32_t x = roots_ntt[rbo_bits(m, rs->nbits)];
+        uint32_t *row = &mat[(size_t)m * E];
         uint32_t pw = 1;
         for (uint32_t i = 0; i < E; ++i) {
             row[i] = S::mul(mix[i], pw);
             pw = S::mul(pw, x);
         }
-        gs_host(roots_i_ecc, row.data(), E);
-        for (uint32_t j = 0; j < E; ++j) {
-            const uint32_t g = row[j], gb[3] = {g & 127u, (g >> 7) & 127u, g >> 14};
-            for (int b = 0; b < 3; ++b) {
-                limb[((size_t)b * kp + m) * E + j] = (uint8_t)gb[b];
-                C[(size_t)b * E + j] += gb[b];
-            }
-        }
+        gs_host(roots_i_ecc, row, E);
     }
-    std::vector<uint8_t> pack((size_t)3 * T * nq * 64 * 16);
-    for (uint32_t b = 0; b < 3; ++b)
-        for (uint32_t t = 0; t < T; ++t)
-            for (uint32_t q = 0; q < nq; ++q)
-                for (uint32_t l = 0; l < 64; ++l)
-                    for (uint32_t bt = 0; bt < 16; ++bt) {
-                        const uint32_t m = 64 * q + 16 * (l / 16) + bt, j = 16 * t + l % 16;
-                        pack[(((size_t)(b * T + t) * nq + q) * 64 + l) * 16 + bt] = limb[((size_t)b * kp + m) * E + j];
-                    }
-    std::vector<uint32_t> K(E);
-    for (uint32_t j = 0; j < E; ++j) {
-        const uint64_t sum = (C[j] + 128 * C[E + j] + 16384 * C[2 * (size_t)E + j]) % P16;
-        K[j] = (uint32_t)(sum * 128 % P16 * 257 % P16);
-    }
-    hipError_t e = hipMalloc(&rs->d_gpack, pack.size());
-    if (e == hipSuccess)
-        e = hipMalloc(&rs->d_kconst, K.size() * 4);
-    if (e == hipSuccess)
-        e = hipMemcpy(rs->d_gpack, pack.data(), pack.size(), hipMemcpyHostToDevice);
-    if (e == hipSuccess)
-        e = hipMemcpy(rs->d_kconst, K.data(), K.size() * 4, hipMemcpyHostToDevice);
-    if (e != hipSuccess)
-        return fail(FFRS_ERR_DEVICE, "MFMA encode tables: %s", hipGetErrorString(e));
-    rs->mfma_nq = nq;
-    return FFRS_OK;
+    return build_contract(&rs->enc, mat, E, nq, nq);
 }
 
-// The syndrome matrix V[m][j] = w^(j rbo(m)) (NTT::pntt, ntt.hpp:133-152) for the MFMA
-// contraction: rows m < k in ceil(k / 64) message chunks, rows k + i (i < E) in the parity
-// chunks after them, packed and offset as build_mfma_encode does.
+// The syndrome matrix w^(j rbo(m)) (NTT::pntt, ntt.hpp:133-152): rows m < k in ceil(k / 64) message
+// chunks, rows k + i (i < E) in the parity chunks after them.
 int build_mfma_synd(ffrs_rsi16 *rs, const std::vector<uint32_t> &roots_ntt)
 {
     const uint32_t k = rs->k, E = rs->E;
-    if (E % 16 || E > 64 || k > 16384)
+    if (E % 16 || E > 256 || k > 16384)
         return FFRS_OK;
-    const uint32_t nqm = (k + 63) / 64, nqe = (E + 63) / 64, nq = nqm + nqe, T = E / 16, kp = nq * 64;
-    std::vector<uint8_t> limb((size_t)3 * kp * E, 0);  // [b][row][j], rows in chunk order
-    std::vector<uint64_t> C((size_t)3 * E, 0);
+    const uint32_t nqm = (k + 63) / 64, nq = nqm + (E + 63) / 64;
+    std::vector<uint32_t> mat((size_t)nq * 64 * E, 0);
     for (uint32_t m = 0; m < k + E; ++m) {
-        const uint32_t r = m < k ? m : nqm * 64 + (m - k);  // row of the packed matrix
         const uint32_t x = roots_ntt[rbo_bits(m, rs->nbits)];
+        uint32_t *row = &mat[(size_t)(m < k ? m : nqm * 64 + (m - k)) * E];
         uint32_t pw = 1;
         for (uint32_t j = 0; j < E; ++j) {
-            const uint32_t g = pw, gb[3] = {g & 127u, (g >> 7) & 127u, g >> 14};
-            for (int b = 0; b < 3; ++b) {
-                limb[((size_t)b * kp + r) * E + j] = (uint8_t)gb[b];
-                C[(size_t)b * E + j] += gb[b];
-            }
+            row[j] = pw;
             pw = S::mul(pw, x);
         }
     }
-    std::vector<uint8_t> pack((size_t)3 * T * nq * 64 * 16);
-    for (uint32_t b = 0; b < 3; ++b)
-        for (uint32_t t = 0; t < T; ++t)
-            for (uint32_t q = 0; q < nq; ++q)
-                for (uint32_t l = 0; l < 64; ++l)
-                    for (uint32_t bt = 0; bt < 16; ++bt) {
-                        const uint32_t m = 64 * q + 16 * (l / 16) + bt, j = 16 * t + l % 16;
-                        pack[(((size_t)(b * T + t) * nq + q) * 64 + l) * 16 + bt] = limb[((size_t)b * kp + m) * E + j];
-                    }
-    std::vector<uint32_t> K(E);
-    for (uint32_t j = 0; j < E; ++j) {
-        const uint64_t sum = (C[j] + 128 * C[E + j] + 16384 * C[2 * (size_t)E + j]) % P16;
-        K[j] = (uint32_t)(sum * 128 % P16 * 257 % P16);
-    }
-    hipError_t e = hipMalloc(&rs->d_vpack, pack.size());
-    if (e == hipSuccess)
-        e = hipMalloc(&rs->d_vconst, K.size() * 4);
-    if (e == hipSuccess)
-        e = hipMemcpy(rs->d_vpack, pack.data(), pack.size(), hipMemcpyHostToDevice);
-    if (e == hipSuccess)
-        e = hipMemcpy(rs->d_vconst, K.data(), K.size() * 4, hipMemcpyHostToDevice);
-    if (e != hipSuccess)
-        return fail(FFRS_ERR_DEVICE, "MFMA syndrome tables: %s", hipGetErrorString(e));
-    rs->synd_nq = nq;
-    rs->synd_nqm = nqm;
-    return FFRS_OK;
+    return build_contract(&rs->synd, mat, E, nq, nqm);
 }
 
 }  // namespace
@@ -3298,14 +3411,9 @@ void ffrs_rsi16_destroy(ffrs_rsi16 *rs)
         (void)hipFree(rs->d_tables);
     if (rs->d_work)
         (void)hipFree(rs->d_work);
-    if (rs->d_gpack)
-        (void)hipFree(rs->d_gpack);
-    if (rs->d_kconst)
-        (void)hipFree(rs->d_kconst);
-    if (rs->d_vpack)
-        (void)hipFree(rs->d_vpack);
-    if (rs->d_vconst)
-        (void)hipFree(rs->d_vconst);
+    for (ContractTab *c : {&rs->enc, &rs->synd})
+        if (c->d)
+            (void)hipFree(c->d);
     if (rs->d_syn)
         (void)hipFree(rs->d_syn);
     delete rs;
