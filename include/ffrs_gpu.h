@@ -156,15 +156,16 @@ int ffrs_rsi16_set_groups(ffrs_rsi16 *rs, unsigned g_encode, unsigned g_repair);
 int ffrs_rsi16_get_groups(const ffrs_rsi16 *rs, unsigned *g_encode, unsigned *g_repair);
 /* Encode kernels (no counterpart in the reference; results do not depend on them). The int8
  * MFMA contraction parity = message . G mod p applies where it is the encode of the words asked
- * for: interleave 1, ecc_len a multiple of 16 up to 256, message_len <= 16384, 16-byte aligned
+ * for: interleave 1, ecc_len 8 or a multiple of 16 up to 256, message_len <= 16384, 16-byte aligned
  * buffers, and with the SIMD words only where no mix constant of rsi16v_impl.hpp:68-86 is 65536.
  * 0 automatic (the contraction where it applies, else the butterfly kernels), 1 always the
  * butterfly kernels, 2 the contraction wherever it applies. */
 int ffrs_rsi16_set_encode_kernel(ffrs_rsi16 *rs, int kernel);
 /* Where the repair computes its syndromes (no counterpart in the reference; results do not
- * depend on it): 0 automatic, 1 inside the repair kernel, 2 as an int8 MFMA contraction of the
- * codewords with the matrix w^(j rbo(m)) ahead of it, where its tables exist (ecc_len a multiple
- * of 16 up to 256, message_len <= 16384; automatic uses it there). */
+ * depend on it): 0 automatic, 1 inside the general repair kernel, 2 as an int8 MFMA contraction of
+ * the codewords with the matrix w^(j rbo(m)) ahead of it, where its tables exist (ecc_len 8 or a
+ * multiple of 16 up to 256, message_len <= 16384, 16-byte aligned buffers); for ecc_len 8 to 32 that
+ * is followed by the one-codeword-per-lane kernel. Automatic picks by ecc_len and count. */
 int ffrs_rsi16_set_repair_syndromes(ffrs_rsi16 *rs, int mode);
 uint32_t ffrs_rsi16_root(const ffrs_rsi16 *rs);
 size_t ffrs_rsi16_ntt_len(const ffrs_rsi16 *rs);

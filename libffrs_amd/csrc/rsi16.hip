@@ -1380,6 +1380,59 @@ __device__ inline uint32_t pr_sugiyama(const Rsi16Dev &T, PR<E> &a1, PR<E> &r1, 
                     t.v[h] = F::fold3(a2.v[h], F::part(n0, a1.v[h]), F::part(n1, pa.v[h]));
                     rn.v[h] = F::fold3(r2.v[h], F::part(n0, r1.v[h]), F::part(n1, pr.v[h]));
                 }
+            } else if (f_len < g_len) {  // a zero quotient: the pair changes places
+                h1 = r1h;
+                carried = false;
+                q_len = 0;
+                t = a2;
+                rn = r2;
+            } else if (E >= 8 && f_len == g_len + 2) {
+                // q_len == 3 (g_len <= E - 2): the same in coefficients. reverse_ntt gives v[j] =
+                // r1[g_len - 1 - j mod E]; the Newton loop's one round a = a0 + c1 x with
+                // c1 = -a0^2 v[1] (v[0] = r1h = 1 / a0), and the last one coefficients 0 .. 2 of
+                // a (2 - a v) mod x^E - 1, reversed; times (f - f0), the quotient as before. After one
+                // such step the reference's lengths alternate between this case and the one above,
+                // and the transforms took most of the time of a codeword that came here.
+                q_len = 3;
+                h1 = r1h;
+                carried = false;
+                const uint32_t a0 = T.inv_tab[r1h];
+                uint32_t v[5];  // v[j + 2]: j = -2 .. 2
+#pragma unroll
+                for (int j = -2; j <= 2; ++j)
+                    v[j + 2] = pr_get<E>(r1, (g_len - 1 - (uint32_t)j) & mask, L);
+                const uint32_t c1 = F::sub(0, F::mul(F::mul(a0, a0), v[3]));
+                uint32_t hh[4], ai[3];  // hh[j + 1] = (2 - a v)[j], j = -1 .. 2
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    hh[j] = F::sub(j == 1 ? 2u : 0u, F::add(F::mul(a0, v[j + 1]), F::mul(c1, v[j])));
+#pragma unroll
+                for (int j = 0; j < 3; ++j)
+                    ai[2 - j] = F::add(F::mul(a0, hh[j + 1]), F::mul(c1, hh[j]));
+                const uint32_t right_n = (uint32_t)E - g_len < 3 ? (uint32_t)E - g_len : 3u;
+                uint32_t q[3];
+#pragma unroll
+                for (uint32_t i = 0; i < 3; ++i) {
+                    const uint32_t at = i < right_n ? g_len + i : i - right_n;
+                    uint32_t s = 0;
+#pragma unroll
+                    for (uint32_t u = 0; u < 3; ++u) {
+                        const uint32_t k = (at - u) & mask;
+                        uint32_t x = pr_get<E>(r2, k, L);
+                        x = k == 0 ? F::sub(x, r2l) : x;
+                        s = F::add(s, F::mul(ai[u], x));
+                    }
+                    q[i] = s;
+                }
+                const PR<E> pa = pr_prev<E>(a1, L), pr = pr_prev<E>(r1, L);
+                const PR<E> pa2 = pr_prev<E>(pa, L), pr2 = pr_prev<E>(pr, L);
+#pragma unroll
+                for (int h = 0; h < C; ++h) {
+                    t.v[h] = F::sub(a2.v[h], F::add(F::mul(q[0], a1.v[h]),
+                                                    F::add(F::mul(q[1], pa.v[h]), F::mul(q[2], pa2.v[h]))));
+                    rn.v[h] = F::sub(r2.v[h], F::add(F::mul(q[0], r1.v[h]),
+                                                     F::add(F::mul(q[1], pr.v[h]), F::mul(q[2], pr2.v[h]))));
+                }
             } else {  // through the transforms
                 h1 = r1h;
                 carried = false;  // r1[g_len - 2] is not read on this path
@@ -1427,12 +1480,17 @@ __device__ inline uint32_t pr_sugiyama(const Rsi16Dev &T, PR<E> &a1, PR<E> &r1, 
 // and derivative copies for Forney, the root list and its count).
 constexpr uint32_t REG_WORDS = 4;
 
-template <int E, bool SIN = false>
+// WAVE: the 64 / G groups of the wave serve one codeword: they take the chunks of the syndromes and
+// of the root search in turn and the roots by lane, and solve the key equation each for itself.
+template <int E, bool SIN = false, bool WAVE = false>
 __device__ inline void repair_group_reg(const Rsi16Dev &T, uint16_t *m, uint16_t *e, uint32_t *base, const LaneR<E> &L,
                                         uint8_t *st, const uint32_t *syn_in = nullptr)
 {
     constexpr uint32_t G = RegShape<E>::G;
     constexpr int C = RegShape<E>::C;
+    constexpr uint32_t NG = WAVE ? 64 / G : 1;             // groups on the codeword
+    const uint32_t gi = WAVE ? L.lane / G : 0;             // this group
+    const uint32_t first = WAVE ? L.lane : L.gl;           // this lane among theirs
     // NTT::pntt (ntt.hpp:133-152) of m || e, one chunk of E symbols at a time; the symbols
     // and shifts of PF chunks are loaded before any is transformed, so their latencies overlap
     constexpr uint32_t PF = C >= 4 ? 1 : 4;
@@ -1443,7 +1501,11 @@ __device__ inline void repair_group_reg(const Rsi16Dev &T, uint16_t *m, uint16_t
         for (int h = 0; h < C; ++h)
             syn.v[h] = syn_in[L.gl + (uint32_t)h * G];
     }
-    for (uint32_t c0 = 0; !SIN && c0 < nb; c0 += PF) {
+    if constexpr (!SIN && WAVE)
+#pragma unroll
+        for (int h = 0; h < C; ++h)
+            syn.v[h] = 0;
+    for (uint32_t c0 = gi * PF; !SIN && c0 < nb; c0 += NG * PF) {
         PR<E> x[PF], sh[PF];
 #pragma unroll
         for (uint32_t u = 0; u < PF; ++u)
@@ -1462,19 +1524,25 @@ __device__ inline void repair_group_reg(const Rsi16Dev &T, uint16_t *m, uint16_t
 #pragma unroll
                 for (int h = 0; h < C; ++h) {
                     const uint32_t v = F::mul(x[u].v[h], sh[u].v[h]);
-                    syn.v[h] = c0 + u ? F::add(syn.v[h], v) : v;
+                    syn.v[h] = WAVE || c0 + u ? F::add(syn.v[h], v) : v;
                 }
             }
     }
+    if constexpr (!SIN && WAVE)
+#pragma unroll
+        for (uint32_t s = G; s < 64; s <<= 1)
+#pragma unroll
+            for (int h = 0; h < C; ++h)
+                syn.v[h] = F::add(syn.v[h], lane_read(syn.v[h], L.lane ^ s));
     if (pr_len<E>(syn, E, L) == 0) {
-        if (L.gl == 0)
+        if (first == 0)
             *st = FFRS_RSI16_NO_ERRORS;
         return;
     }
     PR<E> loc;
     const uint32_t Ln = pr_sugiyama<E>(T, loc, syn, L);
     if (Ln == 0xffffffffu) {
-        if (L.gl == 0)
+        if (first == 0)
             *st = FFRS_RSI16_RAISES;
         return;
     }
@@ -1489,7 +1557,7 @@ __device__ inline void repair_group_reg(const Rsi16Dev &T, uint16_t *m, uint16_t
     }
     const uint32_t der_len = pr_len<E>(der, E, L);
     if (Ln > (uint32_t)E) {  // py_assert at rsi16v_impl.hpp:454
-        if (L.gl == 0)
+        if (first == 0)
             *st = FFRS_RSI16_RAISES;
         return;
     }
@@ -1502,12 +1570,12 @@ __device__ inline void repair_group_reg(const Rsi16Dev &T, uint16_t *m, uint16_t
         ev[L.gl + (uint32_t)h * G] = syn.v[h];
         dv[L.gl + (uint32_t)h * G] = der.v[h];
     }
-    if (L.gl == 0)
+    if (first == 0)
         *nroots = 0;
     wave_sync();
     // NTT::pintt_ecc (ntt.hpp:206-220) chunk by chunk, shifts of PF chunks loaded ahead;
     // zeros listed, corrected afterwards
-    for (uint32_t c0 = 0; c0 < nb; c0 += PF) {
+    for (uint32_t c0 = gi * PF; c0 < nb; c0 += NG * PF) {
         PR<E> sh[PF];
 #pragma unroll
         for (uint32_t u = 0; u < PF; ++u)
@@ -1539,7 +1607,7 @@ __device__ inline void repair_group_reg(const Rsi16Dev &T, uint16_t *m, uint16_t
     wave_sync();
     const uint32_t total = *nroots;
     const uint32_t listed = total < (uint32_t)E ? total : (uint32_t)E;
-    for (uint32_t r = L.gl; r < listed; r += G) {
+    for (uint32_t r = first; r < listed; r += NG * G) {
         const uint32_t pos = list[r];
         const uint32_t ri = rbo_bits(pos, T.nbits);
         const uint32_t x = T.roots_ntt[ri];
@@ -1552,7 +1620,7 @@ __device__ inline void repair_group_reg(const Rsi16Dev &T, uint16_t *m, uint16_t
         uint16_t *at = pos < T.k ? &m[pos] : &e[pos - T.k];
         *at = (uint16_t)(F::add((uint32_t)*at, err) & 0xffff);
     }
-    if (L.gl == 0)
+    if (first == 0)
         *st = total > 0 ? FFRS_RSI16_REPAIR_OK : (lanes ? FFRS_RSI16_ERROR_LOCATION_FAIL : FFRS_RSI16_NO_ERRORS);
 }
 
@@ -1641,6 +1709,18 @@ __global__ __launch_bounds__(64) void rsi16_encode_reg_kernel(const uint16_t *__
     LaneR<E> L;
     L.init(T, threadIdx.x);
     encode_group_reg<O, E>(T, msgs + (size_t)cw * T.k, out + (size_t)cw * E, L);
+}
+
+// One codeword per wave (small launches: the time of one codeword counts).
+template <int E>
+__global__ __launch_bounds__(64) void rsi16_repair_one_kernel(uint16_t *__restrict__ msgs, uint16_t *__restrict__ eccs,
+                                                              uint8_t *__restrict__ status, Rsi16Dev T)
+{
+    __shared__ uint32_t s_mem[REG_WORDS * E];
+    const uint32_t cw = blockIdx.x;
+    LaneR<E> L;
+    L.init(T, threadIdx.x);
+    repair_group_reg<E, false, true>(T, msgs + (size_t)cw * T.k, eccs + (size_t)cw * E, s_mem, L, status + cw);
 }
 
 template <int E, bool SIN = false>
@@ -1887,8 +1967,8 @@ __device__ inline v4i_t as_v4i(const uint4 &v) { return v4i_t{(int)v.x, (int)v.y
 struct ContractIn {  // `count` codewords: message rows of k symbols and (syndromes) parity rows of E
     __amdgpu_buffer_rsrc_t msg, ecc;
     uint32_t k, E, nq_m;
-    // symbols 16 h .. +16 of chunk q of codeword cw: 32-byte aligned reads, wholly inside or wholly
-    // past the buffer
+    // symbols 16 h .. +16 of chunk q of codeword cw: two 16-byte aligned reads, each wholly inside or
+    // wholly past the buffer
     template <bool SYN>
     __device__ void load(uint32_t cw, uint32_t q, uint32_t h, uint4 &x0, uint4 &x1) const
     {
@@ -1910,6 +1990,8 @@ __device__ inline void contract_store(const v4i_t acc[2], const MfmaTab &M, uint
                                       uint32_t E, uint16_t *out, uint32_t *syn)
 {
     const uint32_t j = 16 * t + 4 * h;
+    if (j >= E)  // ecc_len 8
+        return;
     uint32_t v[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i)
@@ -1921,17 +2003,20 @@ __device__ inline void contract_store(const v4i_t acc[2], const MfmaTab &M, uint
             make_uint2((v[0] & 0xffffu) | (v[1] << 16), (v[2] & 0xffffu) | (v[3] << 16));
 }
 
-// ecc_len 16 and 32: a wave takes CG groups of 16 codewords and every output tile; the matrix
+// ecc_len 8 (half a tile of output rows), 16 and 32: a wave takes CG groups of 16 codewords and every output tile; the matrix
 // (a few KB per chunk) comes from the caches. Bound by the codewords' HBM reads (rows of a few
 // hundred bytes): 262,144 RSi16(256,32) parities in 36 us (3.7 TB/s), 39 with three 7-bit limbs.
-template <int T, int CG, bool SYN>
+template <int E, int CG, int D, bool SYN>
 __global__ __launch_bounds__(256) void rsi16_contract_wave_kernel(const uint16_t *__restrict__ msgs, uint32_t msg_bytes,
                                                                   const uint16_t *__restrict__ eccs, uint32_t ecc_bytes,
                                                                   uint32_t count, MfmaTab M, uint32_t k,
                                                                   uint16_t *__restrict__ out,
-                                                                  uint32_t *__restrict__ syn)
+                                                                  uint32_t *__restrict__ syn,
+                                                                  uint32_t *__restrict__ clear)
 {
-    constexpr uint32_t E = 16 * T;
+    constexpr int T = (E + 15) / 16;
+    if (SYN && blockIdx.x == 0 && threadIdx.x == 0)
+        *clear = 0;
     const uint32_t lane = threadIdx.x & 63, c = lane & 15, h = lane >> 4;
     const uint32_t wave = blockIdx.x * 4 + (threadIdx.x >> 6), waves = gridDim.x * 4;
     const ContractIn in{make_rsrc(msgs, msg_bytes), make_rsrc(SYN ? eccs : msgs, SYN ? ecc_bytes : 0), k, E, M.nq_m};
@@ -1946,27 +2031,39 @@ __global__ __launch_bounds__(256) void rsi16_contract_wave_kernel(const uint16_t
                     acc[t][g][0][i] = M.row[16 * t + 4 * h + i].x;
                 acc[t][g][1] = v4i_t{0, 0, 0, 0};
             }
-#pragma unroll 2
-        for (uint32_t q = 0; q < M.nq; ++q) {
-            uint4 x0[CG], x1[CG], a[T][2];
+        uint4 x0[D][CG], x1[D][CG], a[D][T][2];
+        auto fetch = [&](int d, uint32_t q) {
+            if (q >= M.nq)
+                return;
 #pragma unroll
             for (int g = 0; g < CG; ++g) {
                 const uint32_t cw = (grp * CG + g) * 16 + c;
-                in.load<SYN>(cw < count ? cw : count - 1, q, h, x0[g], x1[g]);
+                in.load<SYN>(cw < count ? cw : count - 1, q, h, x0[d][g], x1[d][g]);
             }
 #pragma unroll
             for (int t = 0; t < T; ++t)
 #pragma unroll
                 for (int b = 0; b < 2; ++b)
-                    a[t][b] = M.pack[((t * M.nq + q) * 2 + b) * 64 + lane];
+                    a[d][t][b] = M.pack[((t * M.nq + q) * 2 + b) * 64 + lane];
+        };
 #pragma unroll
-            for (int g = 0; g < CG; ++g) {
-                v4i_t lo, hi;
-                contract_limbs(x0[g], x1[g], lo, hi);
-                const v4i_t nhi = ~hi;
+        for (int d = 0; d < D; ++d)
+            fetch(d, d);
+        for (uint32_t q0 = 0; q0 < M.nq; q0 += D) {
 #pragma unroll
-                for (int t = 0; t < T; ++t)
-                    contract_step(acc[t][g], as_v4i(a[t][0]), as_v4i(a[t][1]), lo, hi, nhi);
+            for (int d = 0; d < D; ++d) {
+                if (q0 + d >= M.nq)
+                    break;
+#pragma unroll
+                for (int g = 0; g < CG; ++g) {
+                    v4i_t lo, hi;
+                    contract_limbs(x0[d][g], x1[d][g], lo, hi);
+                    const v4i_t nhi = ~hi;
+#pragma unroll
+                    for (int t = 0; t < T; ++t)
+                        contract_step(acc[t][g], as_v4i(a[d][t][0]), as_v4i(a[d][t][1]), lo, hi, nhi);
+                }
+                fetch(d, q0 + d + D);
             }
         }
 #pragma unroll
@@ -1991,9 +2088,12 @@ template <int NW, int TPW, int CG, int D, bool SYN>
 __global__ __launch_bounds__(NW * 64) void rsi16_contract_kernel(const uint16_t *__restrict__ msgs, uint32_t msg_bytes,
                                                                  const uint16_t *__restrict__ eccs, uint32_t ecc_bytes,
                                                                  uint32_t count, MfmaTab M, uint32_t k,
-                                                                 uint16_t *__restrict__ out, uint32_t *__restrict__ syn)
+                                                                 uint16_t *__restrict__ out, uint32_t *__restrict__ syn,
+                                                                 uint32_t *__restrict__ clear)
 {
     static_assert(CG <= NW, "one loading wave per group");
+    if (SYN && blockIdx.x == 0 && threadIdx.x == 0)
+        *clear = 0;
     constexpr uint32_t E = 16 * NW * TPW;
     __shared__ uint4 s_x[2][CG][2][64];
     const uint32_t lane = threadIdx.x & 63, c = lane & 15, h = lane >> 4, wave = threadIdx.x >> 6;
@@ -2061,6 +2161,380 @@ __global__ __launch_bounds__(NW * 64) void rsi16_contract_kernel(const uint16_t 
 #pragma unroll
             for (int t = 0; t < TPW; ++t)
                 contract_store<SYN>(acc[t][g], M, wave * TPW + t, h, cw, E, out, syn);
+    }
+}
+
+// ---------------------------------------------------------------- repair, one codeword per lane
+
+// The key equation for ecc_len <= 32 with one codeword per lane. pr_sugiyama's usual step (the
+// quotient has two terms, every remainder one degree below the last) needs no data-dependent
+// index: after s steps the remainder has degree E - 1 - s and the locator degree s, so the steps
+// are unrolled with every polynomial in registers, and lanes whose remainder has dropped below
+// E / 2 keep what they hold. A codeword whose remainder drops by more than one degree and stays at
+// E / 2 or above, or that meets one of the other cases listed at lane_solve, goes to the general
+// kernel (rsi16_repair_list_kernel): about 17 in 65,537 damaged codewords.
+// 262,144 RSi16(256,32) repairs with 0-16 errors: 38 us of syndromes, 96 here and 24 for the 60 odd
+// ones, against 402 + 52 with a codeword per sixteen lanes. Bound by the vector units (a wave's
+// 9,000 instructions, 80 % of the issue slots): a third of them the key equation's steps, the rest
+// the root search's epilogues, Forney and the conversions between.
+//
+// Values are held as b = (v + 32768) mod p in [-1, 65536] (zero is 32768 alone), v = b - 32768 in
+// [-32769, 32768]: a remainder coefficient c2 + n0 c1 + n1 c1' is then
+//   fold16(fold16(b2 + n0 b1 + n1 b1' - 32768 (n0 + n1))),
+// where the sum is taken mod 2^32 and its true value fits an int32 as long as |n0|, |n1| <= 32766
+// (2 * 32766 * 32769 + 65537 < 2^31): two 24-bit multiply-adds, an add and two folds. A step where
+// some lane's factor is larger folds after each product instead.
+constexpr int32_t RBIAS = 0x8000;
+
+__device__ inline int32_t mad24(int32_t a, int32_t b, int32_t c)
+{
+    int32_t r;
+    asm("v_mad_i32_i24 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
+}
+__device__ inline int32_t fold2(int32_t y) { return fold16(fold16(y)); }
+// a b mod p in [-32769, 32768] for |a|, |b| <= 32769
+__device__ inline int32_t bal_mul(int32_t a, int32_t b) { return fold2(mad24(a, b, RBIAS)) - RBIAS; }
+// canonical value of v in [-32769, 32768]
+__device__ inline uint32_t bal_canon(int32_t v) { return (uint32_t)(v + ((v >> 31) & (int32_t)P16)); }
+// 1 / v (1 for 0), balanced
+__device__ inline int32_t bal_inv(const uint32_t *inv_tab, int32_t v)
+{
+    const int32_t c = (int32_t)inv_tab[bal_canon(v)];
+    return c > 32768 ? c - (int32_t)P16 : c;
+}
+// 3^i mod p, balanced
+constexpr int32_t bal_pow3(int i)
+{
+    int64_t r = 1;
+    for (int j = 0; j < i; ++j)
+        r = r * 3 % 65537;
+    return (int32_t)(r > 32768 ? r - 65537 : r);
+}
+
+// c2 + n0 c1 + n1 c1' in the biased form; k = -32768 (n0 + n1) (SAFE: k0, k1 of each product)
+template <bool SAFE>
+__device__ inline int32_t lane_update(int32_t b2, int32_t b1, int32_t b1p, int32_t n0, int32_t n1, int32_t k0, int32_t k1)
+{
+    if constexpr (SAFE)
+        return fold2(mad24(n1, b1p, fold2(mad24(n0, b1, b2 + k0)) + k1));
+    else
+        return fold2(mad24(n1, b1p, mad24(n0, b1, b2 + k0)));
+}
+
+template <int E>
+struct LaneSolve {
+    static constexpr int T = E / 2;
+    int32_t R[2][E];      // remainders, R[s & 1] after s steps
+    int32_t A[2][T + 1];  // their locator cofactors
+    uint32_t steps;
+    bool clean, odd;      // no syndrome; left to the general kernel
+
+    // y <- y - q x for the next remainder and cofactor (s: the steps done after it)
+    template <bool SAFE, int S_>
+    __device__ void update(int32_t n0, int32_t n1)
+    {
+        constexpr int y = S_ & 1, x = y ^ 1;
+        const int32_t k1 = SAFE ? -RBIAS * n1 : 0, k0 = SAFE ? -RBIAS * n0 : -RBIAS * (n0 + n1);
+#pragma unroll
+        for (int i = 0; i <= E - 1 - S_; ++i)
+            R[y][i] = lane_update<SAFE>(R[y][i], R[x][i], i ? R[x][i - 1] : RBIAS, n0, n1, k0, k1);
+#pragma unroll
+        for (int i = 0; i <= S_; ++i)
+            A[y][i] = lane_update<SAFE>(A[y][i], A[x][i], i ? A[x][i - 1] : RBIAS, n0, n1, k0, k1);
+    }
+
+    // After step s: stop where the remainder fell below degree E / 2.
+    template <int S_>
+    __device__ void check(bool &active)
+    {
+        constexpr int y = S_ & 1;
+        if constexpr (S_ == T) {
+            if (active)
+                steps = T;
+        } else if (active && R[y][E - 1 - S_] == RBIAS) {
+            uint32_t high = 0, low = 0;
+#pragma unroll
+            for (int i = T; i < E - 1 - S_; ++i)
+                high |= (uint32_t)(R[y][i] ^ RBIAS);
+#pragma unroll
+            for (int i = 0; i < T; ++i)
+                low |= (uint32_t)(R[y][i] ^ RBIAS);
+            active = false;
+            steps = S_;
+            odd = high != 0 || low == 0;  // an irregular step, or a zero remainder (the reference may raise)
+        }
+    }
+
+    template <int S_>
+    __device__ void step(bool &active, const uint32_t *inv_tab)
+    {
+        if constexpr (S_ <= T) {
+            if (active) {
+                constexpr int y = S_ & 1, x = y ^ 1, g = E - (S_ - 1);  // lengths g + 1 and g
+                const int32_t h1 = R[y][g] - RBIAS, h2 = R[y][g - 1] - RBIAS;
+                const int32_t a0 = bal_inv(inv_tab, R[x][g - 1] - RBIAS), w = bal_mul(a0, R[x][g - 2] - RBIAS);
+                // the quotient's coefficients a0 (h2 - w h1) and a0 h1 (pr_sugiyama), negated
+                const int32_t n1 = -bal_mul(a0, h1);
+                const int32_t n0 = bal_mul(a0, fold2(mad24(w, h1, RBIAS - h2)) - RBIAS);
+                const int32_t big = max(abs(n0), abs(n1));
+                if (__any(big > 32766))
+                    update<true, S_>(n0, n1);
+                else
+                    update<false, S_>(n0, n1);
+            }
+            check<S_>(active);
+            step<S_ + 1>(active, inv_tab);
+        }
+    }
+
+    __device__ void solve(const uint32_t *__restrict__ syn, const uint32_t *__restrict__ inv_tab, bool valid)
+    {
+        uint32_t any = 0;
+#pragma unroll
+        for (int i = 0; i < E; i += 4) {
+            const uint4 v = valid ? *reinterpret_cast<const uint4 *>(syn + i) : make_uint4(0, 0, 0, 0);
+            any |= v.x | v.y | v.z | v.w;
+            R[0][i] = fold16((int32_t)v.x + RBIAS);
+            R[0][i + 1] = fold16((int32_t)v.y + RBIAS);
+            R[0][i + 2] = fold16((int32_t)v.z + RBIAS);
+            R[0][i + 3] = fold16((int32_t)v.w + RBIAS);
+        }
+#pragma unroll
+        for (int i = 0; i < E; ++i)
+            R[1][i] = RBIAS;
+#pragma unroll
+        for (int i = 0; i <= T; ++i)
+            A[0][i] = A[1][i] = RBIAS;
+        A[0][0] = RBIAS + 1;
+        clean = any == 0;
+        odd = !clean && R[0][E - 1] == RBIAS;
+        steps = 0;
+        bool active = !clean && !odd;
+        if (active) {  // the first step, x^E against the syndromes
+            const int32_t a11 = -bal_inv(inv_tab, R[0][E - 1] - RBIAS);
+            const int32_t a10 = bal_mul(R[0][E - 2] - RBIAS, bal_mul(a11, a11));
+            const int32_t k0 = -RBIAS * a10, k1 = -RBIAS * a11;
+#pragma unroll
+            for (int i = 0; i < E - 1; ++i)
+                R[1][i] = lane_update<true>(RBIAS, R[0][i], i ? R[0][i - 1] : RBIAS, a10, a11, k0, k1);
+            A[1][0] = a10 + RBIAS;
+            A[1][1] = fold16(a11 + RBIAS);
+        }
+        check<1>(active);
+        step<2>(active, inv_tab);
+    }
+};
+
+// Roots of the locators on the matrix cores: locator(x) at the n positions' inverse locators
+// x = w^-rbo(m) (NTT::pintt_ecc, ntt.hpp:206-220), as the contraction of (a_i 3^i) with ((x / 3)^i),
+// i = 1 .. T, the limbs of both as in the encode (a matrix power (x / 3)^i is never 32640, the one
+// residue two byte limbs miss; a locator holding it is multiplied by 3, which moves no root), plus
+// a_0. B operand of one MFMA: quarter h of the lanes holds limb h / 2 of coefficients (h & 1) half.
+struct RootTab {
+    const uint64_t *pack;  // tile * 64 + lane: 8 bytes of the A operand
+    const int4 *row;       // tile * 4 + h: sum_i g1 of positions 16 tile + 4 h .. +4
+};
+
+constexpr uint32_t lane_repair_words(int T) { return 64u * (T + 1) + 64u * (uint32_t)(T < 8 ? 8 : T) + 64u; }
+
+template <int E>
+__global__ __launch_bounds__(64, 4) void rsi16_repair_lane_kernel(uint16_t *__restrict__ msgs,
+                                                                  uint16_t *__restrict__ eccs, uint32_t count,
+                                                                  uint8_t *__restrict__ status, Rsi16Dev D, RootTab RT,
+                                                                  const uint32_t *__restrict__ syn,
+                                                                  uint32_t *__restrict__ list)
+{
+    constexpr int T = E / 2, WORDS = T + 1;  // per codeword: T evaluator and T + 1 locator coefficients, u16
+    __shared__ uint32_t s_co[64 * WORDS];
+    __shared__ uint4 s_li[64 * (T < 8 ? 8 : T) / 4];  // the locators' limbs, then the list of roots
+    __shared__ uint32_t s_found[64];
+    const uint32_t lane = threadIdx.x, cw0 = blockIdx.x * 64, cw = cw0 + lane;
+    const bool valid = cw < count;
+    bool clean, odd;
+    {
+        LaneSolve<E> S;
+        S.solve(syn + (size_t)(valid ? cw : 0) * E, D.inv_tab, valid);
+        int32_t a[T + 1], r[T];
+#pragma unroll
+        for (int i = 0; i <= T; ++i)
+            a[i] = ((S.steps & 1) ? S.A[1][i] : S.A[0][i]) - RBIAS;
+#pragma unroll
+        for (int i = 0; i < T; ++i)
+            r[i] = ((S.steps & 1) ? S.R[1][i] : S.R[0][i]) - RBIAS;
+        clean = S.clean;
+        odd = S.odd || (!clean && a[0] == 0);
+        // 65536 does not fit the stored u16 and 32640 not the limbs: another multiple then
+        int32_t v[T];
+        for (int tries = 0;; ++tries) {
+            bool bad = a[0] == -1;
+#pragma unroll
+            for (int i = 0; i < T; ++i) {
+                const int32_t x = bal_mul(a[i + 1], bal_pow3(i + 1));
+                bad |= a[i + 1] == -1 || r[i] == -1 || x == 32640;
+                v[i] = x > 32639 ? x - (int32_t)P16 : x;
+            }
+            bad = bad && !clean && !odd;
+            if (!__any(bad))
+                break;
+            if (tries == 32)
+                odd |= bad;
+            if (bad) {
+#pragma unroll
+                for (int i = 0; i <= T; ++i)
+                    a[i] = bal_mul(a[i], 3);
+#pragma unroll
+                for (int i = 0; i < T; ++i)
+                    r[i] = bal_mul(r[i], 3);
+            }
+        }
+        const bool off = clean || odd;
+        uint32_t *co = s_co + lane * WORDS;
+#pragma unroll
+        for (int i = 0; i < T; i += 2)
+            co[i / 2] = bal_canon(r[i]) | (bal_canon(r[i + 1]) << 16);
+#pragma unroll
+        for (int i = 0; i < T; i += 2)
+            co[T / 2 + i / 2] = (off && i == 0 ? 1u : bal_canon(a[i])) | (bal_canon(a[i + 1]) << 16);
+        co[T] = bal_canon(a[T]);
+        constexpr int TP = T < 16 ? 16 : T;
+        uint32_t lo[TP / 4], hi[TP / 4];
+#pragma unroll
+        for (int i = 0; i < TP; i += 4) {
+            uint32_t p[2] = {0, 0};
+#pragma unroll
+            for (int u = 0; u < 2; ++u)
+                if (i + 2 * u < T) {
+                    const uint32_t t0 = (uint32_t)((v[i + 2 * u] + 0x80) ^ 0x80) & 0xffffu;
+                    const uint32_t t1 = (uint32_t)((v[i + 2 * u + 1] + 0x80) ^ 0x80);
+                    p[u] = off ? 0u : t0 | (t1 << 16);
+                }
+            lo[i / 4] = __builtin_amdgcn_perm(p[1], p[0], 0x06040200u);
+            hi[i / 4] = __builtin_amdgcn_perm(p[1], p[0], 0x07050301u);
+        }
+        s_li[lane * 2] = make_uint4(lo[0], lo[1], lo[2], lo[3]);
+        s_li[lane * 2 + 1] = make_uint4(hi[0], hi[1], hi[2], hi[3]);
+        s_found[lane] = 0;
+    }
+    wave_sync();
+    const uint32_t c = lane & 15, h = lane >> 4;
+    uint64_t b0[4], b1[4];
+    int32_t loc0[4];
+    {
+        const uint64_t *li = reinterpret_cast<const uint64_t *>(s_li);
+        const uint64_t flip = h >= 2 ? ~0ull : 0ull;
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            const uint32_t row = (16 * g + c) * 4 + (h & 1);
+            b0[g] = li[row + (h >> 1) * 2] ^ flip;
+            b1[g] = li[row + ((h >> 1) ^ 1) * 2];
+            loc0[g] = (int32_t)(s_co[(16 * g + c) * WORDS + T / 2] & 0xffffu);
+        }
+    }
+    wave_sync();
+    uint32_t *roots = reinterpret_cast<uint32_t *>(s_li);
+    constexpr uint32_t cap = 64 * (T < 8 ? 8 : T);
+    uint32_t total = 0;
+    const uint32_t tiles = (D.n + 15) / 16;
+    uint64_t An = RT.pack[lane];
+    int4 kn = RT.row[h];
+    for (uint32_t t = 0; t < tiles; ++t) {
+        const uint64_t A = An;
+        const int4 kc = kn;
+        if (t + 1 < tiles) {  // the next tile's operands, a tile ahead
+            An = RT.pack[(t + 1) * 64 + lane];
+            kn = RT.row[(t + 1) * 4 + h];
+        }
+        v4i_t p0[4], p1[4];
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            p0[g] = v4i_t{kc.x + loc0[g], kc.y + loc0[g], kc.z + loc0[g], kc.w + loc0[g]};
+            p1[g] = v4i_t{0, 0, 0, 0};
+            p0[g] = __builtin_amdgcn_mfma_i32_16x16x32_i8((long)A, (long)b0[g], p0[g], 0, 0, 0);
+            p1[g] = __builtin_amdgcn_mfma_i32_16x16x32_i8((long)A, (long)b1[g], p1[g], 0, 0, 0);
+        }
+        uint32_t hits = 0;  // this lane's 16 values, the first in bit 15
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int32_t f = fold2(p0[g][i] + 256 * p1[g][i]);  // |p1| <= 2^19; 0 at a root alone
+                asm("v_cmp_eq_u32 vcc, 0, %1\n\tv_addc_co_u32 %0, vcc, %0, %0, vcc" : "+v"(hits) : "v"(f) : "vcc");
+            }
+        for (uint64_t m = __ballot(hits != 0); m; m = __ballot(hits != 0)) {
+            if (hits) {
+                const uint32_t v = (uint32_t)__builtin_clz(hits) - 16, w = 16 * (v >> 2) + c;
+                const uint32_t at = total + __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
+                                                                     __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+                hits &= ~(0x8000u >> v);
+                if (at < cap)
+                    roots[at] = (w << 16) | (16 * t + 4 * h + (v & 3));
+                s_found[w] = 1;
+            }
+            total += (uint32_t)__popcll(m);
+        }
+    }
+    wave_sync();
+    total = total < cap ? total : cap;  // at most T roots a codeword
+    for (uint32_t q = lane; q < total; q += 64) {
+        const uint32_t pos = roots[q] & 0xffffu, w = roots[q] >> 16;
+        const uint32_t ri = rbo_bits(pos, D.nbits);
+        const uint32_t x = D.roots_ntt[ri], xi = D.roots_ntt[(D.N - ri) & (D.N - 1)];
+        const int32_t xb = (int32_t)xi > 32768 ? (int32_t)xi - (int32_t)P16 : (int32_t)xi;
+        const uint32_t *co = s_co + w * WORDS;
+        int32_t num = 0, den = 0;
+#pragma unroll
+        for (int i = T - 2; i >= 0; i -= 2) {
+            const uint32_t u = co[i / 2];
+            num = fold2(mad24(num, xb, (int32_t)(u >> 16) + RBIAS)) - RBIAS;
+            num = fold2(mad24(num, xb, (int32_t)(u & 0xffffu) + RBIAS)) - RBIAS;
+        }
+        // the locator's derivative: sum i a_i x^(i - 1)
+        uint32_t u = co[T];
+        den = fold2(T * (int32_t)(u & 0xffffu) + RBIAS) - RBIAS;
+#pragma unroll
+        for (int i = T - 1; i >= 1; --i) {
+            if (i & 1)
+                u = co[T / 2 + i / 2];
+            const int32_t ai = (i & 1) ? (int32_t)(u >> 16) : (int32_t)(u & 0xffffu);
+            den = fold2(mad24(den, xb, fold2(i * ai + RBIAS))) - RBIAS;
+        }
+        // _forney (rsi16v_impl.hpp:500-512): both sums are multiples of the normalised ones by the
+        // same factor; where the derivative vanishes the quotient is the normalised numerator
+        const uint32_t nc = bal_canon(num), dc = bal_canon(den);
+        const uint32_t scale = D.inv_tab[dc ? dc : co[T / 2] & 0xffffu];
+        const uint32_t err = F::mul(nc ? F::mul(nc, scale) : 0u, x);
+        const size_t row = cw0 + w;
+        uint16_t *at = pos < D.k ? msgs + row * D.k + pos : eccs + row * E + (pos - D.k);
+        *at = (uint16_t)(F::add((uint32_t)*at, err) & 0xffff);
+    }
+    if (valid) {
+        if (odd)
+            list[1 + atomicAdd(list, 1u)] = cw;
+        else
+            status[cw] = clean ? FFRS_RSI16_NO_ERRORS
+                               : s_found[lane] ? FFRS_RSI16_REPAIR_OK : FFRS_RSI16_ERROR_LOCATION_FAIL;
+    }
+}
+
+// The codewords list[1 .. list[0]] through the general register repair, one per wave: a few in a
+// launch of many, so what counts is the time of one.
+template <int E>
+__global__ __launch_bounds__(64) void rsi16_repair_list_kernel(uint16_t *__restrict__ msgs, uint16_t *__restrict__ eccs,
+                                                               uint8_t *__restrict__ status, Rsi16Dev T,
+                                                               const uint32_t *__restrict__ syn,
+                                                               const uint32_t *__restrict__ list)
+{
+    __shared__ uint32_t s_mem[REG_WORDS * E];
+    if (blockIdx.x >= list[0])
+        return;
+    LaneR<E> L;
+    L.init(T, threadIdx.x);
+    for (uint32_t i = blockIdx.x; i < list[0]; i += gridDim.x) {
+        const uint32_t cw = list[1 + i];
+        repair_group_reg<E, true, true>(T, msgs + (size_t)cw * T.k, eccs + (size_t)cw * E, s_mem, L, status + cw,
+                                        syn + (size_t)cw * E);
+        wave_sync();
     }
 }
 
@@ -2867,6 +3341,10 @@ struct ffrs_rsi16 {
     void *d_work = nullptr;          // workspace of the SIMD-word interleaved repair
     size_t work_size = 0;
     ContractTab enc, synd;           // the encode and the syndromes as int8 MFMA contractions
+    struct {
+        void *d = nullptr;
+        RootTab dev{};
+    } roots;                         // the locator's values at the n positions (ecc_len 8 to 32)
     bool mix_minus_one = false;      // a mix constant is 65536: the SIMD words are not the linear map
     int encode_mode = 0;             // 0 automatic, 1 butterflies, 2 MFMA wherever it applies
     uint32_t *d_syn = nullptr;       // syndromes of the last repair launch
@@ -2949,27 +3427,28 @@ size_t contract_step_count(const ffrs_rsi16 *rs)
     return std::max<size_t>(64, (((size_t)1 << 31) / (rs->k * 2)) & ~(size_t)63);
 }
 
-// One launch of a contraction (count <= contract_step_count) for ecc_len E.
+// One launch of a contraction (count <= contract_step_count) for ecc_len E; syndromes also set
+// *clear to 0.
 template <int E, bool SYN>
 int launch_contract(ffrs_rsi16 *rs, const MfmaTab &M, const uint16_t *d_msg, const uint16_t *d_ecc, size_t count,
-                    uint16_t *d_out, uint32_t *d_syn)
+                    uint16_t *d_out, uint32_t *d_syn, uint32_t *clear)
 {
     const uint32_t mb = (uint32_t)(count * rs->k * 2), eb = (uint32_t)(count * E * 2);
     if constexpr (E <= 32) {
         const size_t groups = (count + 15) / 16;
-        hipLaunchKernelGGL((rsi16_contract_wave_kernel<E / 16, 1, SYN>),
+        hipLaunchKernelGGL((rsi16_contract_wave_kernel<E, 1, 3, SYN>),
                            dim3(persistent_grid(rs->ctx, 8, (groups + 3) / 4)), dim3(256), 0, rs->ctx->stream, d_msg,
-                           mb, d_ecc, eb, (uint32_t)count, M, rs->k, d_out, d_syn);
+                           mb, d_ecc, eb, (uint32_t)count, M, rs->k, d_out, d_syn, clear);
     } else {
         constexpr int NW = E == 64 ? 4 : 8, TPW = E / 16 / NW;
         if ((count + 63) / 64 >= (size_t)rs->ctx->cu_count)
             hipLaunchKernelGGL((rsi16_contract_kernel<NW, TPW, 4, 3, SYN>), dim3((unsigned)((count + 63) / 64)),
                                dim3(NW * 64), 0, rs->ctx->stream, d_msg, mb, d_ecc, eb, (uint32_t)count, M, rs->k, d_out,
-                               d_syn);
+                               d_syn, clear);
         else
             hipLaunchKernelGGL((rsi16_contract_kernel<NW, TPW, 1, 4, SYN>), dim3((unsigned)((count + 15) / 16)),
                                dim3(NW * 64), 0, rs->ctx->stream, d_msg, mb, d_ecc, eb, (uint32_t)count, M, rs->k, d_out,
-                               d_syn);
+                               d_syn, clear);
     }
     FFRS_HIP(hipGetLastError());
     return FFRS_OK;
@@ -2979,14 +3458,15 @@ int launch_contract(ffrs_rsi16 *rs, const MfmaTab &M, const uint16_t *d_msg, con
 int launch_encode_mfma(ffrs_rsi16 *rs, const uint16_t *d_msg, size_t count, uint16_t *d_ecc)
 {
     const size_t step = contract_step_count(rs);
-    auto *f = rs->E == 16    ? launch_contract<16, false>
+    auto *f = rs->E == 8     ? launch_contract<8, false>
+              : rs->E == 16  ? launch_contract<16, false>
               : rs->E == 32  ? launch_contract<32, false>
               : rs->E == 64  ? launch_contract<64, false>
               : rs->E == 128 ? launch_contract<128, false>
                              : launch_contract<256, false>;
     for (size_t b = 0; b < count; b += step)
         if (int r = f(rs, rs->enc.dev, d_msg + b * rs->k, nullptr, std::min(step, count - b), d_ecc + b * rs->E,
-                      nullptr))
+                      nullptr, nullptr))
             return r;
     mark_kernel(rs->ctx);
     return FFRS_OK;
@@ -3049,11 +3529,27 @@ int launch_repair_reg(ffrs_rsi16 *rs, uint16_t *d_msg, uint16_t *d_ecc, size_t c
 {
     constexpr uint32_t cpw = 64 / RegShape<E>::G;
     const size_t lds = (size_t)cpw * REG_WORDS * E * 4;
-    // the syndromes on the matrix cores first, where their tables exist
-    const bool msyn = rs->synd.dev.nq && rs->repair_synd != 1 && (((uintptr_t)d_msg | (uintptr_t)d_ecc) & 15) == 0;
+    // One codeword per wave while that leaves at most two waves per SIMD, the groups of the wave
+    // sharing its chunks (us against the general kernel: 1 codeword RSi16(256,32) 10.4 / 14.6,
+    // (1024,8) 12 / 78, (4096,32) 17 / 61; 2,048: 28 / 30, 18 / 89, 64 / 175; 16,384: 98 / 55).
+    if (E <= 32 && rs->repair_synd != 1 && count <= 8 * (size_t)rs->ctx->cu_count) {
+        hipLaunchKernelGGL(rsi16_repair_one_kernel<E>, dim3((unsigned)count), dim3(64), 0, rs->ctx->stream, d_msg, d_ecc,
+                           d_status, rs->dev);
+        FFRS_HIP(hipGetLastError());
+        mark_kernel(rs->ctx);
+        return FFRS_OK;
+    }
+    // The syndromes on the matrix cores first, where their tables exist; for ecc_len 8 to 32 then one
+    // codeword per lane, from the counts on where 64 codewords per wave fill the chip and the three
+    // launches pay (us, general kernel / this: RSi16(256,32) 16,384 codewords 55 / 64, 32,768 91 / 66,
+    // 262,144 544 / 179; (1024,8) 4,096 89 / 47; (64,8) 32,768 20 / 23, 262,144 74 / 55).
+    const bool lanes = E <= 32 && count * rs->n >= ((size_t)1 << 22) && count >= (E == 8 ? 2048 : 24576);
+    const bool msyn = rs->synd.dev.nq && rs->repair_synd != 1 && (E >= 64 || lanes || rs->repair_synd == 2) &&
+                      (((uintptr_t)d_msg | (uintptr_t)d_ecc) & 15) == 0;
     if (msyn) {
-        const size_t step = contract_step_count(rs);
-        const size_t need = std::min(count, step) * E * 4;
+        // workspace: E syndromes per codeword and the list of those left to the general kernel
+        const size_t step = contract_step_count(rs), chunk = std::min(count, step);
+        const size_t need = chunk * E * 4 + (chunk + 1) * 4;
         if (rs->syn_size < need) {
             if (rs->d_syn)
                 FFRS_HIP(hipFree(rs->d_syn));
@@ -3064,18 +3560,28 @@ int launch_repair_reg(ffrs_rsi16 *rs, uint16_t *d_msg, uint16_t *d_ecc, size_t c
                 return fail(FFRS_ERR_NOMEM, "syndrome workspace of %zu bytes: %s", need, hipGetErrorString(e));
             rs->syn_size = need;
         }
-        if (int r = allow_lds(rsi16_repair_reg_kernel<E, true>, lds))
-            return r;
+        uint32_t *syn = rs->d_syn, *list = syn + chunk * E;
         for (size_t b = 0; b < count; b += step) {
             const size_t c = std::min(step, count - b);
-            if constexpr (E >= 16)
-                if (int r = launch_contract<E, true>(rs, rs->synd.dev, d_msg + b * rs->k, d_ecc + b * E, c, nullptr,
-                                                     rs->d_syn))
+            uint16_t *m = d_msg + b * rs->k, *e = d_ecc + b * E;
+            if constexpr (E >= 8) {
+                if (int r = launch_contract<E, true>(rs, rs->synd.dev, m, e, c, nullptr, syn, list))
                     return r;
-            mark_kernel(rs->ctx);
-            hipLaunchKernelGGL((rsi16_repair_reg_kernel<E, true>), dim3((unsigned)((c + cpw - 1) / cpw)), dim3(64), lds,
-                               rs->ctx->stream, d_msg + b * rs->k, d_ecc + b * E, (uint32_t)c, d_status + b, rs->dev,
-                               (const uint32_t *)rs->d_syn);
+                mark_kernel(rs->ctx);
+            }
+            if constexpr (E >= 8 && E <= 32) {
+                hipLaunchKernelGGL(rsi16_repair_lane_kernel<E>, dim3((unsigned)((c + 63) / 64)), dim3(64), 0,
+                                   rs->ctx->stream, m, e, (uint32_t)c, d_status + b, rs->dev, rs->roots.dev, syn, list);
+                FFRS_HIP(hipGetLastError());
+                mark_kernel(rs->ctx);
+                hipLaunchKernelGGL(rsi16_repair_list_kernel<E>, dim3((unsigned)std::min<size_t>(1024, c)), dim3(64), 0,
+                                   rs->ctx->stream, m, e, d_status + b, rs->dev, syn, list);
+            } else {
+                if (int r = allow_lds(rsi16_repair_reg_kernel<E, true>, lds))
+                    return r;
+                hipLaunchKernelGGL((rsi16_repair_reg_kernel<E, true>), dim3((unsigned)((c + cpw - 1) / cpw)), dim3(64),
+                                   lds, rs->ctx->stream, m, e, (uint32_t)c, d_status + b, rs->dev, syn);
+            }
             FFRS_HIP(hipGetLastError());
             mark_kernel(rs->ctx);
         }
@@ -3147,9 +3653,9 @@ void gs_host(const std::vector<uint32_t> &roots, uint32_t *x, uint32_t len)
 // where no symbol enters), nq_m chunks of them for the message.
 int build_contract(ContractTab *tab, const std::vector<uint32_t> &mat, uint32_t E, uint32_t nq, uint32_t nq_m)
 {
-    const uint32_t T = E / 16, rows = nq * 64;
+    const uint32_t T = (E + 15) / 16, rows = nq * 64;
     std::vector<uint8_t> pack((size_t)T * nq * 2 * 64 * 16);
-    std::vector<int32_t> row((size_t)E * 2);
+    std::vector<int32_t> row((size_t)T * 16 * 2);
     std::vector<uint8_t> seen(P16);
     const uint32_t third = s_pow(3, 65535);
     for (uint32_t j = 0; j < E; ++j) {
@@ -3194,13 +3700,13 @@ int build_contract(ContractTab *tab, const std::vector<uint32_t> &mat, uint32_t 
 
 // The encode's matrix: G[m] = the parity of the unit message at m, i.e. the GS butterfly of
 // mix_i X_m^i with X_m = w^rbo(m) (the message residue of rsi16v_impl.hpp:93-97 is
-// sum_m v_m X_m^i, then :108-119). Shapes with ecc_len not a multiple of 16, above 256, or
-// message_len above 16384 keep the butterfly kernels.
+// sum_m v_m X_m^i, then :108-119). Shapes with ecc_len below 8, above 256, or message_len
+// above 16384 keep the butterfly kernels.
 int build_mfma_encode(ffrs_rsi16 *rs, const std::vector<uint32_t> &mix, const std::vector<uint32_t> &roots_i_ecc,
                       const std::vector<uint32_t> &roots_ntt)
 {
     const uint32_t k = rs->k, E = rs->E;
-    if (E % 16 || E > 256 || k > 16384)
+    if ((E % 16 && E != 8) || E > 256 || k > 16384)
         return FFRS_OK;
     const uint32_t nq = (k + 63) / 64;
     std::vector<uint32_t> mat((size_t)nq * 64 * E, 0);
@@ -3217,12 +3723,51 @@ int build_mfma_encode(ffrs_rsi16 *rs, const std::vector<uint32_t> &mix, const st
     return build_contract(&rs->enc, mat, E, nq, nq);
 }
 
+// The limbs of (w^-rbo(m) / 3)^i, i = 1 .. E / 2, for the lane repair's root search (RootTab);
+// *ok = false where one of them is 32640 (not for block_len <= 32768: w^(rbo(m) i) 32640 is a
+// power of 3^(65536 / N), whose exponent no odd multiple of a power of two below it reaches).
+int build_roots(ffrs_rsi16 *rs, const std::vector<uint32_t> &roots_ntt, bool *ok)
+{
+    const uint32_t n = rs->n, T = rs->E / 2, tiles = (n + 15) / 16, third = s_pow(3, 65535);
+    std::vector<uint8_t> pack((size_t)tiles * 64 * 8, 0);
+    std::vector<int32_t> row((size_t)tiles * 16, 0);
+    for (uint32_t m = 0; m < n; ++m) {
+        const uint32_t ri = rbo_bits(m, rs->nbits);
+        const uint32_t x = S::mul(roots_ntt[(rs->N - ri) & (rs->N - 1)], third);
+        uint32_t pw = 1;
+        for (uint32_t i = 0; i < T; ++i) {
+            pw = S::mul(pw, x);
+            if (pw == 32640)
+                return FFRS_OK;
+            const int32_t v = pw > 32639 ? (int32_t)pw - (int32_t)P16 : (int32_t)pw;
+            const int32_t lo = ((v + 128) & 255) - 128, hi = (v - lo) >> 8;
+            uint8_t *p = &pack[((size_t)(m / 16) * 64 + m % 16 + 16 * (i / 8)) * 8 + i % 8];
+            p[0] = (uint8_t)lo;
+            p[32 * 8] = (uint8_t)hi;
+            row[m] += hi;
+        }
+    }
+    char *d = nullptr;
+    hipError_t e = hipMalloc(&d, pack.size() + row.size() * 4);
+    if (e == hipSuccess) {
+        rs->roots.d = d;
+        e = hipMemcpy(d, pack.data(), pack.size(), hipMemcpyHostToDevice);
+    }
+    if (e == hipSuccess)
+        e = hipMemcpy(d + pack.size(), row.data(), row.size() * 4, hipMemcpyHostToDevice);
+    if (e != hipSuccess)
+        return fail(FFRS_ERR_DEVICE, "root search tables: %s", hipGetErrorString(e));
+    rs->roots.dev = RootTab{(const uint64_t *)d, (const int4 *)(d + pack.size())};
+    *ok = true;
+    return FFRS_OK;
+}
+
 // The syndrome matrix w^(j rbo(m)) (NTT::pntt, ntt.hpp:133-152): rows m < k in ceil(k / 64) message
 // chunks, rows k + i (i < E) in the parity chunks after them.
 int build_mfma_synd(ffrs_rsi16 *rs, const std::vector<uint32_t> &roots_ntt)
 {
     const uint32_t k = rs->k, E = rs->E;
-    if (E % 16 || E > 256 || k > 16384)
+    if ((E % 16 && E != 8) || E > 256 || k > 16384)
         return FFRS_OK;
     const uint32_t nqm = (k + 63) / 64, nq = nqm + (E + 63) / 64;
     std::vector<uint32_t> mat((size_t)nq * 64 * E, 0);
@@ -3234,6 +3779,13 @@ int build_mfma_synd(ffrs_rsi16 *rs, const std::vector<uint32_t> &roots_ntt)
             row[j] = pw;
             pw = S::mul(pw, x);
         }
+    }
+    if (E <= 32) {
+        bool ok = false;
+        if (int r = build_roots(rs, roots_ntt, &ok))
+            return r;
+        if (!ok)
+            return FFRS_OK;
     }
     return build_contract(&rs->synd, mat, E, nq, nqm);
 }
@@ -3411,9 +3963,9 @@ void ffrs_rsi16_destroy(ffrs_rsi16 *rs)
         (void)hipFree(rs->d_tables);
     if (rs->d_work)
         (void)hipFree(rs->d_work);
-    for (ContractTab *c : {&rs->enc, &rs->synd})
-        if (c->d)
-            (void)hipFree(c->d);
+    for (void *d : {rs->enc.d, rs->synd.d, rs->roots.d})
+        if (d)
+            (void)hipFree(d);
     if (rs->d_syn)
         (void)hipFree(rs->d_syn);
     delete rs;
