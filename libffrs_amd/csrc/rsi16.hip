@@ -998,9 +998,12 @@ struct PR {
     uint32_t v[RegShape<E>::C];  // coefficient gl + h G in v[h]
 };
 
-template <int E>
+// WAVE: every group of the wave holds the same codeword (or G = 64), so lane indexes that depend on
+// values of the group are the same in all lanes.
+template <int E, bool WAVE = false>
 struct LaneR {
     using Sh = RegShape<E>;
+    static constexpr bool uniform = WAVE || Sh::G == 64;
     uint32_t gl, base, lane;  // lane in the group, first lane of the group, lane in the wave
     // Stage t (s = 2^t) of both butterfly orders uses roots[j << (LE - 1 - t)], j = i & (s - 1).
     // Stages with partners in other lanes (t < SX): j = gl & (s - 1), kept where this lane is
@@ -1035,10 +1038,20 @@ struct LaneR {
 };
 
 // coefficient idx (the same for the whole group)
-template <int E>
-__device__ inline uint32_t pr_get(const PR<E> &p, uint32_t idx, const LaneR<E> &L)
+template <int E, class LR>
+__device__ inline uint32_t pr_get(const PR<E> &p, uint32_t idx, const LR &L)
 {
     constexpr uint32_t G = RegShape<E>::G;
+    if constexpr (LR::uniform) {
+        const uint32_t at = (uint32_t)__builtin_amdgcn_readfirstlane((int)idx);
+        uint32_t r = 0;
+#pragma unroll
+        for (int h = 0; h < RegShape<E>::C; ++h) {
+            const uint32_t v = (uint32_t)__builtin_amdgcn_readlane((int)p.v[h], (int)(at % G));
+            r = at / G == (uint32_t)h ? v : r;
+        }
+        return r;
+    }
     const uint32_t slot = idx / G;
     // select by the bits of slot (a lookup into p.v would go through scratch memory)
     uint32_t w[RegShape<E>::C];
@@ -1054,8 +1067,8 @@ __device__ inline uint32_t pr_get(const PR<E> &p, uint32_t idx, const LaneR<E> &
 }
 
 // coefficient k of p, k < E chosen per lane
-template <int E>
-__device__ inline uint32_t pr_gather(const PR<E> &p, uint32_t k, const LaneR<E> &L)
+template <int E, class LR>
+__device__ inline uint32_t pr_gather(const PR<E> &p, uint32_t k, const LR &L)
 {
     constexpr uint32_t G = RegShape<E>::G;
     const uint32_t src = L.base + k % G, slot = k / G;
@@ -1072,8 +1085,8 @@ __device__ inline uint32_t pr_gather(const PR<E> &p, uint32_t k, const LaneR<E> 
 }
 
 // p[(i - 1) mod E] for each of the lane's coefficients
-template <int E>
-__device__ inline PR<E> pr_prev(const PR<E> &p, const LaneR<E> &L)
+template <int E, class LR>
+__device__ inline PR<E> pr_prev(const PR<E> &p, const LR &L)
 {
     constexpr uint32_t G = RegShape<E>::G;
     constexpr int C = RegShape<E>::C;
@@ -1081,7 +1094,9 @@ __device__ inline PR<E> pr_prev(const PR<E> &p, const LaneR<E> &L)
     uint32_t r[C];
 #pragma unroll
     for (int h = 0; h < C; ++h)
-        r[h] = lane_read(p.v[h], src);
+        r[h] = G == 64   ? (uint32_t)__builtin_amdgcn_mov_dpp((int)p.v[h], 0x13C, 0xf, 0xf, true)  // wave_ror:1
+               : G == 16 ? (uint32_t)__builtin_amdgcn_mov_dpp((int)p.v[h], 0x121, 0xf, 0xf, true)  // row_ror:1
+                         : lane_read(p.v[h], src);
     PR<E> o;
 #pragma unroll
     for (int h = 0; h < C; ++h)
@@ -1090,10 +1105,21 @@ __device__ inline PR<E> pr_prev(const PR<E> &p, const LaneR<E> &L)
 }
 
 // degree + 1 of p restricted to [0, max) (group_len)
-template <int E>
-__device__ inline uint32_t pr_len(const PR<E> &p, uint32_t max, const LaneR<E> &L)
+template <int E, class LR>
+__device__ inline uint32_t pr_len(const PR<E> &p, uint32_t max, const LR &L)
 {
     constexpr uint32_t G = RegShape<E>::G;
+    if constexpr (LR::uniform) {
+        constexpr uint64_t mine = G == 64 ? ~0ull : (1ull << (G & 63)) - 1;
+        uint32_t top = 0;
+#pragma unroll
+        for (int h = 0; h < RegShape<E>::C; ++h) {
+            const uint64_t m = __ballot(L.gl + (uint32_t)h * G < max && p.v[h] != 0) & mine;
+            if (m)
+                top = (uint32_t)h * G + 64 - (uint32_t)__builtin_clzll(m);
+        }
+        return top;
+    }
     uint32_t hi = 0;
 #pragma unroll
     for (int h = 0; h < RegShape<E>::C; ++h) {
@@ -1110,8 +1136,8 @@ __device__ inline uint32_t pr_len(const PR<E> &p, uint32_t max, const LaneR<E> &
 }
 
 // ct_full (RBO in, natural out, full reduction), ntt.hpp:225-249
-template <int E>
-__device__ inline void pr_ct(PR<E> &x, const uint32_t *xw, const uint32_t *ww, const LaneR<E> &L)
+template <int E, class LR>
+__device__ inline void pr_ct(PR<E> &x, const uint32_t *xw, const uint32_t *ww, const LR &L)
 {
     constexpr int C = RegShape<E>::C;
 #pragma unroll
@@ -1138,8 +1164,8 @@ __device__ inline void pr_ct(PR<E> &x, const uint32_t *xw, const uint32_t *ww, c
 }
 
 // gs_full (natural in, RBO out) with full reduction, ntt.hpp:280-302
-template <int E>
-__device__ inline void pr_gs(PR<E> &x, const uint32_t *xw, const uint32_t *ww, const LaneR<E> &L)
+template <int E, class LR>
+__device__ inline void pr_gs(PR<E> &x, const uint32_t *xw, const uint32_t *ww, const LR &L)
 {
     constexpr int C = RegShape<E>::C;
 #pragma unroll
@@ -1163,14 +1189,14 @@ __device__ inline void pr_gs(PR<E> &x, const uint32_t *xw, const uint32_t *ww, c
     }
 }
 
-template <int E>
-__device__ inline void pr_nttr(PR<E> &x, const LaneR<E> &L)
+template <int E, class LR>
+__device__ inline void pr_nttr(PR<E> &x, const LR &L)
 {
     pr_gs<E>(x, L.x_e, L.w_e, L);
 }
 
-template <int E>
-__device__ inline void pr_inttr(const Rsi16Dev &T, PR<E> &x, const LaneR<E> &L)
+template <int E, class LR>
+__device__ inline void pr_inttr(const Rsi16Dev &T, PR<E> &x, const LR &L)
 {
     pr_ct<E>(x, L.x_i, L.w_i, L);
 #pragma unroll
@@ -1179,8 +1205,8 @@ __device__ inline void pr_inttr(const Rsi16Dev &T, PR<E> &x, const LaneR<E> &L)
 }
 
 // NTT::_reverse_ntt_vec (ntt.hpp:344-354) in gather form, as reverse_ntt
-template <int E>
-__device__ inline void pr_reverse_ntt(const Rsi16Dev &T, PR<E> &v, uint32_t shift, const LaneR<E> &L)
+template <int E, class LR>
+__device__ inline void pr_reverse_ntt(const Rsi16Dev &T, PR<E> &v, uint32_t shift, const LR &L)
 {
     PR<E> out;
 #pragma unroll
@@ -1197,9 +1223,9 @@ __device__ inline void pr_reverse_ntt(const Rsi16Dev &T, PR<E> &v, uint32_t shif
 }
 
 // NTT::poly_inv_mod_xn_rev (ntt.hpp:363-469), as poly_inv_mod_xn_rev
-template <int E>
+template <int E, class LR>
 __device__ inline bool pr_poly_inv(const Rsi16Dev &T, PR<E> &g, uint32_t g_len, uint32_t g0, uint32_t a_len, PR<E> &a,
-                                   const LaneR<E> &L)
+                                   const LR &L)
 {
     constexpr int C = RegShape<E>::C;
     constexpr uint32_t G = RegShape<E>::G;
@@ -1239,10 +1265,10 @@ __device__ inline bool pr_poly_inv(const Rsi16Dev &T, PR<E> &g, uint32_t g_len, 
 }
 
 // NTT::poly_div_ntt (ntt.hpp:471-564), as poly_div_ntt
-template <int E>
+template <int E, class LR>
 __device__ inline bool pr_poly_div(const Rsi16Dev &T, const PR<E> &f, uint32_t f_len, const PR<E> &g, uint32_t g_len,
                                    uint32_t f0, uint32_t g0, PR<E> &t, PR<E> &q, uint32_t *q_len_out,
-                                   const LaneR<E> &L)
+                                   const LR &L)
 {
     constexpr int C = RegShape<E>::C;
     constexpr uint32_t G = RegShape<E>::G;
@@ -1280,8 +1306,8 @@ __device__ inline bool pr_poly_div(const Rsi16Dev &T, const PR<E> &f, uint32_t f
 // RSi16v<1>::_sugiyama (rsi16v_impl.hpp:271-440) in coefficient form, as sugiyama: r1 holds
 // the syndromes on entry and the normalised evaluator on exit. Returns the locator length,
 // or 0xFFFFFFFF where the reference raises.
-template <int E>
-__device__ inline uint32_t pr_sugiyama(const Rsi16Dev &T, PR<E> &a1, PR<E> &r1, const LaneR<E> &L)
+template <int E, class LR>
+__device__ inline uint32_t pr_sugiyama(const Rsi16Dev &T, PR<E> &a1, PR<E> &r1, const LR &L)
 {
     constexpr uint32_t G = RegShape<E>::G, mask = E - 1;
     constexpr int C = RegShape<E>::C;
@@ -1480,10 +1506,14 @@ __device__ inline uint32_t pr_sugiyama(const Rsi16Dev &T, PR<E> &a1, PR<E> &r1, 
 // and derivative copies for Forney, the root list and its count).
 constexpr uint32_t REG_WORDS = 4;
 
+template <int E, bool WAVE, class LR>
+__device__ inline void repair_finish_reg(const Rsi16Dev &T, uint16_t *m, uint16_t *e, uint32_t *base, const LR &L,
+                                         uint8_t *st, const PR<E> &loc, const PR<E> &syn, uint32_t Ln);
+
 // WAVE: the 64 / G groups of the wave serve one codeword: they take the chunks of the syndromes and
 // of the root search in turn and the roots by lane, and solve the key equation each for itself.
-template <int E, bool SIN = false, bool WAVE = false>
-__device__ inline void repair_group_reg(const Rsi16Dev &T, uint16_t *m, uint16_t *e, uint32_t *base, const LaneR<E> &L,
+template <int E, bool SIN = false, bool WAVE = false, class LR>
+__device__ inline void repair_group_reg(const Rsi16Dev &T, uint16_t *m, uint16_t *e, uint32_t *base, const LR &L,
                                         uint8_t *st, const uint32_t *syn_in = nullptr)
 {
     constexpr uint32_t G = RegShape<E>::G;
@@ -1546,6 +1576,19 @@ __device__ inline void repair_group_reg(const Rsi16Dev &T, uint16_t *m, uint16_t
             *st = FFRS_RSI16_RAISES;
         return;
     }
+    repair_finish_reg<E, WAVE>(T, m, e, base, L, st, loc, syn, Ln);
+}
+
+// The second half of repair_group_reg: roots and corrections from the normalised locator (length Ln)
+// and evaluator.
+template <int E, bool WAVE, class LR>
+__device__ inline void repair_finish_reg(const Rsi16Dev &T, uint16_t *m, uint16_t *e, uint32_t *base, const LR &L,
+                                         uint8_t *st, const PR<E> &loc, const PR<E> &syn, uint32_t Ln)
+{
+    constexpr uint32_t G = RegShape<E>::G;
+    constexpr int C = RegShape<E>::C;
+    constexpr uint32_t PF = C >= 4 ? 1 : 4, NG = WAVE ? 64 / G : 1;
+    const uint32_t gi = WAVE ? L.lane / G : 0, first = WAVE ? L.lane : L.gl, nb = T.n / E;
     const uint32_t eval_len = E - Ln + 1;
     // _deriv (rsi16v_impl.hpp:608-616): der[i] = (i + 1) loc[i + 1]
     PR<E> der;
@@ -1718,16 +1761,15 @@ __global__ __launch_bounds__(64) void rsi16_repair_one_kernel(uint16_t *__restri
 {
     __shared__ uint32_t s_mem[REG_WORDS * E];
     const uint32_t cw = blockIdx.x;
-    LaneR<E> L;
+    LaneR<E, true> L;
     L.init(T, threadIdx.x);
     repair_group_reg<E, false, true>(T, msgs + (size_t)cw * T.k, eccs + (size_t)cw * E, s_mem, L, status + cw);
 }
 
-template <int E, bool SIN = false>
+template <int E>
 __global__ __launch_bounds__(64) void rsi16_repair_reg_kernel(uint16_t *__restrict__ msgs,
                                                                uint16_t *__restrict__ eccs, uint32_t count,
-                                                               uint8_t *__restrict__ status, Rsi16Dev T,
-                                                               const uint32_t *__restrict__ syn = nullptr)
+                                                               uint8_t *__restrict__ status, Rsi16Dev T)
 {
     extern __shared__ uint32_t s_mem[];
     constexpr uint32_t G = RegShape<E>::G, cpw = 64 / G;
@@ -1737,8 +1779,7 @@ __global__ __launch_bounds__(64) void rsi16_repair_reg_kernel(uint16_t *__restri
         return;
     LaneR<E> L;
     L.init(T, threadIdx.x);
-    repair_group_reg<E, SIN>(T, msgs + (size_t)cw * T.k, eccs + (size_t)cw * E, s_mem + grp * REG_WORDS * E, L,
-                             status + cw, SIN ? syn + (size_t)cw * E : nullptr);
+    repair_group_reg<E>(T, msgs + (size_t)cw * T.k, eccs + (size_t)cw * E, s_mem + grp * REG_WORDS * E, L, status + cw);
 }
 
 __global__ __launch_bounds__(64) void rsi16_repair_kernel(uint16_t *__restrict__ msgs, uint16_t *__restrict__ eccs,
@@ -1982,6 +2023,14 @@ struct ContractIn {  // `count` codewords: message rows of k symbols and (syndro
             x1 = buf_load_u32x4(ecc, off + 16);
         }
     }
+    // symbols 8 u .. +8 of the chunk (no branch, so that the compiler can count the loads in flight)
+    template <bool SYN>
+    __device__ uint4 load8(uint32_t cw, uint32_t q, uint32_t u) const
+    {
+        const bool m = !SYN || q < nq_m;
+        const __amdgpu_buffer_rsrc_t r = m ? msg : ecc;
+        return buf_load_u32x4(r, cw * (m ? k : E) * 2 + (64 * (m ? q : q - nq_m) + 8 * u) * 2);
+    }
 };
 
 // Output rows 16 t + 4 h .. +4 of codeword cw: parity symbols, or canonical syndromes (u32)
@@ -2079,8 +2128,8 @@ __global__ __launch_bounds__(256) void rsi16_contract_wave_kernel(const uint16_t
 
 // ecc_len 64 to 256: a workgroup of NW waves takes CG groups of 16 codewords and every output tile,
 // TPW of them per wave, so that the matrix is read once per 16 CG codewords; the codewords' limbs
-// go through LDS (double buffered, one barrier per chunk), loaded D chunks ahead by the first CG
-// waves, the matrix limbs D chunks ahead by the wave that uses them. 64 codewords per workgroup
+// go through LDS (double buffered, one barrier per chunk), loaded D chunks ahead by all waves in
+// turn, the matrix limbs D chunks ahead by the wave that uses them. 64 codewords per workgroup
 // (CG = 4) where that gives every CU one, 16 below. 16,384 RSi16(4096,256) parities in 72 us
 // (1.9 TB/s; the matrix cores need 26 at their peak), 168 with the butterflies in registers, 623
 // with the matrix read once per 16 codewords.
@@ -2091,7 +2140,8 @@ __global__ __launch_bounds__(NW * 64) void rsi16_contract_kernel(const uint16_t 
                                                                  uint16_t *__restrict__ out, uint32_t *__restrict__ syn,
                                                                  uint32_t *__restrict__ clear)
 {
-    static_assert(CG <= NW, "one loading wave per group");
+    constexpr int UPW = CG * 2 > NW ? CG * 2 / NW : 1;  // 8-symbol units of a lane: waves load UPW each
+    static_assert(UPW * NW >= CG * 2, "every unit is loaded");
     if (SYN && blockIdx.x == 0 && threadIdx.x == 0)
         *clear = 0;
     constexpr uint32_t E = 16 * NW * TPW;
@@ -2099,8 +2149,6 @@ __global__ __launch_bounds__(NW * 64) void rsi16_contract_kernel(const uint16_t 
     const uint32_t lane = threadIdx.x & 63, c = lane & 15, h = lane >> 4, wave = threadIdx.x >> 6;
     const uint32_t cw0 = blockIdx.x * 16 * CG;
     const ContractIn in{make_rsrc(msgs, msg_bytes), make_rsrc(SYN ? eccs : msgs, SYN ? ecc_bytes : 0), k, E, M.nq_m};
-    const bool loader = wave < CG;
-    const uint32_t mine = min(cw0 + wave * 16 + c, count - 1);
     v4i_t acc[TPW][CG][2];
 #pragma unroll
     for (int t = 0; t < TPW; ++t)
@@ -2111,24 +2159,33 @@ __global__ __launch_bounds__(NW * 64) void rsi16_contract_kernel(const uint16_t 
                 acc[t][g][0][i] = M.row[16 * (wave * TPW + t) + 4 * h + i].x;
             acc[t][g][1] = v4i_t{0, 0, 0, 0};
         }
-    uint4 a[D][TPW][2], x[D][2];
-    auto fetch = [&](int d, uint32_t q) {
-        if (q >= M.nq)
-            return;
+    uint4 a[D][TPW][2], x[D][UPW];
+    auto fetch = [&](int d, uint32_t q_) {
+        const uint32_t q = min(q_, M.nq - 1);
 #pragma unroll
         for (int t = 0; t < TPW; ++t)
 #pragma unroll
             for (int b = 0; b < 2; ++b)
                 a[d][t][b] = M.pack[(((wave * TPW + t) * M.nq + q) * 2 + b) * 64 + lane];
-        if (loader)
-            in.load<SYN>(mine, q, h, x[d][0], x[d][1]);
+#pragma unroll
+        for (int i = 0; i < UPW; ++i) {  // unit u: half u % 2 of group u / 2
+            const uint32_t u = (wave * UPW + i) % (CG * 2);
+            x[d][i] = in.load8<SYN>(min(cw0 + (u / 2) * 16 + c, count - 1), q, 2 * h + u % 2);
+        }
     };
     auto stage = [&](int d, uint32_t q) {
-        if (loader && q < M.nq) {
-            v4i_t lo, hi;
-            contract_limbs(x[d][0], x[d][1], lo, hi);
-            s_x[q & 1][wave][0][lane] = make_uint4((uint32_t)lo[0], (uint32_t)lo[1], (uint32_t)lo[2], (uint32_t)lo[3]);
-            s_x[q & 1][wave][1][lane] = make_uint4((uint32_t)hi[0], (uint32_t)hi[1], (uint32_t)hi[2], (uint32_t)hi[3]);
+        if (wave * UPW >= CG * 2)
+            return;
+#pragma unroll
+        for (int i = 0; i < UPW; ++i) {
+            const uint32_t u = wave * UPW + i;
+            const uint4 v = x[d][i];
+            auto limb = [&](uint32_t sel) {
+                return make_uint2(__builtin_amdgcn_perm(v.y, v.x, sel) ^ 0x80808080u,
+                                  __builtin_amdgcn_perm(v.w, v.z, sel) ^ 0x80808080u);
+            };
+            reinterpret_cast<uint2 *>(&s_x[q & 1][u / 2][0][lane])[u % 2] = limb(0x06040200u);
+            reinterpret_cast<uint2 *>(&s_x[q & 1][u / 2][1][lane])[u % 2] = limb(0x07050301u);
         }
     };
 #pragma unroll
@@ -2192,6 +2249,12 @@ __device__ inline int32_t mad24(int32_t a, int32_t b, int32_t c)
     asm("v_mad_i32_i24 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
     return r;
 }
+// v in a register of its own: a sum with it stays an add (2.9 clocks a wave; as a multiply-add 4.7)
+__device__ inline int32_t held(int32_t v)
+{
+    asm("" : "+v"(v));
+    return v;
+}
 __device__ inline int32_t fold2(int32_t y) { return fold16(fold16(y)); }
 // a b mod p in [-32769, 32768] for |a|, |b| <= 32769
 __device__ inline int32_t bal_mul(int32_t a, int32_t b) { return fold2(mad24(a, b, RBIAS)) - RBIAS; }
@@ -2235,7 +2298,7 @@ struct LaneSolve {
     __device__ void update(int32_t n0, int32_t n1)
     {
         constexpr int y = S_ & 1, x = y ^ 1;
-        const int32_t k1 = SAFE ? -RBIAS * n1 : 0, k0 = SAFE ? -RBIAS * n0 : -RBIAS * (n0 + n1);
+        const int32_t k1 = SAFE ? -RBIAS * n1 : 0, k0 = held(SAFE ? -RBIAS * n0 : -RBIAS * (n0 + n1));
 #pragma unroll
         for (int i = 0; i <= E - 1 - S_; ++i)
             R[y][i] = lane_update<SAFE>(R[y][i], R[x][i], i ? R[x][i - 1] : RBIAS, n0, n1, k0, k1);
@@ -2332,8 +2395,11 @@ struct LaneSolve {
 // residue two byte limbs miss; a locator holding it is multiplied by 3, which moves no root), plus
 // a_0. B operand of one MFMA: quarter h of the lanes holds limb h / 2 of coefficients (h & 1) half.
 struct RootTab {
-    const uint64_t *pack;  // tile * 64 + lane: 8 bytes of the A operand
-    const int4 *row;       // tile * 4 + h: sum_i g1 of positions 16 tile + 4 h .. +4
+    // A operands of the position tiles: low then high limbs of T coefficients (16 of each for
+    // ecc_len <= 32: one product of 32 bytes, 8 a lane; above 2 T / 64 products of 64, 16 a lane)
+    const uint64_t *pack;
+    const int4 *row;      // tile * 4 + h: sum_i g1 of positions 16 tile + 4 h .. +4
+    const int32_t *pow3;  // 3^i, i <= T, balanced
 };
 
 constexpr uint32_t lane_repair_words(int T) { return 64u * (T + 1) + 64u * (uint32_t)(T < 8 ? 8 : T) + 64u; }
@@ -2517,8 +2583,41 @@ __global__ __launch_bounds__(64, 4) void rsi16_repair_lane_kernel(uint16_t *__re
     }
 }
 
-// The codewords list[1 .. list[0]] through the general register repair, one per wave: a few in a
-// launch of many, so what counts is the time of one.
+constexpr uint8_t ODD = 254, ODD_SOLVED = 253;  // transient statuses of listed codewords (ecc_len >= 64)
+
+// The codewords list[1 .. list[0]] through the general register repair, one per wave (worker
+// `first` of `step`): a few in a launch of many, so what counts is the time of one.
+template <int E>
+__device__ inline void repair_listed(uint16_t *msgs, uint16_t *eccs, uint8_t *status, const Rsi16Dev &T,
+                                     const uint32_t *syn, const uint32_t *list, uint32_t *lds, uint32_t first,
+                                     uint32_t step)
+{
+    if (first >= list[0])
+        return;
+    LaneR<E, true> L;
+    L.init(T, threadIdx.x);
+    for (uint32_t i = first; i < list[0]; i += step) {
+        const uint32_t cw = list[1 + i];
+        uint16_t *m = msgs + (size_t)cw * T.k, *e = eccs + (size_t)cw * E;
+        const uint32_t *row = syn + (size_t)cw * E;
+        if (E >= 64 && status[cw] == ODD_SOLVED) {  // rsi16_solve_wave_kernel left locator and evaluator
+            const uint16_t *ev = reinterpret_cast<const uint16_t *>(row), *lo = ev + E;
+            const uint32_t inv0 = T.inv_tab[lo[0]];
+            PR<E> loc, syn_;
+#pragma unroll
+            for (int h = 0; h < RegShape<E>::C; ++h) {
+                const uint32_t i = L.gl + (uint32_t)h * RegShape<E>::G;
+                syn_.v[h] = F::mul(ev[i], inv0);
+                loc.v[h] = i <= (uint32_t)E / 2 ? F::mul(lo[i], inv0) : 0u;
+            }
+            repair_finish_reg<E, true>(T, m, e, lds, L, status + cw, loc, syn_, row[3 * E / 4 + 1]);
+        } else {
+            repair_group_reg<E, true, true>(T, m, e, lds, L, status + cw, row);
+        }
+        wave_sync();
+    }
+}
+
 template <int E>
 __global__ __launch_bounds__(64) void rsi16_repair_list_kernel(uint16_t *__restrict__ msgs, uint16_t *__restrict__ eccs,
                                                                uint8_t *__restrict__ status, Rsi16Dev T,
@@ -2526,16 +2625,538 @@ __global__ __launch_bounds__(64) void rsi16_repair_list_kernel(uint16_t *__restr
                                                                const uint32_t *__restrict__ list)
 {
     __shared__ uint32_t s_mem[REG_WORDS * E];
-    if (blockIdx.x >= list[0])
-        return;
-    LaneR<E> L;
-    L.init(T, threadIdx.x);
-    for (uint32_t i = blockIdx.x; i < list[0]; i += gridDim.x) {
-        const uint32_t cw = list[1 + i];
-        repair_group_reg<E, true, true>(T, msgs + (size_t)cw * T.k, eccs + (size_t)cw * E, s_mem, L, status + cw,
-                                        syn + (size_t)cw * E);
-        wave_sync();
+    repair_listed<E>(msgs, eccs, status, T, syn, list, s_mem, blockIdx.x, gridDim.x);
+}
+
+// ---------------------------------------------------------------- repair, one wave per key equation
+
+// ecc_len 64 to 256: the usual steps of LaneSolve with one wave per codeword, each lane holding E / 64
+// consecutive remainder coefficients and the locator's a_1 .. a_T (T = E / 2) spread likewise. A
+// coefficient's lower neighbour is the lane's own register or one wave_shr away; indexes and lengths
+// are scalar work. Irregular steps (irregular()) stay here too. The codeword's row of syndromes (E
+// words) is replaced by what the root search needs, a record of 3 T / 2 + 1 words:
+//   bytes   a_i 3^i, i = 1 .. T, as low and high int8 limbs (T bytes each; RootTab)
+//   int16   evaluator coefficients 0 .. T - 1, then i a_i (the locator's derivative), i = 1 .. T
+//   word    a_0 + 65536 * steps
+// and status set to 2 (to be searched). Codewords that took irregular steps can have longer evaluators;
+// they are listed for the general root search with status ODD_SOLVED and a row of 3 T / 2 + 2 words:
+//   u16     evaluator coefficients 0 .. E - 1, then a_0 .. a_T; a last word with the locator's length
+// Those left unsolved keep their syndromes and are listed with status ODD.
+template <int E>
+struct WaveSolve {
+    static constexpr int T = E / 2, C = E / 64, CA = C > 1 ? C / 2 : 1;
+    int32_t R[2][C];   // remainder coefficients C lane + h, biased
+    int32_t A[2][CA];  // locator coefficients 1 + CA lane + h, biased
+    int32_t A0[2];     // its constant coefficient, biased
+
+    template <int H>
+    __device__ static int32_t get(const int32_t (&v)[C], uint32_t idx)  // coefficient idx, idx % C == H
+    {
+        return __builtin_amdgcn_readlane(v[H], (int)(idx / C)) - RBIAS;
     }
+    __device__ static int32_t get_any(const int32_t (&v)[C], uint32_t idx)
+    {
+        int32_t r = 0;
+#pragma unroll
+        for (int h = 0; h < C; ++h) {
+            const int32_t x = __builtin_amdgcn_readlane(v[h], (int)(idx / C));
+            r = idx % C == (uint32_t)h ? x : r;
+        }
+        return r - RBIAS;
+    }
+    __device__ static int32_t shr(int32_t v, int32_t first)  // the lane below's v, `first` in lane 0
+    {
+        return __builtin_amdgcn_update_dpp(first, v, 0x138, 0xf, 0xf, false);  // wave_shr:1
+    }
+
+    template <bool SAFE, int Y>
+    __device__ void update(int32_t n0, int32_t n1)
+    {
+        constexpr int X = Y ^ 1;
+        const int32_t k1 = SAFE ? -RBIAS * n1 : 0, k0 = held(SAFE ? -RBIAS * n0 : -RBIAS * (n0 + n1));
+        const int32_t rp = shr(R[X][C - 1], RBIAS), ap = shr(A[X][CA - 1], A0[X]);
+#pragma unroll
+        for (int h = 0; h < C; ++h)
+            R[Y][h] = lane_update<SAFE>(R[Y][h], R[X][h], h ? R[X][h - 1] : rp, n0, n1, k0, k1);
+#pragma unroll
+        for (int h = 0; h < CA; ++h)
+            A[Y][h] = lane_update<SAFE>(A[Y][h], A[X][h], h ? A[X][h - 1] : ap, n0, n1, k0, k1);
+        A0[Y] = fold2(mad24(n0, A0[X] - RBIAS, A0[Y]));
+    }
+
+    __device__ static uint32_t length(const int32_t (&v)[C])
+    {
+        uint32_t len = 0;
+#pragma unroll
+        for (int h = 0; h < C; ++h) {
+            const uint64_t m = __ballot(v[h] != RBIAS);
+            if (m)
+                len = max(len, (uint32_t)(C * (63 - __builtin_clzll(m)) + h + 1));
+        }
+        return len;
+    }
+
+    // The regular steps from the syndromes in R[0]: the steps done, the last remainder in R[steps & 1]
+    // (0 where the last syndrome is 0).
+    __device__ uint32_t solve(const uint32_t *__restrict__ inv_tab)
+    {
+        constexpr int U = C > 2 ? C : 2;
+#pragma unroll
+        for (int h = 0; h < C; ++h)
+            R[1][h] = RBIAS;
+#pragma unroll
+        for (int h = 0; h < CA; ++h)
+            A[0][h] = A[1][h] = RBIAS;
+        A0[0] = RBIAS + 1;
+        A0[1] = RBIAS;
+        // leading coefficients of the divisor (r1h, r1s) and of the dividend (h1, h2)
+        int32_t h1 = get<C - 1>(R[0], E - 1), h2 = get<(E - 2) % C>(R[0], E - 2);
+        if (h1 == 0)
+            return 0;
+        {  // the first step, x^E against the syndromes
+            const int32_t a11 = -bal_inv(inv_tab, h1), a10 = bal_mul(h2, bal_mul(a11, a11));
+            const int32_t rp = shr(R[0][C - 1], RBIAS);
+#pragma unroll
+            for (int h = 0; h < C; ++h)
+                R[1][h] = lane_update<true>(RBIAS, R[0][h], h ? R[0][h - 1] : rp, a10, a11, -RBIAS * a10, -RBIAS * a11);
+            A0[1] = a10 + RBIAS;
+            if ((threadIdx.x & 63) == 0)
+                A[1][0] = fold16(a11 + RBIAS);
+        }
+        int32_t r1h = get<(E - 2) % C>(R[1], E - 2);
+        if (r1h == 0)
+            return 1;
+        for (uint32_t s0 = 2; s0 <= (uint32_t)T; s0 += U) {
+            uint32_t done = 0;
+            auto one = [&](auto u_) {
+                constexpr int u = decltype(u_)::value, Y = u & 1, X = Y ^ 1;
+                const uint32_t s = s0 + u;
+                if (done || s > (uint32_t)T)
+                    return;
+                const int32_t r1s = get<(2 * C - 3 - u % C) % C>(R[X], E - 1 - s);
+                const int32_t a0 = bal_inv(inv_tab, r1h), w = bal_mul(a0, r1s);
+                const int32_t n1 = -bal_mul(a0, h1);
+                const int32_t n0 = bal_mul(a0, fold2(mad24(w, h1, RBIAS - h2)) - RBIAS);
+                if (__any(max(abs(n0), abs(n1)) > 32766))
+                    update<true, Y>(n0, n1);
+                else
+                    update<false, Y>(n0, n1);
+                h1 = r1h;
+                h2 = r1s;
+                r1h = get<(2 * C - 3 - u % C) % C>(R[Y], E - 1 - s);
+                if (r1h == 0)
+                    done = s;
+            };
+            one(std::integral_constant<int, 0>{});
+            one(std::integral_constant<int, 1>{});
+            if constexpr (U > 2) {
+                one(std::integral_constant<int, 2>{});
+                one(std::integral_constant<int, 3>{});
+            }
+            if (done)
+                return done;
+        }
+        return T;
+    }
+
+    // The steps after an irregular one (the remainder of step s, of length g >= T, is shorter than
+    // regular), as pr_sugiyama: r1 and a1 in R[1], A[1], r2 and a2 in R[0], A[0] on entry and return.
+    // The polynomials' degrees stay below their lengths' bounds here, so no product wraps mod x^E - 1
+    // and the coefficients above a length are zero. With the quotient of three terms pr_sugiyama's
+    // (2 - a v) is 1, 0, v2' = -(a0 v2 + c1 v1), and the quotient's coefficients, b = {a0 v2', c1, a0}
+    // against r2, do not cancel the leading terms: the lengths then alternate until the steps end.
+    // False where the codeword needs the general code (a raise, another quotient length, a locator
+    // of more than T + 1 coefficients).
+    __device__ bool irregular(uint32_t s, uint32_t r2_len, uint32_t r1_len, const uint32_t *__restrict__ inv_tab)
+    {
+        uint32_t a1_deg = s, a2_deg = s - 1;
+        for (++s; s <= (uint32_t)T; ++s) {
+            if (r1_len < (uint32_t)T)
+                return div_ok(E, r2_len, r1_len);
+            const uint32_t g = r1_len;
+            if (r2_len >= g) {
+                if (r2_len != g + 1 && r2_len != g + 2)
+                    return false;
+                const uint32_t q_deg = r2_len - g;
+                const int32_t a0 = bal_inv(inv_tab, get_any(R[1], g - 1));
+                const int32_t v1 = get_any(R[1], g - 2), f0 = get_any(R[0], g), f1 = get_any(R[0], g - 1);
+                int32_t n[3];  // minus the quotient
+                if (q_deg == 1) {
+                    const int32_t w = bal_mul(a0, v1);
+                    n[0] = bal_mul(a0, fold2(mad24(w, f0, RBIAS - f1)) - RBIAS);
+                    n[1] = -bal_mul(a0, f0);
+                    n[2] = 0;
+                } else {
+                    const int32_t v2 = get_any(R[1], g - 3), up = get_any(R[0], g + 1), f2 = get_any(R[0], g - 2);
+                    const int32_t c1 = -bal_mul(bal_mul(a0, a0), v1);
+                    const int32_t b0 = -bal_mul(a0, fold2(mad24(c1, v1, RBIAS + bal_mul(a0, v2))) - RBIAS);
+                    auto dot = [&](int32_t x, int32_t y, int32_t z) {  // b0 x + c1 y + a0 z
+                        return fold2(mad24(a0, z, fold2(mad24(c1, y, fold2(mad24(b0, x, RBIAS)))))) - RBIAS;
+                    };
+                    n[0] = -dot(f0, f1, f2);
+                    n[1] = -dot(up, f0, f1);
+                    n[2] = -dot(0, up, f0);
+                }
+                a2_deg = max(a2_deg, a1_deg + q_deg);
+                if (a2_deg > (uint32_t)T)
+                    return false;
+                // r2, a2 += n r1, n a1
+                int32_t x[C], xa[CA], x0 = A0[1];
+#pragma unroll
+                for (int h = 0; h < C; ++h)
+                    x[h] = R[1][h];
+#pragma unroll
+                for (int h = 0; h < CA; ++h)
+                    xa[h] = A[1][h];
+#pragma unroll
+                for (int u = 0; u < 3; ++u) {
+                    const int32_t k = -RBIAS * n[u];
+#pragma unroll
+                    for (int h = 0; h < C; ++h)
+                        R[0][h] = fold2(mad24(n[u], x[h], R[0][h] + k));
+#pragma unroll
+                    for (int h = 0; h < CA; ++h)
+                        A[0][h] = fold2(mad24(n[u], xa[h], A[0][h] + k));
+                    A0[0] = fold2(mad24(n[u], x0, A0[0] + k));
+                    const int32_t rp = shr(x[C - 1], RBIAS), ap = shr(xa[CA - 1], x0);  // times x
+#pragma unroll
+                    for (int h = C - 1; h > 0; --h)
+                        x[h] = x[h - 1];
+                    x[0] = rp;
+#pragma unroll
+                    for (int h = CA - 1; h > 0; --h)
+                        xa[h] = xa[h - 1];
+                    xa[0] = ap;
+                    x0 = RBIAS;
+                }
+            }
+            auto swap = [](auto &p, auto &q) {
+                const auto v = p;
+                p = q;
+                q = v;
+            };
+#pragma unroll
+            for (int h = 0; h < C; ++h)
+                swap(R[0][h], R[1][h]);
+#pragma unroll
+            for (int h = 0; h < CA; ++h)
+                swap(A[0][h], A[1][h]);
+            swap(A0[0], A0[1]);
+            swap(a1_deg, a2_deg);
+            r2_len = r1_len;
+            r1_len = length(R[1]);
+        }
+        return true;
+    }
+};
+
+// 16,384 RSi16(4096,256) codewords with 0-128 errors in 190 us (E / 4 + E / 8 coefficients of five
+// vector instructions a step, about 25 more for the quotient); the shuffles, table loads and lengths of
+// the general kernel's steps took about 1.1 ms.
+template <int E>
+__global__ __launch_bounds__(64) void rsi16_solve_wave_kernel(uint32_t count, uint8_t *__restrict__ status, Rsi16Dev D,
+                                                              const int32_t *__restrict__ pow3,
+                                                              uint32_t *__restrict__ syn, uint32_t *__restrict__ list)
+{
+    using W = WaveSolve<E>;
+    constexpr int T = W::T, C = W::C, CA = W::CA;
+    const uint32_t lane = threadIdx.x, cw = blockIdx.x;
+    uint32_t *row = syn + (size_t)cw * E;
+    W S;
+    uint32_t any = 0;
+#pragma unroll
+    for (int h = 0; h < C; ++h) {
+        const uint32_t v = row[C * lane + h];
+        any |= v;
+        S.R[0][h] = fold16((int32_t)v + RBIAS);
+    }
+    if (__ballot(any != 0) == 0) {
+        if (lane == 0)
+            status[cw] = FFRS_RSI16_NO_ERRORS;
+        return;
+    }
+    uint32_t steps = S.solve(D.inv_tab);
+    bool solved = steps != 0, odd = false;
+    if (steps & 1) {  // the results in R[1], A[1]
+    } else {
+#pragma unroll
+        for (int h = 0; h < C; ++h) {
+            const int32_t v = S.R[0][h];
+            S.R[0][h] = S.R[1][h];
+            S.R[1][h] = v;
+        }
+#pragma unroll
+        for (int h = 0; h < CA; ++h) {
+            const int32_t v = S.A[0][h];
+            S.A[0][h] = S.A[1][h];
+            S.A[1][h] = v;
+        }
+        const int32_t v = S.A0[0];
+        S.A0[0] = S.A0[1];
+        S.A0[1] = v;
+    }
+    if (solved && steps < (uint32_t)T) {
+        const uint32_t len = W::length(S.R[1]);
+        odd = len >= (uint32_t)T;
+        if (odd)
+            solved = S.irregular(steps, E + 1 - steps, len, D.inv_tab);
+        else
+            solved = len != 0;
+    }
+    int32_t a0 = S.A0[1] - RBIAS, a[CA], r[C], v[CA], d[CA];
+#pragma unroll
+    for (int h = 0; h < CA; ++h)
+        a[h] = S.A[1][h] - RBIAS;
+#pragma unroll
+    for (int h = 0; h < C; ++h)
+        r[h] = S.R[1][h] - RBIAS;
+    solved = solved && a0 != 0;
+    // Stored int16 miss 32768, u16 65536 and the limbs 32640: another multiple then
+    const bool has_a = CA * lane < (uint32_t)T, has_r = C * lane < (uint32_t)T;
+    for (int tries = 0; solved; ++tries) {
+        bool bad = a0 == -1;
+#pragma unroll
+        for (int h = 0; h < CA; ++h) {
+            const int32_t i = CA * (int32_t)lane + h + 1;
+            const int32_t x = bal_mul(a[h], has_a ? pow3[i] : 0);
+            v[h] = x > 32639 ? x - (int32_t)P16 : x;
+            d[h] = bal_mul(a[h], i);
+            bad |= odd ? a[h] == -1 : has_a && (x == 32640 || d[h] == 32768 || d[h] == -32769);
+        }
+#pragma unroll
+        for (int h = 0; h < C; ++h)
+            bad |= odd ? r[h] == -1 : has_r && (r[h] == 32768 || r[h] == -32769);
+        if (__ballot(bad) == 0)
+            break;
+        solved = tries < 64;
+        a0 = bal_mul(a0, 3);
+#pragma unroll
+        for (int h = 0; h < CA; ++h)
+            a[h] = bal_mul(a[h], 3);
+#pragma unroll
+        for (int h = 0; h < C; ++h)
+            r[h] = bal_mul(r[h], 3);
+    }
+    if (!solved || odd) {
+        uint16_t *ev = reinterpret_cast<uint16_t *>(row), *lo = reinterpret_cast<uint16_t *>(row + T);
+        if (solved) {
+            uint32_t len = 1;
+#pragma unroll
+            for (int h = 0; h < CA; ++h) {
+                const uint64_t m = __ballot(a[h] != 0);
+                if (m)
+                    len = max(len, (uint32_t)(CA * (63 - __builtin_clzll(m)) + h + 2));
+                if (has_a)
+                    lo[1 + CA * lane + h] = (uint16_t)bal_canon(a[h]);
+            }
+#pragma unroll
+            for (int h = 0; h < C; ++h)
+                ev[C * lane + h] = (uint16_t)bal_canon(r[h]);
+            if (lane == 0) {
+                lo[0] = (uint16_t)bal_canon(a0);
+                row[3 * T / 2 + 1] = len;
+            }
+        }
+        if (lane == 0) {
+            list[1 + atomicAdd(list, 1u)] = cw;
+            status[cw] = solved ? ODD_SOLVED : ODD;
+        }
+        return;
+    }
+    uint8_t *lim = reinterpret_cast<uint8_t *>(row);
+    int16_t *ev = reinterpret_cast<int16_t *>(row + T / 2), *de = reinterpret_cast<int16_t *>(row + T);
+    if (has_a) {
+#pragma unroll
+        for (int h = 0; h < CA; ++h) {
+            const uint32_t t = (uint32_t)((v[h] + 0x80) ^ 0x80);
+            lim[CA * lane + h] = (uint8_t)t;
+            lim[T + CA * lane + h] = (uint8_t)(t >> 8);
+            de[CA * lane + h] = (int16_t)d[h];
+        }
+    }
+    if (has_r)
+#pragma unroll
+        for (int h = 0; h < C; ++h)
+            ev[C * lane + h] = (int16_t)r[h];
+    if (lane == 0) {
+        row[3 * T / 2] = bal_canon(a0) | (steps << 16);
+        status[cw] = FFRS_RSI16_REPAIR_OK;
+    }
+}
+
+// Roots and corrections for ecc_len 64 to 256: a workgroup of eight waves takes 16 CG codewords whose
+// limbs stay in registers (B operands) while the waves go through the tiles of 16 positions; the
+// roots are listed in LDS and corrected one per lane from the evaluator and derivative staged there.
+// The contraction's K bytes are the low then the high limbs of the T coefficients, 2 T / 64 products
+// of 64 for either sum: P0 pairs the matrix limbs (g0 | g1) with (lo | ~hi), P1 with (hi | lo).
+// The first list_blocks workgroups take the odd codewords meanwhile (list[1 .. list[0]], one at a
+// time through the general repair, whose latency would otherwise come on top).
+template <int E, int CG>
+__global__ __launch_bounds__(512) void rsi16_roots_wave_kernel(uint16_t *__restrict__ msgs, uint16_t *__restrict__ eccs,
+                                                               uint32_t count, uint8_t *__restrict__ status, Rsi16Dev D,
+                                                               RootTab RT, const uint32_t *__restrict__ rec,
+                                                               const uint32_t *__restrict__ list, uint32_t list_blocks)
+{
+    constexpr uint32_t NW = 8;
+    constexpr int T = E / 2, KF = 2 * T / 64, CW = 16 * CG, WORDS = T + 1;  // T / 2 words of either, odd stride
+    __shared__ uint32_t s_co[CW * WORDS];
+    __shared__ uint32_t s_last[CW];        // a_0 + 65536 * steps
+    __shared__ uint32_t s_found[CW];
+    __shared__ uint32_t s_list[CW * T < REG_WORDS * E ? REG_WORDS * E : CW * T];
+    __shared__ uint32_t s_total;
+    const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c = lane & 15, h = lane >> 4;
+    if (blockIdx.x < list_blocks) {
+        if (wave == 0)
+            repair_listed<E>(msgs, eccs, status, D, rec, list, s_list, blockIdx.x, list_blocks);
+        return;
+    }
+    const uint32_t cw0 = (blockIdx.x - list_blocks) * CW;
+    for (uint32_t i = threadIdx.x; i < (uint32_t)CW * T; i += 64 * NW) {
+        const uint32_t w = i / T, j = i % T;
+        s_co[w * WORDS + j] = rec[(size_t)min(cw0 + w, count - 1) * E + T / 2 + j];
+    }
+    if (threadIdx.x < CW) {
+        const uint32_t cw = min(cw0 + threadIdx.x, count - 1);
+        const bool on = cw0 + threadIdx.x < count && status[cw] == FFRS_RSI16_REPAIR_OK;
+        s_last[threadIdx.x] = on ? rec[(size_t)cw * E + 3 * T / 2] : 1u;  // the constant 1: no roots
+        s_found[threadIdx.x] = on ? 0u : 1u;
+    }
+    if (threadIdx.x == 0)
+        s_total = 0;
+    v4i_t lo[CG][KF], alt[CG][KF];  // P0's operands, P1's (KF == 1; else they are lo's in another order)
+    int32_t loc0[CG];
+    __syncthreads();
+#pragma unroll
+    for (int g = 0; g < CG; ++g) {
+        const uint32_t w = 16 * g + c, cw = min(cw0 + w, count - 1);
+        const bool on = (s_found[w] & 1) == 0;
+        const uint4 *lim = reinterpret_cast<const uint4 *>(rec + (size_t)cw * E);
+#pragma unroll
+        for (int f = 0; f < KF; ++f) {
+            lo[g][f] = as_v4i(lim[4 * f + h]) & (on ? -1 : 0);
+            if constexpr (KF == 1)
+                alt[g][f] = as_v4i(lim[h ^ 2]) & (on ? -1 : 0);
+        }
+        loc0[g] = (int32_t)(s_last[w] & 0xffffu);
+    }
+    __syncthreads();  // s_found is read before the root search writes it
+    const uint4 *pack = reinterpret_cast<const uint4 *>(RT.pack);
+    const uint32_t tiles = (D.n + 15) / 16;
+    const int32_t flip = h >= 2 ? -1 : 0;  // KF == 1: quarters 2 and 3 hold the high limbs
+    uint4 an[KF];
+    int4 kn;
+    if (wave < tiles) {
+#pragma unroll
+        for (int f = 0; f < KF; ++f)
+            an[f] = pack[(wave * KF + f) * 64 + lane];
+        kn = RT.row[wave * 4 + h];
+    }
+    for (uint32_t t = wave; t < tiles; t += NW) {
+        v4i_t a[KF];
+#pragma unroll
+        for (int f = 0; f < KF; ++f)
+            a[f] = as_v4i(an[f]);
+        const int4 kc = kn;
+        if (t + NW < tiles) {
+#pragma unroll
+            for (int f = 0; f < KF; ++f)
+                an[f] = pack[((t + NW) * KF + f) * 64 + lane];
+            kn = RT.row[(t + NW) * 4 + h];
+        }
+        v4i_t p0[CG], p1[CG];
+#pragma unroll
+        for (int g = 0; g < CG; ++g) {
+            p0[g] = v4i_t{kc.x + loc0[g], kc.y + loc0[g], kc.z + loc0[g], kc.w + loc0[g]};
+            p1[g] = v4i_t{0, 0, 0, 0};
+        }
+#pragma unroll
+        for (int f = 0; f < KF; ++f)
+#pragma unroll
+            for (int g = 0; g < CG; ++g) {
+                const v4i_t b0 = KF == 1 ? lo[g][f] ^ flip : 2 * f >= KF ? ~lo[g][f] : lo[g][f];
+                const v4i_t b1 = KF == 1 ? alt[g][f] : lo[g][(f + KF / 2) % KF];
+                p0[g] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[f], b0, p0[g], 0, 0, 0);
+                p1[g] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[f], b1, p1[g], 0, 0, 0);
+            }
+        uint32_t hits = 0;  // this lane's 4 CG values, the first in the highest bit
+#pragma unroll
+        for (int g = 0; g < CG; ++g)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int32_t f = fold2(p0[g][i] + 256 * p1[g][i]);  // |p1| <= 2^22; 0 at a root alone
+                asm("v_cmp_eq_u32 vcc, 0, %1\n\tv_addc_co_u32 %0, vcc, %0, %0, vcc" : "+v"(hits) : "v"(f) : "vcc");
+            }
+        while (hits) {
+            const uint32_t v = (uint32_t)__builtin_clz(hits) - (32 - 4 * CG), w = 16 * (v >> 2) + c;
+            hits &= ~((1u << (4 * CG - 1)) >> v);
+            const uint32_t at = atomicAdd(&s_total, 1u);
+            if (at < (uint32_t)CW * T)
+                s_list[at] = (w << 16) | (16 * t + 4 * h + (v & 3));
+            s_found[w] = 1;
+        }
+    }
+    __syncthreads();
+    const uint32_t total = min(s_total, (uint32_t)CW * T);  // at most T roots a codeword
+    // a root's operands, loaded a round ahead
+    struct Root {
+        uint32_t w, x, xi, sym;
+        uint16_t *at;
+    };
+    auto fetch = [&](uint32_t q) {
+        const uint32_t v = s_list[min(q, total - 1)], pos = v & 0xffffu, ri = rbo_bits(pos, D.nbits);
+        Root r;
+        r.w = v >> 16;
+        r.x = D.roots_ntt[ri];
+        r.xi = D.roots_ntt[(D.N - ri) & (D.N - 1)];
+        const size_t row = cw0 + r.w;
+        r.at = pos < D.k ? msgs + row * D.k + pos : eccs + row * E + (pos - D.k);
+        r.sym = *r.at;
+        return r;
+    };
+    Root next{};
+    if (total)
+        next = fetch(threadIdx.x);
+    for (uint32_t q = threadIdx.x; q < total; q += 64 * NW) {
+        const Root r = next;
+        next = fetch(q + 64 * NW);
+        const int32_t xb = (int32_t)r.xi > 32768 ? (int32_t)r.xi - (int32_t)P16 : (int32_t)r.xi;
+        const int32_t x2 = bal_mul(xb, xb);
+        const uint32_t *co = s_co + r.w * WORDS;
+        // both have degree below steps; in blocks of four pairs, whose coefficients are read at once
+        const int32_t pairs = (int32_t)(((s_last[r.w] >> 16) + 7) / 8) * 4;
+        int32_t nb = RBIAS, db = RBIAS;
+        if (__any(max(abs(xb), abs(x2)) > 32766)) {
+            for (int32_t j = pairs; j-- > 0;) {
+                const int32_t u = (int32_t)co[j], d = (int32_t)co[T / 2 + j];
+                nb = fold2(mad24(nb - RBIAS, xb, (u >> 16) + RBIAS));
+                nb = fold2(mad24(nb - RBIAS, xb, (int16_t)u + RBIAS));
+                db = fold2(mad24(db - RBIAS, xb, (d >> 16) + RBIAS));
+                db = fold2(mad24(db - RBIAS, xb, (int16_t)d + RBIAS));
+            }
+        } else {  // two terms at once: |s x^2 + c1 x + c0 + 32768| < 2^31
+            const int32_t kx = held(RBIAS - RBIAS * x2);
+            for (int32_t j = pairs; j > 0; j -= 4) {
+                int32_t u[4], d[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    u[i] = (int32_t)co[j - 1 - i];
+                    d[i] = (int32_t)co[T / 2 + j - 1 - i];
+                }
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    nb = fold2(mad24(nb, x2, mad24(u[i] >> 16, xb, (int16_t)u[i] + kx)));
+                    db = fold2(mad24(db, x2, mad24(d[i] >> 16, xb, (int16_t)d[i] + kx)));
+                }
+            }
+        }
+        // _forney (rsi16v_impl.hpp:500-512), as in rsi16_repair_lane_kernel
+        const uint32_t nc = bal_canon(nb - RBIAS), dc = bal_canon(db - RBIAS);
+        const uint32_t scale = D.inv_tab[dc ? dc : s_last[r.w] & 0xffffu];
+        const uint32_t err = F::mul(nc ? F::mul(nc, scale) : 0u, r.x);
+        *r.at = (uint16_t)(F::add(r.sym, err) & 0xffff);
+    }
+    if (threadIdx.x < CW && s_found[threadIdx.x] == 0)
+        status[cw0 + threadIdx.x] = FFRS_RSI16_ERROR_LOCATION_FAIL;
 }
 
 // ---------------------------------------------------------------- interleaved repair, SIMD words
@@ -3344,7 +3965,7 @@ struct ffrs_rsi16 {
     struct {
         void *d = nullptr;
         RootTab dev{};
-    } roots;                         // the locator's values at the n positions (ecc_len 8 to 32)
+    } roots;                         // the locator's values at the n positions
     bool mix_minus_one = false;      // a mix constant is 65536: the SIMD words are not the linear map
     int encode_mode = 0;             // 0 automatic, 1 butterflies, 2 MFMA wherever it applies
     uint32_t *d_syn = nullptr;       // syndromes of the last repair launch
@@ -3532,7 +4153,8 @@ int launch_repair_reg(ffrs_rsi16 *rs, uint16_t *d_msg, uint16_t *d_ecc, size_t c
     // One codeword per wave while that leaves at most two waves per SIMD, the groups of the wave
     // sharing its chunks (us against the general kernel: 1 codeword RSi16(256,32) 10.4 / 14.6,
     // (1024,8) 12 / 78, (4096,32) 17 / 61; 2,048: 28 / 30, 18 / 89, 64 / 175; 16,384: 98 / 55).
-    if (E <= 32 && rs->repair_synd != 1 && count <= 8 * (size_t)rs->ctx->cu_count) {
+    if constexpr (E <= 32)
+    if (rs->repair_synd != 1 && count <= 8 * (size_t)rs->ctx->cu_count) {
         hipLaunchKernelGGL(rsi16_repair_one_kernel<E>, dim3((unsigned)count), dim3(64), 0, rs->ctx->stream, d_msg, d_ecc,
                            d_status, rs->dev);
         FFRS_HIP(hipGetLastError());
@@ -3576,11 +4198,20 @@ int launch_repair_reg(ffrs_rsi16 *rs, uint16_t *d_msg, uint16_t *d_ecc, size_t c
                 mark_kernel(rs->ctx);
                 hipLaunchKernelGGL(rsi16_repair_list_kernel<E>, dim3((unsigned)std::min<size_t>(1024, c)), dim3(64), 0,
                                    rs->ctx->stream, m, e, d_status + b, rs->dev, syn, list);
-            } else {
-                if (int r = allow_lds(rsi16_repair_reg_kernel<E, true>, lds))
-                    return r;
-                hipLaunchKernelGGL((rsi16_repair_reg_kernel<E, true>), dim3((unsigned)((c + cpw - 1) / cpw)), dim3(64),
-                                   lds, rs->ctx->stream, m, e, (uint32_t)c, d_status + b, rs->dev, syn);
+            } else if constexpr (E >= 64) {
+                hipLaunchKernelGGL(rsi16_solve_wave_kernel<E>, dim3((unsigned)c), dim3(64), 0, rs->ctx->stream,
+                                   (uint32_t)c, d_status + b, rs->dev, rs->roots.dev.pow3, syn, list);
+                FFRS_HIP(hipGetLastError());
+                mark_kernel(rs->ctx);
+                const unsigned lb = (unsigned)std::min<size_t>(c, (size_t)rs->ctx->cu_count);
+                if ((c + 31) / 32 >= 2 * (size_t)rs->ctx->cu_count)
+                    hipLaunchKernelGGL((rsi16_roots_wave_kernel<E, 2>), dim3(lb + (unsigned)((c + 31) / 32)), dim3(512), 0,
+                                       rs->ctx->stream, m, e, (uint32_t)c, d_status + b, rs->dev, rs->roots.dev, syn,
+                                       list, lb);
+                else
+                    hipLaunchKernelGGL((rsi16_roots_wave_kernel<E, 1>), dim3(lb + (unsigned)((c + 15) / 16)), dim3(512), 0,
+                                       rs->ctx->stream, m, e, (uint32_t)c, d_status + b, rs->dev, rs->roots.dev, syn,
+                                       list, lb);
             }
             FFRS_HIP(hipGetLastError());
             mark_kernel(rs->ctx);
@@ -3723,14 +4354,20 @@ int build_mfma_encode(ffrs_rsi16 *rs, const std::vector<uint32_t> &mix, const st
     return build_contract(&rs->enc, mat, E, nq, nq);
 }
 
-// The limbs of (w^-rbo(m) / 3)^i, i = 1 .. E / 2, for the lane repair's root search (RootTab);
+// The limbs of (w^-rbo(m) / 3)^i, i = 1 .. E / 2, for the root search (RootTab);
 // *ok = false where one of them is 32640 (not for block_len <= 32768: w^(rbo(m) i) 32640 is a
 // power of 3^(65536 / N), whose exponent no odd multiple of a power of two below it reaches).
 int build_roots(ffrs_rsi16 *rs, const std::vector<uint32_t> &roots_ntt, bool *ok)
 {
     const uint32_t n = rs->n, T = rs->E / 2, tiles = (n + 15) / 16, third = s_pow(3, 65535);
-    std::vector<uint8_t> pack((size_t)tiles * 64 * 8, 0);
-    std::vector<int32_t> row((size_t)tiles * 16, 0);
+    const uint32_t half = std::max<uint32_t>(16, T);          // coefficients of either limb
+    const uint32_t kb = T <= 16 ? 32 : 64, bl = kb / 4;       // bytes of a product, of a lane's share
+    std::vector<uint8_t> pack((size_t)tiles * 16 * 2 * half, 0);
+    std::vector<int32_t> row((size_t)tiles * 16, 0), pow3(T + 1);
+    auto slot = [&](uint32_t m, uint32_t kpos) -> uint8_t & {  // byte kpos of position m
+        const uint32_t f = kpos / kb, lane = m % 16 + 16 * (kpos % kb / bl);
+        return pack[(((size_t)(m / 16) * (2 * half / kb) + f) * 64 + lane) * bl + kpos % bl];
+    };
     for (uint32_t m = 0; m < n; ++m) {
         const uint32_t ri = rbo_bits(m, rs->nbits);
         const uint32_t x = S::mul(roots_ntt[(rs->N - ri) & (rs->N - 1)], third);
@@ -3741,23 +4378,27 @@ int build_roots(ffrs_rsi16 *rs, const std::vector<uint32_t> &roots_ntt, bool *ok
                 return FFRS_OK;
             const int32_t v = pw > 32639 ? (int32_t)pw - (int32_t)P16 : (int32_t)pw;
             const int32_t lo = ((v + 128) & 255) - 128, hi = (v - lo) >> 8;
-            uint8_t *p = &pack[((size_t)(m / 16) * 64 + m % 16 + 16 * (i / 8)) * 8 + i % 8];
-            p[0] = (uint8_t)lo;
-            p[32 * 8] = (uint8_t)hi;
+            slot(m, i) = (uint8_t)lo;
+            slot(m, half + i) = (uint8_t)hi;
             row[m] += hi;
         }
     }
+    for (uint32_t i = 0, v = 1; i <= T; ++i, v = S::mul(v, 3))
+        pow3[i] = v > 32768 ? (int32_t)v - (int32_t)P16 : (int32_t)v;
+    const size_t at_row = pack.size(), at_pow3 = at_row + row.size() * 4;
     char *d = nullptr;
-    hipError_t e = hipMalloc(&d, pack.size() + row.size() * 4);
+    hipError_t e = hipMalloc(&d, at_pow3 + pow3.size() * 4);
     if (e == hipSuccess) {
         rs->roots.d = d;
         e = hipMemcpy(d, pack.data(), pack.size(), hipMemcpyHostToDevice);
     }
     if (e == hipSuccess)
-        e = hipMemcpy(d + pack.size(), row.data(), row.size() * 4, hipMemcpyHostToDevice);
+        e = hipMemcpy(d + at_row, row.data(), row.size() * 4, hipMemcpyHostToDevice);
+    if (e == hipSuccess)
+        e = hipMemcpy(d + at_pow3, pow3.data(), pow3.size() * 4, hipMemcpyHostToDevice);
     if (e != hipSuccess)
         return fail(FFRS_ERR_DEVICE, "root search tables: %s", hipGetErrorString(e));
-    rs->roots.dev = RootTab{(const uint64_t *)d, (const int4 *)(d + pack.size())};
+    rs->roots.dev = RootTab{(const uint64_t *)d, (const int4 *)(d + at_row), (const int32_t *)(d + at_pow3)};
     *ok = true;
     return FFRS_OK;
 }
@@ -3780,13 +4421,11 @@ int build_mfma_synd(ffrs_rsi16 *rs, const std::vector<uint32_t> &roots_ntt)
             pw = S::mul(pw, x);
         }
     }
-    if (E <= 32) {
-        bool ok = false;
-        if (int r = build_roots(rs, roots_ntt, &ok))
-            return r;
-        if (!ok)
-            return FFRS_OK;
-    }
+    bool ok = false;
+    if (int r = build_roots(rs, roots_ntt, &ok))
+        return r;
+    if (!ok)
+        return FFRS_OK;
     return build_contract(&rs->synd, mat, E, nq, nqm);
 }
 
