@@ -3618,6 +3618,63 @@ __global__ __launch_bounds__(256) void rsi16_simd_writeback_kernel(const Rsi16De
     }
 }
 
+// ---------------------------------------------------------------- short parity, one wave per codeword
+
+// For ecc_len 2, 4 and 8 the syndromes and (with the conditions of the contraction, above) the parity
+// are a few sums over a long row: a wave takes a codeword, each lane every 64th symbol, with the map's
+// matrix as balanced words (row m: E of them). Where there are few codewords (a CIRC16 file has
+// hundreds to thousands of inner rows) a lane group or lane per codeword leaves the chip idle:
+// 1,024 rows of RSi16(2052,4) took 475 us (syndromes 516) with two lanes each, 6 here.
+template <int E, class TM>
+__device__ inline void row_accumulate(const TM *__restrict__ m, uint32_t count, const int32_t *__restrict__ tab,
+                                      uint32_t lane, int32_t (&acc)[E])
+{
+#pragma unroll 4
+    for (uint32_t i = lane; i < count; i += 64) {
+        int32_t c = (int32_t)m[i];
+        c = c > 32768 ? c - (int32_t)P16 : c;
+#pragma unroll
+        for (int j = 0; j < E; ++j)
+            acc[j] += fold16(c * tab[(size_t)i * E + j]);  // each in [-32767, 98303]; at most 1,024 a lane
+    }
+}
+
+// the wave's sums, canonical, in every lane
+template <int E>
+__device__ inline void row_reduce(int32_t (&acc)[E])
+{
+#pragma unroll
+    for (int j = 0; j < E; ++j) {
+        int32_t v = fold2(acc[j]);
+#pragma unroll
+        for (int s = 1; s < 64; s <<= 1)
+            v += __shfl_xor(v, s);
+        v = fold2(v);
+        acc[j] = v + ((v >> 31) & (int32_t)P16);
+    }
+}
+
+// parity (e == nullptr: & 0xFFFF where TO is u16) or syndromes of `rows` codewords, message q at
+// m + q k, parity at e + q E
+template <int E, class TM, class TO>
+__global__ __launch_bounds__(256) void rsi16_rows_kernel(const TM *__restrict__ m, const uint32_t *__restrict__ e,
+                                                         uint32_t rows, uint32_t k, const int32_t *__restrict__ tab,
+                                                         TO *__restrict__ out)
+{
+    const uint32_t lane = threadIdx.x & 63, q = blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (q >= rows)
+        return;
+    int32_t acc[E] = {};
+    row_accumulate<E, TM>(m + (size_t)q * k, k, tab, lane, acc);
+    if (e)
+        row_accumulate<E, uint32_t>(e + (size_t)q * E, E, tab + (size_t)k * E, lane, acc);
+    row_reduce<E>(acc);
+#pragma unroll
+    for (int j = 0; j < E; ++j)
+        if (lane == (uint32_t)j)
+            out[(size_t)q * E + j] = (TO)acc[j];
+}
+
 // ---------------------------------------------------------------- CIRC16 (pycirc16.hpp)
 
 // One CIRC16 block (pycirc16.hpp:45-64, 423-441): message row r (r < outer k) holds the inner
@@ -3664,9 +3721,12 @@ __global__ __launch_bounds__(64) void circ16_synd_kernel(const Rsi16Dev T, const
 // rows (message at rso32 + q k, parity at rsio32 + q E): where its syndromes are not all zero
 // and it holds 1 .. E zero symbols, the known-position repair at those positions; where every
 // repaired value is 0 mod 0x10000 the values are written back and the syndromes recomputed.
+// ER: ecc_len where its syndrome rows `tab` exist, else 0.
+template <int ER>
 __global__ __launch_bounds__(64) void circ16_outer_zeros_kernel(const Rsi16Dev T, uint32_t *__restrict__ rso32,
                                                                  uint32_t *__restrict__ rsio32, uint32_t rows,
-                                                                 uint32_t *__restrict__ syn)
+                                                                 uint32_t *__restrict__ syn,
+                                                                 const int32_t *__restrict__ tab)
 {
     extern __shared__ uint32_t s_mem[];
     const uint32_t q = blockIdx.x, lane = threadIdx.x, E = T.E, k = T.k;
@@ -3716,9 +3776,21 @@ __global__ __launch_bounds__(64) void circ16_outer_zeros_kernel(const Rsi16Dev T
             e[p - k] = err[r];
     }
     __syncthreads();  // the stores above are read back by other lanes below
-    pntt_codeword<uint32_t, uint32_t>(T, m, e, chunk, ev, G);  // synd_block (pyrsi16.hpp:186-189)
-    for (uint32_t j = lane; j < E; j += 64)
-        sy[j] = ev[j];
+    // synd_block (pyrsi16.hpp:186-189)
+    if constexpr (ER > 0) {
+        int32_t acc[ER] = {};
+        row_accumulate<ER, uint32_t>(m, k, tab, lane, acc);
+        row_accumulate<ER, uint32_t>(e, ER, tab + (size_t)k * ER, lane, acc);
+        row_reduce<ER>(acc);
+#pragma unroll
+        for (int j = 0; j < ER; ++j)
+            if (lane == (uint32_t)j)
+                sy[j] = (uint32_t)acc[j];
+    } else {
+        pntt_codeword<uint32_t, uint32_t>(T, m, e, chunk, ev, G);
+        for (uint32_t j = lane; j < E; j += 64)
+            sy[j] = ev[j];
+    }
 }
 
 // repair_inner_zeros (pycirc16.hpp:246-289) and find_error_locations (:291-295), one wave per
@@ -3795,6 +3867,111 @@ __global__ __launch_bounds__(64) void circ16_outer_known_kernel(const Rsi16Dev T
     });
 }
 
+// The same repair for outer ecc_len <= 256 as a linear map of the column: the error rows are those of
+// the whole interleave block, so e_i = sum_m c_m W[m][i] with one matrix per block. For the unit
+// column at m (S_j = X_m^j) the evaluator S(z) Lambda(z) mod z^E at y = 1 / x_i, where Lambda
+// vanishes, is ((X_m y)^E Lambda(1 / X_m)) / (X_m y - 1), or -y Lambda'(y) where X_m = x_i, and Forney
+// gives
+//   W[m][i] = A_m B_i / (X_m y_i - 1), W[pos_i][i] = -1, with A_m = X_m^E Lambda(1 / X_m),
+//   B_i = x_i y_i^E / Lambda'(y_i), Lambda'(y_i) = -x_i prod_(j != i) (1 - x_j y_i).
+// All of it is exact, so a column gets the values of the transforms (232 us for 8,192 columns of
+// outer RSi16(512,256) at 21 rows with those, one wave a column; 12 + 33 us here).
+constexpr uint32_t KNOWN_E = 256;
+
+// W of interleave block blockIdx.y, rows blockIdx.x * 256 + thread: balanced words at
+// (kk n + m) E + i, i < cnt[kk].
+__global__ __launch_bounds__(256) void circ16_known_map_kernel(const Rsi16Dev T, const uint32_t *__restrict__ pos,
+                                                               const uint32_t *__restrict__ cnt,
+                                                               int32_t *__restrict__ W)
+{
+    __shared__ uint32_t s_x[KNOWN_E], s_y[KNOWN_E], s_b[KNOWN_E];
+    const uint32_t kk = blockIdx.y, E = T.E, r = cnt[kk], t = threadIdx.x;
+    if (r == 0 || r > E || E > KNOWN_E)
+        return;
+    if (t < r) {
+        const uint32_t ri = rbo_bits(pos[(size_t)kk * E + t], T.nbits);
+        s_x[t] = T.roots_ntt[ri];
+        s_y[t] = T.roots_ntt[(T.N - ri) & (T.N - 1)];
+    }
+    __syncthreads();
+    if (t < r) {
+        uint32_t d = F::sub(0, s_x[t]);
+        for (uint32_t j = 0; j < r; ++j)
+            d = j == t ? d : F::mul(d, F::sub(1, F::mul(s_x[j], s_y[t])));
+        s_b[t] = F::mul(F::mul(s_x[t], s_pow(s_y[t], E)), T.inv_tab[d]);
+    }
+    __syncthreads();
+    const uint32_t m = blockIdx.x * 256 + t;
+    if (m >= T.n)
+        return;
+    const uint32_t ri = rbo_bits(m, T.nbits);
+    const uint32_t X = T.roots_ntt[ri], Xi = T.roots_ntt[(T.N - ri) & (T.N - 1)];
+    uint32_t a = s_pow(X, E);
+    for (uint32_t j = 0; j < r; ++j)
+        a = F::mul(a, F::sub(1, F::mul(s_x[j], Xi)));
+    int32_t *w = W + ((size_t)kk * T.n + m) * E;
+    for (uint32_t i = 0; i < r; ++i) {
+        const uint32_t den = F::sub(F::mul(X, s_y[i]), 1);
+        const uint32_t v = den ? F::mul(F::mul(a, s_b[i]), T.inv_tab[den]) : P16 - 1;
+        w[i] = v > 32768 ? (int32_t)v - (int32_t)P16 : (int32_t)v;
+    }
+}
+
+// The corrections of 64 columns (of one interleave block: col0 counts within block blockIdx.y) per
+// workgroup of 16 waves: each wave sums every 16th symbol, KNOWN_I error rows at a time.
+constexpr int KNOWN_I = 8;
+__global__ __launch_bounds__(1024) void circ16_known_apply_kernel(const Rsi16Dev T, uint16_t *__restrict__ msg,
+                                                                  uint32_t *__restrict__ rso32, uint32_t il,
+                                                                  uint32_t ik, const uint32_t *__restrict__ pos,
+                                                                  const uint32_t *__restrict__ cnt,
+                                                                  const int32_t *__restrict__ W)
+{
+    __shared__ int32_t s_part[16][KNOWN_I][64];
+    __shared__ uint32_t s_err[KNOWN_E][64];
+    const uint32_t kk = blockIdx.y, E = T.E, k = T.k, n = T.n, r = cnt[kk];
+    if (r == 0 || r > E || E > KNOWN_E)
+        return;
+    const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t in = blockIdx.x * 64 + lane;
+    const bool valid = in < ik;
+    const size_t col = (size_t)kk * ik + (valid ? in : 0);
+    for (uint32_t i0 = 0; i0 < r; i0 += KNOWN_I) {
+        int32_t acc[KNOWN_I] = {};
+        for (uint32_t m = wave; m < n; m += 16) {
+            int32_t c = m < k ? (int32_t)msg[(size_t)m * il + col] : (int32_t)rso32[(size_t)(m - k) * il + col];
+            c = c > 32768 ? c - (int32_t)P16 : c;
+            const int32_t *w = W + ((size_t)kk * n + m) * E + i0;
+#pragma unroll
+            for (int u = 0; u < KNOWN_I; ++u)  // past r: words of the row that no error uses
+                acc[u] += fold16(c * (i0 + u < E ? w[u] : 0));
+        }
+#pragma unroll
+        for (int u = 0; u < KNOWN_I; ++u)
+            s_part[wave][u][lane] = fold2(acc[u]);
+        __syncthreads();
+        if (wave < KNOWN_I && i0 + wave < r) {
+            int32_t v = 0;
+            for (int p = 0; p < 16; ++p)
+                v += s_part[p][wave][lane];
+            v = fold2(v);
+            s_err[i0 + wave][lane] = (uint32_t)(v + ((v >> 31) & (int32_t)P16));
+        }
+        __syncthreads();
+    }
+    if (!valid)
+        return;
+    for (uint32_t i = wave; i < r; i += 16) {
+        const uint32_t p = pos[(size_t)kk * E + i], v = s_err[i][lane];
+        if (p < k) {
+            uint16_t *at = msg + (size_t)p * il + col;
+            *at = (uint16_t)(S::add((uint32_t)*at, v) & 0xffffu);
+        } else {
+            uint32_t *at = rso32 + (size_t)(p - k) * il + col;
+            *at = S::add(*at, v);
+        }
+    }
+}
+
 // dump_ecc (pycirc16.hpp:323-327) of `blocks` blocks: out block b = [outer parity (u32 state)
 // & 0xFFFF | inner parity of the message rows | inner parity of the outer parity rows]
 __global__ __launch_bounds__(256) void circ16_assemble_kernel(const uint32_t *__restrict__ rso32,
@@ -3804,19 +3981,17 @@ __global__ __launch_bounds__(256) void circ16_assemble_kernel(const uint32_t *__
                                                                uint16_t *__restrict__ out)
 {
     const uint32_t el = rso_len + rsi_len + rsio_len;
-    const size_t total = (size_t)el * blocks;
-    for (size_t t = (size_t)blockIdx.x * 256 + threadIdx.x; t < total; t += (size_t)gridDim.x * 256) {
-        const size_t b = t / el;
-        const uint32_t x = (uint32_t)(t - b * el);
-        uint16_t v;
-        if (x < rso_len)
-            v = (uint16_t)(rso32[b * rso_len + x] & 0xffffu);
-        else if (x < rso_len + rsi_len)
-            v = rsi16[b * rsi_len + (x - rso_len)];
-        else
-            v = rsio16[b * rsio_len + (x - rso_len - rsi_len)];
-        out[t] = v;
-    }
+    for (size_t b = blockIdx.y; b < blocks; b += gridDim.y)
+        for (uint32_t x = blockIdx.x * 256 + threadIdx.x; x < el; x += gridDim.x * 256) {
+            uint16_t v;
+            if (x < rso_len)
+                v = (uint16_t)(rso32[b * rso_len + x] & 0xffffu);
+            else if (x < rso_len + rsi_len)
+                v = rsi16[b * rsi_len + (x - rso_len)];
+            else
+                v = rsio16[b * rsio_len + (x - rso_len - rsi_len)];
+            out[b * el + x] = v;
+        }
 }
 
 // ---------------------------------------------------------------- mixed-size plans
@@ -3966,6 +4141,7 @@ struct ffrs_rsi16 {
         void *d = nullptr;
         RootTab dev{};
     } roots;                         // the locator's values at the n positions
+    int32_t *d_rows_enc = nullptr, *d_rows_syn = nullptr;  // balanced rows of the same maps (ecc_len 2 to 8)
     bool mix_minus_one = false;      // a mix constant is 65536: the SIMD words are not the linear map
     int encode_mode = 0;             // 0 automatic, 1 butterflies, 2 MFMA wherever it applies
     uint32_t *d_syn = nullptr;       // syndromes of the last repair launch
@@ -4331,8 +4507,53 @@ int build_contract(ContractTab *tab, const std::vector<uint32_t> &mat, uint32_t 
 
 // The encode's matrix: G[m] = the parity of the unit message at m, i.e. the GS butterfly of
 // mix_i X_m^i with X_m = w^rbo(m) (the message residue of rsi16v_impl.hpp:93-97 is
-// sum_m v_m X_m^i, then :108-119). Shapes with ecc_len below 8, above 256, or message_len
-// above 16384 keep the butterfly kernels.
+// sum_m v_m X_m^i, then :108-119); row m holds E entries.
+void encode_matrix(const ffrs_rsi16 *rs, const std::vector<uint32_t> &mix, const std::vector<uint32_t> &roots_i_ecc,
+                   const std::vector<uint32_t> &roots_ntt, std::vector<uint32_t> &mat)
+{
+    for (uint32_t m = 0; m < rs->k; ++m) {
+        const uint32_t x = roots_ntt[rbo_bits(m, rs->nbits)];
+        uint32_t *row = &mat[(size_t)m * rs->E];
+        uint32_t pw = 1;
+        for (uint32_t i = 0; i < rs->E; ++i) {
+            row[i] = S::mul(mix[i], pw);
+            pw = S::mul(pw, x);
+        }
+        gs_host(roots_i_ecc, row, rs->E);
+    }
+}
+
+// The same matrix and the syndromes' w^(j rbo(m)) (NTT::pntt, ntt.hpp:133-152) as balanced words, for
+// rsi16_rows_kernel.
+int build_rows(ffrs_rsi16 *rs, const std::vector<uint32_t> &mix, const std::vector<uint32_t> &roots_i_ecc,
+               const std::vector<uint32_t> &roots_ntt)
+{
+    const uint32_t E = rs->E, n = rs->n, k = rs->k;
+    if (E < 2 || E > 8 || k > 16384)
+        return FFRS_OK;
+    std::vector<uint32_t> enc((size_t)k * E), syn((size_t)n * E);
+    encode_matrix(rs, mix, roots_i_ecc, roots_ntt, enc);
+    for (uint32_t m = 0; m < n; ++m)
+        for (uint32_t j = 0, pw = 1; j < E; ++j) {
+            syn[(size_t)m * E + j] = pw;
+            pw = S::mul(pw, roots_ntt[rbo_bits(m, rs->nbits)]);
+        }
+    for (auto *v : {&enc, &syn}) {
+        for (uint32_t &x : *v)
+            x = x > 32768 ? x - P16 : x;
+        int32_t *d = nullptr;
+        hipError_t e = hipMalloc(&d, v->size() * 4);
+        if (e == hipSuccess) {
+            (v == &enc ? rs->d_rows_enc : rs->d_rows_syn) = d;
+            e = hipMemcpy(d, v->data(), v->size() * 4, hipMemcpyHostToDevice);
+        }
+        if (e != hipSuccess)
+            return fail(FFRS_ERR_DEVICE, "row tables: %s", hipGetErrorString(e));
+    }
+    return FFRS_OK;
+}
+
+// Shapes with ecc_len below 8, above 256, or message_len above 16384 have no contraction tables.
 int build_mfma_encode(ffrs_rsi16 *rs, const std::vector<uint32_t> &mix, const std::vector<uint32_t> &roots_i_ecc,
                       const std::vector<uint32_t> &roots_ntt)
 {
@@ -4341,16 +4562,7 @@ int build_mfma_encode(ffrs_rsi16 *rs, const std::vector<uint32_t> &mix, const st
         return FFRS_OK;
     const uint32_t nq = (k + 63) / 64;
     std::vector<uint32_t> mat((size_t)nq * 64 * E, 0);
-    for (uint32_t m = 0; m < k; ++m) {
-        const uint32_t x = roots_ntt[rbo_bits(m, rs->nbits)];
-        uint32_t *row = &mat[(size_t)m * E];
-        uint32_t pw = 1;
-        for (uint32_t i = 0; i < E; ++i) {
-            row[i] = S::mul(mix[i], pw);
-            pw = S::mul(pw, x);
-        }
-        gs_host(roots_i_ecc, row, E);
-    }
+    encode_matrix(rs, mix, roots_i_ecc, roots_ntt, mat);
     return build_contract(&rs->enc, mat, E, nq, nq);
 }
 
@@ -4567,6 +4779,10 @@ int ffrs_rsi16_create(ffrs_ctx *ctx, size_t block_len, size_t ecc_len, uint32_t 
         ffrs_rsi16_destroy(rs);
         return r;
     }
+    if (int r = build_rows(rs, mix, roots_i_ecc, roots_ntt)) {
+        ffrs_rsi16_destroy(rs);
+        return r;
+    }
     *out = rs;
     return FFRS_OK;
 }
@@ -4602,7 +4818,7 @@ void ffrs_rsi16_destroy(ffrs_rsi16 *rs)
         (void)hipFree(rs->d_tables);
     if (rs->d_work)
         (void)hipFree(rs->d_work);
-    for (void *d : {rs->enc.d, rs->synd.d, rs->roots.d})
+    for (void *d : {rs->enc.d, rs->synd.d, rs->roots.d, (void *)rs->d_rows_enc, (void *)rs->d_rows_syn})
         if (d)
             (void)hipFree(d);
     if (rs->d_syn)
@@ -5438,6 +5654,19 @@ int circ_reserve(ffrs_circ16 *c, size_t bytes)
 
 size_t al256(size_t x) { return (x + 255) & ~(size_t)255; }
 
+// rsi16_rows_kernel on `rows` codewords: syndromes where e is given, else the parity.
+template <class TM, class TO>
+int launch_rows(ffrs_rsi16 *rs, const TM *m, const uint32_t *e, size_t rows, TO *out)
+{
+    auto *k = rs->E == 2   ? rsi16_rows_kernel<2, TM, TO>
+              : rs->E == 4 ? rsi16_rows_kernel<4, TM, TO>
+                           : rsi16_rows_kernel<8, TM, TO>;
+    hipLaunchKernelGGL(k, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, rs->ctx->stream, m, e, (uint32_t)rows, rs->k,
+                       (const int32_t *)(e ? rs->d_rows_syn : rs->d_rows_enc), out);
+    FFRS_HIP(hipGetLastError());
+    return FFRS_OK;
+}
+
 // The generic lane-group encode of `count` codewords (interleave stride I), u16 or u32 symbols in
 // and out, in the SIMD or scalar words.
 template <class TI, class TO>
@@ -5445,6 +5674,8 @@ int circ_encode(ffrs_rsi16 *rs, const TI *d_in, size_t count, TO *d_out, bool ve
 {
     if (count == 0)
         return FFRS_OK;
+    if (I == 1 && rs->d_rows_enc && !(vec && rs->mix_minus_one))
+        return launch_rows<TI, TO>(rs, d_in, nullptr, count, d_out);
     const uint32_t g = rs->g_enc == 1 && rs->E <= 32 ? group_size(rs->E) : rs->g_enc, cpw = 64 / g;
     const size_t lds = (size_t)cpw * 2 * rs->E * 4;
     auto *kv = rsi16_encode_kernel<VectorOps, TI, TO>;
@@ -5458,12 +5689,22 @@ int circ_encode(ffrs_rsi16 *rs, const TI *d_in, size_t count, TO *d_out, bool ve
     return FFRS_OK;
 }
 
+// The inner parity of `rows` message rows.
+int circ_encode_rows(ffrs_circ16 *c, const uint16_t *d_msg, size_t rows, uint16_t *d_rsi)
+{
+    ffrs_rsi16 *rs = c->ri;
+    if (rs->d_rows_enc && rs->E <= 4 && !(c->W > 1 && rs->mix_minus_one))
+        return launch_rows<uint16_t, uint16_t>(rs, d_msg, nullptr, rows, d_rsi);
+    return launch_encode(rs, d_msg, rows, d_rsi, c->W > 1 ? 1 : 0);
+}
+
 // Repair workspace of one block: u16 message and ecc, u32 outer parity, u32 inner parity,
 // u32 syndromes, row flags, error rows per interleave block and their counts, group statuses.
 struct CircWs {
     uint16_t *msg, *ecc;
     uint32_t *rso32, *rsi32, *syn, *pos, *cnt;
     uint8_t *flag, *gst;
+    int32_t *map;  // outer ecc_len <= KNOWN_E: the known-position repair's matrix per interleave block
     uint32_t *work;
     size_t work_lanes;
 };
@@ -5490,6 +5731,7 @@ size_t circ_repair_layout(const ffrs_circ16 *c, CircWs *w, char *base)
     w->pos = (uint32_t *)take((size_t)c->I * c->oE * 4);
     w->cnt = (uint32_t *)take((size_t)c->I * 4);
     w->gst = (uint8_t *)take(ngr);
+    w->map = (int32_t *)take(c->oE <= KNOWN_E ? (size_t)c->I * c->on * c->oE * 4 : 0);
     w->work = (uint32_t *)take(lanes * wrows * 4);
     w->work_lanes = lanes;
     return o;
@@ -5502,27 +5744,38 @@ int circ_prepare(ffrs_circ16 *c, const CircWs &w)
     hipStream_t st = c->ri->ctx->stream;
     const uint32_t rows = c->on * c->I, mrows = c->ok * c->I, erows = c->oE * c->I, iE = c->iE;
     const size_t rsi_all = (size_t)rows * iE;
-    hipLaunchKernelGGL(circ16_expand_kernel, dim3(256), dim3(256), 0, st, (const uint16_t *)w.ecc, w.rso32,
+    hipLaunchKernelGGL(circ16_expand_kernel, dim3(2048), dim3(256), 0, st, (const uint16_t *)w.ecc, w.rso32,
                        (uint32_t)c->rso_len, w.rsi32, (uint32_t)rsi_all);
     FFRS_HIP(hipGetLastError());
-    const uint32_t g = group_size(iE), cpw = 64 / g;
-    const size_t lds = (size_t)cpw * 2 * iE * 4;
-    if (int r = allow_lds(circ16_synd_kernel<uint16_t>, lds))
-        return r;
-    if (int r = allow_lds(circ16_synd_kernel<uint32_t>, lds))
-        return r;
-    hipLaunchKernelGGL(circ16_synd_kernel<uint16_t>, dim3((mrows + cpw - 1) / cpw), dim3(64), lds, st, c->ri->dev,
-                       (const uint16_t *)w.msg, (const uint32_t *)w.rsi32, mrows, w.syn, g);
-    FFRS_HIP(hipGetLastError());
-    hipLaunchKernelGGL(circ16_synd_kernel<uint32_t>, dim3((erows + cpw - 1) / cpw), dim3(64), lds, st, c->ri->dev,
-                       (const uint32_t *)w.rso32, (const uint32_t *)(w.rsi32 + (size_t)mrows * iE), erows,
-                       w.syn + (size_t)mrows * iE, g);
-    FFRS_HIP(hipGetLastError());
+    uint32_t *esyn = w.syn + (size_t)mrows * iE, *ersi = w.rsi32 + (size_t)mrows * iE;
+    if (c->ri->d_rows_syn) {
+        if (int r = launch_rows<uint16_t, uint32_t>(c->ri, w.msg, w.rsi32, mrows, w.syn))
+            return r;
+        if (int r = launch_rows<uint32_t, uint32_t>(c->ri, w.rso32, ersi, erows, esyn))
+            return r;
+    } else {
+        const uint32_t g = group_size(iE), cpw = 64 / g;
+        const size_t lds = (size_t)cpw * 2 * iE * 4;
+        if (int r = allow_lds(circ16_synd_kernel<uint16_t>, lds))
+            return r;
+        if (int r = allow_lds(circ16_synd_kernel<uint32_t>, lds))
+            return r;
+        hipLaunchKernelGGL(circ16_synd_kernel<uint16_t>, dim3((mrows + cpw - 1) / cpw), dim3(64), lds, st, c->ri->dev,
+                           (const uint16_t *)w.msg, (const uint32_t *)w.rsi32, mrows, w.syn, g);
+        FFRS_HIP(hipGetLastError());
+        hipLaunchKernelGGL(circ16_synd_kernel<uint32_t>, dim3((erows + cpw - 1) / cpw), dim3(64), lds, st, c->ri->dev,
+                           (const uint32_t *)w.rso32, (const uint32_t *)ersi, erows, esyn, g);
+        FFRS_HIP(hipGetLastError());
+    }
     const size_t lz = (size_t)9 * iE * 4;
-    if (int r = allow_lds(circ16_outer_zeros_kernel, lz))
+    auto *zk = !c->ri->d_rows_syn ? circ16_outer_zeros_kernel<0>
+               : iE == 2          ? circ16_outer_zeros_kernel<2>
+               : iE == 4          ? circ16_outer_zeros_kernel<4>
+                                  : circ16_outer_zeros_kernel<8>;
+    if (int r = allow_lds(zk, lz))
         return r;
-    hipLaunchKernelGGL(circ16_outer_zeros_kernel, dim3(erows), dim3(64), lz, st, c->ri->dev, w.rso32,
-                       w.rsi32 + (size_t)mrows * iE, erows, w.syn + (size_t)mrows * iE);
+    hipLaunchKernelGGL(zk, dim3(erows), dim3(64), lz, st, c->ri->dev, w.rso32, ersi, erows, esyn,
+                       (const int32_t *)c->ri->d_rows_syn);
     FFRS_HIP(hipGetLastError());
     if (int r = allow_lds(circ16_inner_zeros_kernel, (size_t)iE * 4))
         return r;
@@ -5624,11 +5877,11 @@ int ffrs_circ16_encode(ffrs_circ16 *c, const uint16_t *msg, size_t blocks, uint1
     // parity of the message rows and of the outer parity rows
     if (int r = circ_encode<uint16_t, uint32_t>(c->ro, d_msg, blocks * c->rI, d_rso, vec, c->rI))
         return r;
-    if (int r = launch_encode(c->ri, d_msg, blocks * c->ok * c->I, d_rsi, vec ? 1 : 0))
+    if (int r = circ_encode_rows(c, d_msg, blocks * c->ok * c->I, d_rsi))
         return r;
     if (int r = circ_encode<uint32_t, uint16_t>(c->ri, d_rso, blocks * c->oE * c->I, d_rsio, vec, 1))
         return r;
-    hipLaunchKernelGGL(circ16_assemble_kernel, dim3(1024), dim3(256), 0, st, (const uint32_t *)d_rso,
+    hipLaunchKernelGGL(circ16_assemble_kernel, dim3(1024, (unsigned)std::min<size_t>(blocks, 16)), dim3(256), 0, st, (const uint32_t *)d_rso,
                        (const uint16_t *)d_rsi, (const uint16_t *)d_rsio, (uint32_t)c->rso_len, (uint32_t)c->rsi_len,
                        (uint32_t)c->rsio_len, (uint32_t)blocks, d_out);
     FFRS_HIP(hipGetLastError());
@@ -5705,12 +5958,22 @@ int ffrs_circ16_repair(ffrs_circ16 *c, uint16_t *msg, uint16_t *ecc, int *raised
     if (std::any_of(cnt.begin(), cnt.end(), [](uint32_t v) { return v != 0; })) {
         FFRS_HIP(hipMemcpyAsync(w.pos, pos.data(), pos.size() * 4, hipMemcpyHostToDevice, st));
         FFRS_HIP(hipMemcpyAsync(w.cnt, cnt.data(), cnt.size() * 4, hipMemcpyHostToDevice, st));
-        const size_t lds = (size_t)7 * c->oE * 4;
-        if (int r = allow_lds(circ16_outer_known_kernel, lds))
-            return r;
-        hipLaunchKernelGGL(circ16_outer_known_kernel, dim3(c->rI), dim3(64), lds, st, c->ro->dev, w.msg, w.rso32,
-                           c->rI, c->ik, (const uint32_t *)w.pos, (const uint32_t *)w.cnt);
-        FFRS_HIP(hipGetLastError());
+        if (c->oE <= KNOWN_E) {
+            hipLaunchKernelGGL(circ16_known_map_kernel, dim3((c->on + 255) / 256, c->I), dim3(256), 0, st, c->ro->dev,
+                               (const uint32_t *)w.pos, (const uint32_t *)w.cnt, w.map);
+            FFRS_HIP(hipGetLastError());
+            hipLaunchKernelGGL(circ16_known_apply_kernel, dim3((c->ik + 63) / 64, c->I), dim3(1024), 0, st, c->ro->dev,
+                               w.msg, w.rso32, c->rI, c->ik, (const uint32_t *)w.pos, (const uint32_t *)w.cnt,
+                               (const int32_t *)w.map);
+            FFRS_HIP(hipGetLastError());
+        } else {
+            const size_t lds = (size_t)7 * c->oE * 4;
+            if (int r = allow_lds(circ16_outer_known_kernel, lds))
+                return r;
+            hipLaunchKernelGGL(circ16_outer_known_kernel, dim3(c->rI), dim3(64), lds, st, c->ro->dev, w.msg, w.rso32,
+                               c->rI, c->ik, (const uint32_t *)w.pos, (const uint32_t *)w.cnt);
+            FFRS_HIP(hipGetLastError());
+        }
     }
     // without positions: the reference's SIMD groups of W columns from the block's first column
     // (pyrsi16.hpp:391-456), in block order; a group that raises stops the repair there
@@ -5763,11 +6026,11 @@ int ffrs_circ16_repair(ffrs_circ16 *c, uint16_t *msg, uint16_t *ecc, int *raised
     // recompute_inner_ecc (pycirc16.hpp:317-321) and dump_ecc
     const bool vec = W > 1;
     uint16_t *d_rsi = w.ecc + c->rso_len, *d_rsio = d_rsi + c->rsi_len;
-    if (int r = launch_encode(c->ri, w.msg, (size_t)c->ok * c->I, d_rsi, vec ? 1 : 0))
+    if (int r = circ_encode_rows(c, w.msg, (size_t)c->ok * c->I, d_rsi))
         return r;
     if (int r = circ_encode<uint32_t, uint16_t>(c->ri, w.rso32, (size_t)c->oE * c->I, d_rsio, vec, 1))
         return r;
-    hipLaunchKernelGGL(circ16_assemble_kernel, dim3(64), dim3(256), 0, st, (const uint32_t *)w.rso32,
+    hipLaunchKernelGGL(circ16_assemble_kernel, dim3(1024), dim3(256), 0, st, (const uint32_t *)w.rso32,
                        (const uint16_t *)d_rsi, (const uint16_t *)d_rsio, (uint32_t)c->rso_len, 0u, 0u, 1u, w.ecc);
     FFRS_HIP(hipGetLastError());
     FFRS_HIP(hipMemcpyAsync(msg, w.msg, c->msg_len * 2, hipMemcpyDeviceToHost, st));
