@@ -99,9 +99,10 @@ int ffrs_ctx_kernel_times(ffrs_ctx *ctx, float *ms, int cap, int *count);
 int ffrs_rs256_create(ffrs_ctx *ctx, unsigned ecc_len, unsigned primitive, unsigned polynomial,
                       ffrs_rs256 **out);
 void ffrs_rs256_destroy(ffrs_rs256 *rs);
-/* Repair kernels (no counterpart in the reference; results do not depend on it): 0 and 1
- * use the syndrome / Berlekamp-Massey / Chien pipeline where ecc_len <= 32 (default), 2
- * one kernel with one codeword per lane; ecc_len > 32 always uses the latter. */
+/* Repair kernels (no counterpart in the reference; results do not depend on it): 0 automatic (for
+ * ecc_len <= 32 one codeword per wave in small launches, else the syndrome / Berlekamp-Massey /
+ * Chien pipeline; above 32 one codeword per wave), 1 the pipeline for ecc_len <= 32 at every size,
+ * 2 one kernel with one codeword per lane. */
 int ffrs_rs256_set_repair_mode(ffrs_rs256 *rs, int mode);
 
 /* generator[0..ecc_len], highest degree first (libffrs/reed_solomon.hpp:55-88) */

@@ -901,7 +901,8 @@ __global__ __launch_bounds__(WG) void rs256_repair_kernel(uint8_t *__restrict__ 
 }
 
 // ======================================================================
-// Wave-cooperative repair, one codeword per wave, for ecc_len 33..252 (the same steps and
+// Wave-cooperative repair, one codeword per wave, for ecc_len 33..252 and small launches of
+// shorter codes (the same steps and
 // results as repair_one, reed_solomon.hpp:559-595, spread over the 64 lanes instead of run by
 // one):
 //   syndromes  S_i = sum_j c_j alpha^(i (n-1-j)), syndrome i by lane i % 64 (direct sums over
@@ -950,18 +951,21 @@ __device__ inline uint8_t repair_wave(uint8_t *pm, uint8_t *pe, uint32_t k, uint
         w.lc[j] = (uint16_t)gf.log2[c];
     }
     __builtin_amdgcn_wave_barrier();
-    // ---- syndromes: lane l sums S_(l + 64 q) over the positions
-    uint32_t sy[NS], e[NS], st[NS];
+    // ---- syndromes: lane l sums S_(l + 64 q) over the positions; for E <= 32 the lanes are SG
+    // groups of 64 / SG, each over every SG-th run of eight positions, XORed together afterwards
+    const uint32_t SG = NS > 1 || E > 32 ? 1 : E > 16 ? 2 : E > 8 ? 4 : 8, EP = 64 / SG, seg = lane / EP;
+    uint32_t sy[NS], e[NS], st[NS], skip[NS];
 #pragma unroll
     for (int q = 0; q < NS; ++q) {
-        const uint32_t i = lane + 64 * q;
+        const uint32_t i = lane % EP + 64 * q;
         sy[q] = 0;
         st[q] = i % 255;
-        e[q] = (i * (n - 1)) % 255;  // exponent of alpha^i at position j = 0
+        e[q] = (i * ((n - 1 + 255 - 8 * seg) % 255)) % 255;  // exponent of alpha^i at position 8 seg
+        skip[q] = (i * 8 * (SG - 1)) % 255;
     }
     // eight positions per pass: their logs in one 16-byte read (positions past n hold ZLOG
     // logs of zero bytes, which add nothing), then the eight lookups of each syndrome together
-    for (uint32_t j0 = 0; j0 < n; j0 += 8) {
+    for (uint32_t j0 = 8 * seg; j0 < n; j0 += 8 * SG) {
         const uint4 l8 = *reinterpret_cast<const uint4 *>(&w.lc[j0]);
         const uint32_t lw[4] = {l8.x, l8.y, l8.z, l8.w};
 #pragma unroll
@@ -972,11 +976,14 @@ __device__ inline uint8_t repair_wave(uint8_t *pm, uint8_t *pe, uint32_t k, uint
                 t[u] = gf.exp2[((lw[u >> 1] >> (16 * (u & 1))) & 0xffffu) + e[q]];
                 e[q] = e[q] >= st[q] ? e[q] - st[q] : e[q] + 255 - st[q];
             }
+            e[q] = e[q] >= skip[q] ? e[q] - skip[q] : e[q] + 255 - skip[q];
 #pragma unroll
             for (int u = 0; u < 8; ++u)
                 sy[q] ^= t[u];
         }
     }
+    for (uint32_t s = EP; s < 64; s <<= 1)
+        sy[0] ^= (uint32_t)__shfl_xor((int)sy[0], (int)s);
     uint32_t any = 0;
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
@@ -1206,12 +1213,10 @@ __global__ __launch_bounds__(256) void rs256_synds_kernel(const uint8_t *__restr
 //   rs256_synd_kernel    lane per codeword: remainder + XOR parity; zero -> status 1;
 //                        else syndromes from nibble tables ST[j][h][v] (E bytes each:
 //                        (v << 4h) alpha^(i (E-1-j)), i < E) and status PENDING
-//   rs256_bm_kernel      lane per codeword: Berlekamp-Massey; L > E/2 -> status 0; else
-//                        a record {L, Lambda_0..L, Omega_0..L-1} (Omega = S Lambda mod x^E
-//                        has degree < L once the LFSR of length L generates all E syndromes)
-//                        (ecc 2, 4, 8, 16, 32: the Chien kernel runs this BM itself per tile
-//                        and keeps the records in registers)
-//   rs256_chien16_kernel Chien search, eight lanes per codeword over nibble tables, then
+//   rs256_chien16_kernel lane per codeword: Berlekamp-Massey; L > E/2 -> status 0; else a record
+//                        {L, Lambda_0..L, Omega_0..L-1} in registers (Omega = S Lambda mod x^E has
+//                        degree < L once the LFSR of length L generates all E syndromes); then
+//                        the Chien search, eight lanes per codeword over nibble tables, and
 //                        Forney at the roots.
 // ======================================================================
 
@@ -1223,7 +1228,6 @@ constexpr uint32_t CHIEN_TABLE_BYTES = CHIEN_LMAX * 2 * 16 * 256;
 // bytes 20..36 Lambda_0..16, zero-filled, 48 bytes.
 __host__ __device__ inline uint32_t rec_lam_off() { return 20; }
 __host__ __device__ inline uint32_t rec_om_off(uint32_t) { return 4; }
-__host__ __device__ inline uint32_t rec_stride(uint32_t) { return 48; }
 
 // LM: message loads, as for rs256_encode_kernel.
 template <int EW, int S, int WG, int LM = LOAD_LANE>
@@ -1321,107 +1325,6 @@ __global__ __launch_bounds__(WG) void rs256_synd_kernel(const uint8_t *__restric
     }
 }
 
-// Per-lane LDS row of the BM kernel: S[E], logS[E] (u16), Lambda[E], B[E].
-__host__ __device__ inline uint32_t bm_row_stride(uint32_t E)
-{
-    uint32_t dw = (E + 2 * E + E + E + 3) / 4;
-    return ((dw & 1) ? dw : dw + 1) * 4;
-}
-
-template <int WG>
-__global__ __launch_bounds__(WG) void rs256_bm_kernel(uint32_t count, uint32_t E, uint32_t sstride_words,
-                                                       uint8_t *__restrict__ status, const uint32_t *__restrict__ synd,
-                                                       uint8_t *__restrict__ rec, Rs256Tables tab)
-{
-    extern __shared__ uint32_t s_mem[];
-    uint8_t *s_exp2 = reinterpret_cast<uint8_t *>(s_mem);
-    uint16_t *s_log2 = reinterpret_cast<uint16_t *>(s_exp2 + EXP2_LEN);
-    uint8_t *s_rows = reinterpret_cast<uint8_t *>(s_log2 + 256);
-    for (uint32_t i = threadIdx.x; i < (uint32_t)EXP2_LEN; i += blockDim.x)
-        s_exp2[i] = tab.exp2[i];
-    for (uint32_t i = threadIdx.x; i < 256u; i += blockDim.x)
-        s_log2[i] = tab.log2[i];
-    __syncthreads();
-    GfLds gf{s_exp2, s_log2};
-    uint8_t *row = s_rows + threadIdx.x * bm_row_stride(E);
-    uint8_t *Sy = row;
-    uint16_t *lS = reinterpret_cast<uint16_t *>(row + ((E + 1) & ~1u));
-    uint8_t *lam = row + ((E + 1) & ~1u) + 2 * E;
-    uint8_t *Bx = lam + E;
-    const uint32_t RS = rec_stride(E), LO = rec_lam_off(), OO = rec_om_off(E);
-
-    for (uint32_t cw = blockIdx.x * blockDim.x + threadIdx.x; cw < count; cw += gridDim.x * blockDim.x) {
-        if (status[cw] != RS_PENDING)
-            continue;
-        const uint32_t *sw = synd + (size_t)cw * sstride_words;
-        for (uint32_t w = 0; w < (E + 3) / 4; ++w) {
-            uint32_t v = sw[w];
-            for (uint32_t b = 0; b < 4 && w * 4 + b < E; ++b) {
-                uint32_t sb = (v >> (8 * b)) & 0xffu;
-                Sy[w * 4 + b] = (uint8_t)sb;
-                lS[w * 4 + b] = gf.log2[sb];
-            }
-        }
-        for (uint32_t i = 0; i < E; ++i) {
-            lam[i] = 0;
-            Bx[i] = 0;
-        }
-        lam[0] = 1;
-        Bx[0] = 1;
-        // reed_solomon.hpp:655-702, natural order; lenL / lenB bound the non-zero terms
-        uint32_t L = 0, m = 1, b = 1, lenL = 1, lenB = 1;
-        for (uint32_t nn = 0; nn < E; ++nn) {
-            uint32_t d = Sy[nn];
-            uint32_t top = L < lenL - 1 ? L : lenL - 1;
-            for (uint32_t i = 1; i <= top; ++i)
-                d ^= gf.exp2[gf.log2[lam[i]] + lS[nn - i]];
-            if (d == 0) {
-                m += 1;
-                continue;
-            }
-            uint32_t lc = gf.log2[gf.div(d, b)];
-            bool grow = 2 * L <= nn;
-            uint32_t hiB = m + lenB < E ? m + lenB : E;  // x^m B truncated to degrees < E
-            uint32_t hi = grow ? (hiB > lenL ? hiB : lenL) : hiB;
-            for (uint32_t ii = hi; ii-- > 0;) {
-                uint32_t old = lam[ii];
-                uint32_t sb = (ii >= m && ii < hiB) ? (uint32_t)Bx[ii - m] : 0u;
-                lam[ii] = (uint8_t)(old ^ gf.mul_log(lc, sb));
-                if (grow)
-                    Bx[ii] = (uint8_t)old;
-            }
-            if (grow) {
-                lenB = lenL;
-                L = nn + 1 - L;
-                b = d;
-                m = 1;
-            } else {
-                m += 1;
-            }
-            if (hiB > lenL)
-                lenL = hiB;
-        }
-        if (L > E / 2) {
-            status[cw] = 0;
-            continue;
-        }
-        uint8_t *r = rec + (size_t)cw * RS;
-        for (uint32_t i = 0; i < RS; ++i)
-            r[i] = 0;
-        r[0] = (uint8_t)L;
-        for (uint32_t i = 0; i <= E / 2; ++i)
-            r[LO + i] = i <= L ? lam[i] : 0;
-        // Omega_k = sum_{i <= k} Lambda_i S_{k-i}, k < L (reed_solomon.hpp:708-728)
-        for (uint32_t kk = 0; kk < E / 2; ++kk) {
-            uint32_t v = 0;
-            if (kk < L)
-                for (uint32_t i = 0; i <= kk; ++i)
-                    v ^= gf.exp2[gf.log2[lam[i]] + lS[kk - i]];
-            r[OO + kk] = (uint8_t)v;
-        }
-    }
-}
-
 // Log / exp tables of the register BM: EXP2 (1,024 bytes, zero above 509) and LOG2 (u16,
 // log 0 = ZLOG = 511), so that a product of logs is one read at the sum.
 struct LogExp1K {
@@ -1442,8 +1345,12 @@ struct LogExp1K {
 // Returns false when L > E/2 (not repairable); otherwise the 48-byte record in words[]:
 // L in byte 0, Omega_0..Omega_(E/2-1) from byte rec_om_off, Lambda_0..Lambda_(E/2) from byte
 // rec_lam_off.
+// e is the ecc_len, at most E (the terms unrolled past e / 2 only meet codewords whose L exceeds
+// e / 2). After iteration n, L is (n + 2) / 2 unless discrepancies of 0 made it lag and then jump, by
+// one for each; the terms above one such jump (a fifth of the lookups) run only where a lane of the
+// wave has them.
 template <int E, class T>
-__device__ inline bool bm_fixed_one(const uint32_t *__restrict__ sw, const T &tb, uint32_t (&words)[12])
+__device__ inline bool bm_fixed_one(const uint32_t *__restrict__ sw, uint32_t e, const T &tb, uint32_t (&words)[12])
 {
     constexpr int EW = (E + 3) / 4;
     constexpr uint32_t ZL = T::Z;
@@ -1472,38 +1379,55 @@ __device__ inline bool bm_fixed_one(const uint32_t *__restrict__ sw, const T &tb
     uint32_t L = 0, lb = 0;
 #pragma unroll
     for (int n = 0; n < E; ++n) {
-        uint32_t d = (sv[n >> 2] >> (8 * (n & 3))) & 0xffu;
+        if ((uint32_t)n < e) {
+            uint32_t d = (sv[n >> 2] >> (8 * (n & 3))) & 0xffu;
+            const int dt = n < H ? n : H, db = (n + 1) / 2 + 1 < dt ? (n + 1) / 2 + 1 : dt;
 #pragma unroll
-        for (int i = 1; i <= (n < H ? n : H); ++i)
-            d ^= tb.exp_sum(llam[i] + lS[n - i]);
-        bool nz = d != 0;
-        bool grow = nz && (2 * L <= (uint32_t)n);
-        uint32_t ld = tb.log(d);
-        uint32_t lc = ld + 255 - lb;
-        lc = lc >= 255 ? lc - 255 : lc;
-        // d == 0: the zero log puts every product below at zero, so no per-term select is needed
-        lc = nz ? lc : ZL;
-        const int hi = n + 1 < H ? n + 1 : H;
-        uint32_t old_llam[E];
+            for (int i = 1; i <= db; ++i)
+                d ^= tb.exp_sum(llam[i] + lS[n - i]);
+            if (db < dt && __any(L > (uint32_t)db)) {
 #pragma unroll
-        for (int i = 0; i < E; ++i)
-            old_llam[i] = llam[i];
+                for (int i = db + 1; i <= dt; ++i)
+                    d ^= tb.exp_sum(llam[i] + lS[n - i]);
+            }
+            bool nz = d != 0;
+            bool grow = nz && (2 * L <= (uint32_t)n);
+            uint32_t ld = tb.log(d);
+            uint32_t lc = ld + 255 - lb;
+            lc = lc >= 255 ? lc - 255 : lc;
+            // d == 0: the zero log puts every product below at zero, so no per-term select is needed
+            lc = nz ? lc : ZL;
+            const int hi = n + 1 < H ? n + 1 : H;
+            uint32_t old_llam[E];
 #pragma unroll
-        for (int i = 1; i <= hi; ++i) {
-            lam[i] ^= tb.exp_sum(lc + lBp[i]);
-            llam[i] = tb.log(lam[i]);
-        }
-        const int bh = n + 2 < H + 1 ? n + 2 : (H + 1 < E - 1 ? H + 1 : E - 1);
+            for (int i = 0; i < E; ++i)
+                old_llam[i] = llam[i];
+            const int hb = (n + 2) / 2 + 1 < hi ? (n + 2) / 2 + 1 : hi;
 #pragma unroll
-        for (int i = bh; i >= 1; --i)
-            lBp[i] = grow ? old_llam[i - 1] : lBp[i - 1];
-        lBp[0] = ZL;
-        if (grow) {
-            L = (uint32_t)n + 1 - L;
-            lb = ld;
+            for (int i = 1; i <= hb; ++i) {
+                lam[i] ^= tb.exp_sum(lc + lBp[i]);
+                llam[i] = tb.log(lam[i]);
+            }
+            // deg Lambda is at most the new L
+            if (hb < hi && __any((grow ? (uint32_t)n + 1 - L : L) > (uint32_t)hb)) {
+#pragma unroll
+                for (int i = hb + 1; i <= hi; ++i) {
+                    lam[i] ^= tb.exp_sum(lc + lBp[i]);
+                    llam[i] = tb.log(lam[i]);
+                }
+            }
+            const int bh = n + 2 < H + 1 ? n + 2 : (H + 1 < E - 1 ? H + 1 : E - 1);
+#pragma unroll
+            for (int i = bh; i >= 1; --i)
+                lBp[i] = grow ? old_llam[i - 1] : lBp[i - 1];
+            lBp[0] = ZL;
+            if (grow) {
+                L = (uint32_t)n + 1 - L;
+                lb = ld;
+            }
         }
     }
-    if (L > (uint32_t)E / 2)
+    if (L > e / 2)
         return false;
 #pragma unroll
     for (int w = 0; w < 12; ++w)
@@ -1645,16 +1569,15 @@ __device__ inline void wave_lds_sync()
 }
 
 
-// EB > 0: the BM records come from bm_fixed_one<EB> run per tile, one pending codeword per lane,
-// on the syndromes `synd` (its LDS lookups overlap the Chien loops of other waves); EB == 0:
-// from `rec`. G lanes per codeword in the Chien passes: 16 (sixteen positions each, four
+// The BM records come from bm_fixed_one<EB> run per tile, one pending codeword per lane, on the
+// syndromes `synd` (its LDS lookups overlap the Chien loops of other waves); ecc_len is at most EB. A BM kernel of its own, with records in HBM, took 56 us and this kernel 34 for 100,003
+// codewords of ecc 21; together 43. G lanes per codeword in the Chien passes: 16 (sixteen positions each, four
 // codewords per pass) or 8 (thirty-two each, eight per pass: half the per-pass work per
 // codeword, for small ecc where that work dominates).
-template <int WG, int EB, int G = 16>
+template <int WG, int EB, int G = 8>
 __global__ __launch_bounds__(WG) void rs256_chien16_kernel(uint8_t *__restrict__ msgs, uint8_t *__restrict__ eccs,
                                                             uint32_t count, uint32_t k, uint32_t E,
                                                             uint8_t *__restrict__ status,
-                                                            const uint32_t *__restrict__ rec,
                                                             const uint32_t *__restrict__ synd,
                                                             const uint32_t *__restrict__ ctab, Rs256Tables tab)
 {
@@ -1664,12 +1587,13 @@ __global__ __launch_bounds__(WG) void rs256_chien16_kernel(uint8_t *__restrict__
     __shared__ uint8_t s_exp2[EXP2_LEN];
     __shared__ uint16_t s_log2[256];
     static_assert(G == 16 || G == 8, "16 or 8 lanes per codeword");
-    // with the BM in the kernel (EB > 0) L <= EB / 2: only the nibble words of coefficients
-    // 1 .. EB / 2 travel between lanes and only that many degrees are ranked
-    constexpr int LMX = EB > 0 ? EB / 2 : CHIEN_LMAX;
-    constexpr int NW = EB > 0 ? (EB >= 8 ? EB / 4 : 1) : 8;
+    // L <= EB / 2: only the nibble words of coefficients 1 .. EB / 2 travel between lanes and only
+    // that many degrees are ranked
+    constexpr int LMX = EB / 2;
+    constexpr int NW = EB >= 8 ? EB / 4 : 1;
+    constexpr int EWS = EB <= 4 ? 1 : EB <= 8 ? 2 : EB <= 16 ? 4 : 8;  // syndrome dwords per codeword
     constexpr int D = 64 / G;               // position dwords per lane, and codewords per pass
-    constexpr int RS = D * LMX > 64 ? D * LMX : 64;  // root slots per wave (a pass has <= D LMX roots)
+    constexpr int RS = D * LMX + 64;  // root slots per wave (a pass has <= D LMX roots, 63 wait)
     __shared__ uint32_t s_roots[WG / 64 * RS];
     for (uint32_t i = threadIdx.x; i < CHIEN_TABLE_BYTES / 16; i += WG)
         s_ct4[i] = reinterpret_cast<const uint4 *>(ctab)[i];
@@ -1690,30 +1614,16 @@ __global__ __launch_bounds__(WG) void rs256_chien16_kernel(uint8_t *__restrict__
         const uint32_t cw = base + lane;
         bool pend = cw < count && status[cw] == RS_PENDING;
         uint32_t r[12];
-        if constexpr (EB > 0) {
 #pragma unroll
-            for (int w = 0; w < 12; ++w)
-                r[w] = 0;
-            if (pend && !bm_fixed_one<EB>(synd + (size_t)cw * ((EB + 3) / 4), tb, r)) {
-                status[cw] = 0;
-                pend = false;
-            }
+        for (int w = 0; w < 12; ++w)
+            r[w] = 0;
+        if (pend && !bm_fixed_one<EB>(synd + (size_t)cw * EWS, E, tb, r)) {
+            status[cw] = 0;
+            pend = false;
         }
         const uint64_t pm = __ballot(pend);
         if (!pm)
             continue;
-        if (EB > 0) {
-        } else if (pend) {
-            const uint4 *r4 = reinterpret_cast<const uint4 *>(rec + (size_t)cw * 12);
-            const uint4 a = r4[0], b = r4[1], c = r4[2];
-            r[0] = a.x; r[1] = a.y; r[2] = a.z; r[3] = a.w;
-            r[4] = b.x; r[5] = b.y; r[6] = b.z; r[7] = b.w;
-            r[8] = c.x; r[9] = c.y; r[10] = c.z; r[11] = c.w;
-        } else {
-#pragma unroll
-            for (int w = 0; w < 12; ++w)
-                r[w] = 0;
-        }
         const uint32_t L = r[0] & 0xffu;
         // bit 7 of byte q of dword d: position chien_pos(d, q) lies in the codeword (set up
         // after BM, whose registers it would otherwise add to)
@@ -1757,6 +1667,45 @@ __global__ __launch_bounds__(WG) void rs256_chien16_kernel(uint8_t *__restrict__
             rank = npend + __builtin_amdgcn_mbcnt_hi((uint32_t)(~pm >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)~pm, 0u));
         // lane r receives the lane of the codeword ranked r
         const uint32_t src = (uint32_t)__builtin_amdgcn_ds_permute((int)(rank * 4), (int)lane);
+        // One root per lane, `cnt` of them from slot `first`: Omega(X^-1) = sum_k Omega_k alpha^(-k p)
+        // from the logs held by the codeword's lane, then Forney's magnitude (as the reference's e = X
+        // Omega(X^-1) / Lambda'(X^-1), with Lambda' = X Lambda_odd in characteristic 2). The passes
+        // ascend in L, so Lmax of the last one bounds the degrees of all.
+        auto forney = [&](uint32_t first, uint32_t cnt, uint32_t Lmax) {
+            const uint32_t e = lane < cnt ? s_rt[first + lane] : 0u;
+            const uint32_t oc = e & 63u;
+            uint32_t ol[NWO];
+#pragma unroll
+            for (int m = 0; m < NWO; ++m)
+                ol[m] = (uint32_t)__builtin_amdgcn_ds_bpermute((int)(oc * 4), (int)olog[m]);
+            if (lane < cnt) {
+                const uint32_t p = (e >> 8) & 0xffu, dod = e >> 16;
+                // four terms at a time (their reads in flight together), up to the pass's
+                // largest degree; ek = -k p mod 255
+                uint32_t num = 0, ek = 0;
+#pragma unroll
+                for (int g4 = 0; g4 < (LMX + 3) / 4; ++g4) {
+                    if ((uint32_t)(4 * g4) >= Lmax)
+                        break;
+                    uint32_t x[4];
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) {
+                        const int kk = 4 * g4 + u;
+                        x[u] = kk < LMX ? s_exp2[((ol[kk >> 1] >> (16 * (kk & 1))) & 0xffffu) + ek] : 0u;
+                        ek = ek >= p ? ek - p : ek + 255 - p;
+                    }
+                    num ^= x[0] ^ x[1] ^ x[2] ^ x[3];
+                }
+                if (num) {
+                    const uint32_t lnm = s_log2[num], ld = s_log2[dod];
+                    const uint32_t mag = dod ? (uint32_t)s_exp2[lnm + 255 - ld] : (uint32_t)s_exp2[p + lnm];
+                    const uint32_t at = n - 1 - p;
+                    const size_t cwo = base + oc;
+                    xor_byte(at < k ? msgs + cwo * k + at : eccs + cwo * E + (at - k), mag);
+                }
+            }
+        };
+        uint32_t waiting = 0, Llast = 0;  // roots in the slots, taken 64 at a time
         const uint32_t npass = (npend + D - 1) / D;
         for (uint32_t ps = 0; ps < npass; ++ps) {
             const uint32_t rr = D * ps + grp;
@@ -1799,7 +1748,7 @@ __global__ __launch_bounds__(WG) void rs256_chien16_kernel(uint8_t *__restrict__
                 rm |= z[d] >> (7 - d);
             rm = ok ? rm : 0u;
             const uint32_t nr = (uint32_t)__builtin_popcount(rm);
-            uint32_t slot = 0, total = 0;  // exclusive prefix sum of nr (<= 4 D) by bit planes
+            uint32_t slot = waiting, total = 0;  // exclusive prefix sum of nr (<= 4 D) by bit planes
 #pragma unroll
             for (int b = 0; b < (D == 8 ? 6 : 5); ++b) {
                 const uint64_t m = __ballot((nr >> b) & 1u);
@@ -1819,45 +1768,17 @@ __global__ __launch_bounds__(WG) void rs256_chien16_kernel(uint8_t *__restrict__
                 s_rt[slot++] = o | (p << 8) | (((ov >> (8 * q)) & 0xffu) << 16);
             }
             wave_lds_sync();
-            // one root per lane: Omega(X^-1) = sum_k Omega_k alpha^(-k p) from the logs held by
-            // the codeword's lane, then Forney's magnitude (as the reference's e = X Omega(X^-1) /
-            // Lambda'(X^-1), with Lambda' = X Lambda_odd in characteristic 2)
-            for (uint32_t r0 = 0; r0 < total; r0 += 64) {
-                const uint32_t e = r0 + lane < total ? s_rt[r0 + lane] : 0u;
-                const uint32_t oc = e & 63u;
-                uint32_t ol[NWO];
-#pragma unroll
-                for (int m = 0; m < NWO; ++m)
-                    ol[m] = (uint32_t)__builtin_amdgcn_ds_bpermute((int)(oc * 4), (int)olog[m]);
-                if (r0 + lane < total) {
-                    const uint32_t p = (e >> 8) & 0xffu, dod = e >> 16;
-                    // four terms at a time (their reads in flight together), up to the pass's
-                    // largest degree; ek = -k p mod 255
-                    uint32_t num = 0, ek = 0;
-#pragma unroll
-                    for (int g4 = 0; g4 < (LMX + 3) / 4; ++g4) {
-                        if ((uint32_t)(4 * g4) >= Lmax)
-                            break;
-                        uint32_t x[4];
-#pragma unroll
-                        for (int u = 0; u < 4; ++u) {
-                            const int kk = 4 * g4 + u;
-                            x[u] = kk < LMX ? s_exp2[((ol[kk >> 1] >> (16 * (kk & 1))) & 0xffffu) + ek] : 0u;
-                            ek = ek >= p ? ek - p : ek + 255 - p;
-                        }
-                        num ^= x[0] ^ x[1] ^ x[2] ^ x[3];
-                    }
-                    if (num) {
-                        const uint32_t lnm = s_log2[num], ld = s_log2[dod];
-                        const uint32_t mag = dod ? (uint32_t)s_exp2[lnm + 255 - ld] : (uint32_t)s_exp2[p + lnm];
-                        const uint32_t at = n - 1 - p;
-                        const size_t cwo = base + oc;
-                        xor_byte(at < k ? msgs + cwo * k + at : eccs + cwo * E + (at - k), mag);
-                    }
-                }
+            waiting += total;
+            Llast = Lmax;
+            while (waiting >= 64) {
+                waiting -= 64;
+                forney(waiting, 64, Lmax);
             }
             wave_lds_sync();  // the next pass rewrites the slots
         }
+        if (waiting)
+            forney(0, waiting, Llast);
+        wave_lds_sync();
     }
 }
 
@@ -2215,7 +2136,7 @@ int launch_repair(ffrs_rs256 *rs, uint8_t *d_msg, uint8_t *d_ecc, size_t count, 
     return FFRS_OK;
 }
 
-// The wave-cooperative repair (ecc_len 33..254).
+// The wave-cooperative repair (ecc_len 33..254, and small launches of shorter ones).
 int launch_repair_wave(ffrs_rs256 *rs, uint8_t *d_msg, uint8_t *d_ecc, size_t count, uint32_t k, uint8_t *d_status)
 {
     ffrs_ctx *ctx = rs->ctx;
@@ -2308,22 +2229,20 @@ int reserve_work(ffrs_rs256 *rs, size_t bytes)
     return FFRS_OK;
 }
 
-// Whether the Chien kernel runs Berlekamp-Massey itself (ecc 2, 4, 8, 16, 32), so that the
-// pipeline keeps no BM records.
-bool bm_in_chien(uint32_t E) { return E == 2 || E == 4 || E == 8 || E == 16 || E == 32; }
+// Workspace of the repair pipeline for `count` codewords: the syndromes, EW dwords per codeword.
+size_t pipeline_work_bytes(uint32_t EW, size_t count) { return count * EW * 4; }
 
-// Workspace of the repair pipeline for `count` codewords of ecc E (word class EW): the
-// syndromes (EW dwords per codeword), then, for ecc outside bm_in_chien, the 48-byte BM
-// records from the next 256-byte boundary.
-size_t pipeline_work_bytes(uint32_t E, uint32_t EW, size_t count)
+// What a call of the allocation-free entry point may hold (its documented limit): the syndromes, and
+// for ecc_len outside 2, 4, 8, 16, 32 a 48-byte record per codeword.
+size_t noalloc_bytes(uint32_t E, uint32_t EW, size_t count)
 {
     const size_t synd_bytes = count * EW * 4;
-    if (bm_in_chien(E))
+    if (E == 2 || E == 4 || E == 8 || E == 16 || E == 32)
         return synd_bytes;
-    return ((synd_bytes + 255) & ~(size_t)255) + count * rec_stride(E);
+    return ((synd_bytes + 255) & ~(size_t)255) + count * 48;
 }
 
-// The pipeline over a workspace `work` of at least pipeline_work_bytes(E, EW, count) bytes.
+// The pipeline over a workspace `work` of at least pipeline_work_bytes(EW, count) bytes.
 // Nothing in it needs to start at zero: the syndrome kernel writes the syndromes of every
 // codeword it marks pending, and only pending codewords' entries are read after it.
 template <int EW, int S>
@@ -2332,9 +2251,7 @@ int launch_repair_pipeline(ffrs_rs256 *rs, uint8_t *d_msg, uint8_t *d_ecc, size_
 {
     ffrs_ctx *ctx = rs->ctx;
     const uint32_t E = rs->ecc;
-    size_t synd_bytes = count * EW * 4;
     uint32_t *d_synd = (uint32_t *)work;
-    uint8_t *d_rec = (uint8_t *)work + ((synd_bytes + 255) & ~(size_t)255);
     Rs256Tables tab{rs->d_lut, rs->d_exp2, rs->d_log2};
 
     const bool coop = lfsr_load_mode<EW, S>(k, true) == LOAD_COOP;
@@ -2353,45 +2270,31 @@ int launch_repair_pipeline(ffrs_rs256 *rs, uint8_t *d_msg, uint8_t *d_ecc, size_
     FFRS_HIP(hipGetLastError());
     mark_kernel(ctx);
 
-    // ecc 2, 4, 8, 16, 32: BM inside the Chien kernel, no records (512 threads for ecc 32,
-    // whose BM would spill registers at 768); eight lanes per codeword in its passes, faster
-    // than sixteen at every ecc measured (1 M codewords of ecc 32: 402 vs 416 us; 2 M of ecc
-    // 16: 317 vs 348 us; 4 M of ecc 8: 384 vs 412 us)
+    // BM inside the Chien kernel, unrolled for the next of 2, 4, 8, 16, 24, 32. The last two hold more
+    // registers: 768 threads where that fills the CUs, 512 below (us, 512 / 768: 1 M codewords of ecc
+    // 32 421 / 381, of ecc 24 274 / 263; 131,072 of ecc 27 53 / 65); eight lanes per codeword in its passes, faster
+    // than sixteen at every ecc measured (1 M codewords of ecc 32: 402 vs 416 us; 2 M of ecc 16: 317
+    // vs 348 us; 4 M of ecc 8: 384 vs 412 us)
     auto fused = [&](auto kern, int wg) -> int {
         int g = persistent_grid(ctx, 1, (count + wg - 1) / wg);
         hipLaunchKernelGGL(kern, dim3(g), dim3(wg), 0, ctx->stream, d_msg, d_ecc, (uint32_t)count, k, E, d_status,
-                           (const uint32_t *)nullptr, (const uint32_t *)d_synd, rs->d_ctab, tab);
+                           (const uint32_t *)d_synd, rs->d_ctab, tab);
         FFRS_HIP(hipGetLastError());
         mark_kernel(ctx);
         return FFRS_OK;
     };
-    switch (E) {
-    case 2: return fused(rs256_chien16_kernel<1024, 2, 8>, 1024);
-    case 4: return fused(rs256_chien16_kernel<1024, 4, 8>, 1024);
-    case 8: return fused(rs256_chien16_kernel<1024, 8, 8>, 1024);
-    case 16: return fused(rs256_chien16_kernel<1024, 16, 8>, 1024);
-    case 32: return fused(rs256_chien16_kernel<512, 32, 8>, 512);
-    default: break;
-    }
-    // other ecc: Berlekamp-Massey from the log tables, one lane per codeword, records in the
-    // workspace
-    size_t lds2 = EXP2_LEN + 512 + (size_t)256 * bm_row_stride(E);
-    if (int r = allow_lds(rs256_bm_kernel<256>, lds2))
-        return r;
-    int g2 = persistent_grid(ctx, (int)std::max<size_t>(1, (160 * 1024) / lds2), (count + 255) / 256);
-    hipLaunchKernelGGL((rs256_bm_kernel<256>), dim3(g2), dim3(256), lds2, ctx->stream, (uint32_t)count, E,
-                       (uint32_t)EW, d_status, (const uint32_t *)d_synd, d_rec, tab);
-    FFRS_HIP(hipGetLastError());
-    mark_kernel(ctx);
-    // Chien + Forney: the 128 KB table fills the CU's LDS, one workgroup of sixteen waves per CU
-    constexpr int WGC = 1024;
-    int gc = persistent_grid(ctx, 1, (count + WGC - 1) / WGC);
-    hipLaunchKernelGGL((rs256_chien16_kernel<WGC, 0, 8>), dim3(gc), dim3(WGC), 0, ctx->stream, d_msg, d_ecc,
-                       (uint32_t)count, k, E, d_status, (const uint32_t *)d_rec, (const uint32_t *)d_synd, rs->d_ctab,
-                       tab);
-    FFRS_HIP(hipGetLastError());
-    mark_kernel(ctx);
-    return FFRS_OK;
+    if (E <= 2)
+        return fused(rs256_chien16_kernel<1024, 2>, 1024);
+    if (E <= 4)
+        return fused(rs256_chien16_kernel<1024, 4>, 1024);
+    if (E <= 8)
+        return fused(rs256_chien16_kernel<1024, 8>, 1024);
+    if (E <= 16)
+        return fused(rs256_chien16_kernel<1024, 16>, 1024);
+    const bool wide = count >= (size_t)ctx->cu_count * 768;
+    if (E <= 24)
+        return wide ? fused(rs256_chien16_kernel<768, 24>, 768) : fused(rs256_chien16_kernel<512, 24>, 512);
+    return wide ? fused(rs256_chien16_kernel<768, 32>, 768) : fused(rs256_chien16_kernel<512, 32>, 512);
 }
 
 // The replicated tables (128 KB per workgroup to load) for launches of at least 8,192
@@ -2433,7 +2336,16 @@ int encode_device(ffrs_rs256 *rs, size_t message_len, const uint8_t *d_msg, size
 // workspace) or the one-kernel lane mode (which does not).
 bool uses_pipeline(const ffrs_rs256 *rs) { return rs->EW <= 8 && rs->repair_mode != 2; }
 
-// `work`: the pipeline's workspace, at least pipeline_work_bytes(ecc, EW, min(count,
+// Small launches take one codeword per wave: the pipeline's kernels load up to 128 KB of tables per
+// workgroup and need 64 codewords per wave to fill (us, pipeline / wave: ecc 32 k 223 one codeword
+// 41 / 20, 4,096 78 / 35, 8,192 90 / 55, 16,384 90 / 97; ecc 8 4,096 39 / 16, 16,384 45 / 39, 24,576
+// 46 / 54).
+bool small_repair(const ffrs_rs256 *rs, size_t count)
+{
+    return rs->repair_mode == 0 && rs->EW <= 8 && count <= 12288;
+}
+
+// `work`: the pipeline's workspace, at least pipeline_work_bytes(EW, min(count,
 // max_batch)) bytes, or nullptr to use (and grow) the codec's own.
 int repair_device(ffrs_rs256 *rs, size_t message_len, uint8_t *d_msg, uint8_t *d_ecc, size_t count,
                   uint8_t *d_status, void *work = nullptr)
@@ -2443,11 +2355,13 @@ int repair_device(ffrs_rs256 *rs, size_t message_len, uint8_t *d_msg, uint8_t *d
         return FFRS_OK;
     uint32_t k = (uint32_t)message_len;
     size_t step = max_batch(message_len);
-    // The pipeline is faster at every batch size measured (142 codewords of ecc 32:
-    // 274 us against 373 us lane by lane); the lane kernel stays selectable.
+    if (small_repair(rs, count))
+        return launch_repair_wave(rs, d_msg, d_ecc, count, k, d_status);
+    // The lane kernel stays selectable (142 codewords of ecc 32: 373 us against 274 us in the
+    // pipeline).
     const bool pipe = uses_pipeline(rs);
     if (pipe && !work) {
-        if (int r = reserve_work(rs, pipeline_work_bytes(rs->ecc, rs->EW, std::min(step, count))))
+        if (int r = reserve_work(rs, pipeline_work_bytes(rs->EW, std::min(step, count))))
             return r;
         work = rs->d_work;
     }
@@ -2668,12 +2582,12 @@ int ffrs_rs256_repair_device_noalloc(ffrs_rs256 *rs, size_t message_len, uint8_t
     void *work = nullptr;
     if (count && uses_pipeline(rs)) {
         const size_t per_launch = std::min(max_batch(message_len), count);
-        const size_t need = pipeline_work_bytes(rs->ecc, rs->EW, per_launch);
+        const size_t need = noalloc_bytes(rs->ecc, rs->EW, per_launch);
         if (need > (size_t)FFRS_RS256_NOALLOC_SCRATCH_BYTES) {
             size_t most = 0;  // the largest count whose workspace fits
             for (size_t lo = 0, hi = per_launch; lo <= hi;) {
                 const size_t mid = lo + (hi - lo) / 2;
-                if (pipeline_work_bytes(rs->ecc, rs->EW, mid) <= (size_t)FFRS_RS256_NOALLOC_SCRATCH_BYTES) {
+                if (noalloc_bytes(rs->ecc, rs->EW, mid) <= (size_t)FFRS_RS256_NOALLOC_SCRATCH_BYTES) {
                     most = mid;
                     lo = mid + 1;
                 } else {
