@@ -1766,10 +1766,12 @@ __global__ __launch_bounds__(64) void rsi16_repair_one_kernel(uint16_t *__restri
     repair_group_reg<E, false, true>(T, msgs + (size_t)cw * T.k, eccs + (size_t)cw * E, s_mem, L, status + cw);
 }
 
-template <int E>
+// One codeword per lane group; SIN: the syndromes are given.
+template <int E, bool SIN = false>
 __global__ __launch_bounds__(64) void rsi16_repair_reg_kernel(uint16_t *__restrict__ msgs,
                                                                uint16_t *__restrict__ eccs, uint32_t count,
-                                                               uint8_t *__restrict__ status, Rsi16Dev T)
+                                                               uint8_t *__restrict__ status, Rsi16Dev T,
+                                                               const uint32_t *__restrict__ syn = nullptr)
 {
     extern __shared__ uint32_t s_mem[];
     constexpr uint32_t G = RegShape<E>::G, cpw = 64 / G;
@@ -1779,7 +1781,8 @@ __global__ __launch_bounds__(64) void rsi16_repair_reg_kernel(uint16_t *__restri
         return;
     LaneR<E> L;
     L.init(T, threadIdx.x);
-    repair_group_reg<E>(T, msgs + (size_t)cw * T.k, eccs + (size_t)cw * E, s_mem + grp * REG_WORDS * E, L, status + cw);
+    repair_group_reg<E, SIN>(T, msgs + (size_t)cw * T.k, eccs + (size_t)cw * E, s_mem + grp * REG_WORDS * E, L,
+                             status + cw, SIN ? syn + (size_t)cw * E : nullptr);
 }
 
 __global__ __launch_bounds__(64) void rsi16_repair_kernel(uint16_t *__restrict__ msgs, uint16_t *__restrict__ eccs,
@@ -4326,23 +4329,32 @@ int launch_repair_reg(ffrs_rsi16 *rs, uint16_t *d_msg, uint16_t *d_ecc, size_t c
 {
     constexpr uint32_t cpw = 64 / RegShape<E>::G;
     const size_t lds = (size_t)cpw * REG_WORDS * E * 4;
-    // One codeword per wave while that leaves at most two waves per SIMD, the groups of the wave
-    // sharing its chunks (us against the general kernel: 1 codeword RSi16(256,32) 10.4 / 14.6,
-    // (1024,8) 12 / 78, (4096,32) 17 / 61; 2,048: 28 / 30, 18 / 89, 64 / 175; 16,384: 98 / 55).
+    const size_t cus = rs->ctx->cu_count;
+    // One codeword per wave, its groups sharing the chunks, while the chip takes the waves in a few
+    // rounds: the longer the block, the more of them the general kernel's serial chunks cost (us, this
+    // / best other: RSi16(64,16) 512 codewords 16 / 16, 2,048 21 / 16; (256,32) 2,048 29 / 36, 4,096
+    // 46 / 36; (1024,16) 8,192 52 / 55, 16,384 92 / 71; (2048,32) 4,096 66 / 75, 8,192 108 / 93).
     if constexpr (E <= 32)
-    if (rs->repair_synd != 1 && count <= 8 * (size_t)rs->ctx->cu_count) {
+    if (rs->repair_synd == 0 && count <= std::min<size_t>((E == 32 ? 16 : 32) * cus, cus / 2 * rs->n / E)) {
         hipLaunchKernelGGL(rsi16_repair_one_kernel<E>, dim3((unsigned)count), dim3(64), 0, rs->ctx->stream, d_msg, d_ecc,
                            d_status, rs->dev);
         FFRS_HIP(hipGetLastError());
         mark_kernel(rs->ctx);
         return FFRS_OK;
     }
-    // The syndromes on the matrix cores first, where their tables exist; for ecc_len 8 to 32 then one
-    // codeword per lane, from the counts on where 64 codewords per wave fill the chip and the three
-    // launches pay (us, general kernel / this: RSi16(256,32) 16,384 codewords 55 / 64, 32,768 91 / 66,
-    // 262,144 544 / 179; (1024,8) 4,096 89 / 47; (64,8) 32,768 20 / 23, 262,144 74 / 55).
-    const bool lanes = E <= 32 && count * rs->n >= ((size_t)1 << 22) && count >= (E == 8 ? 2048 : 24576);
-    const bool msyn = rs->synd.dev.nq && rs->repair_synd != 1 && (E >= 64 || lanes || rs->repair_synd == 2) &&
+    // The syndromes on the matrix cores first, where their tables exist. For ecc_len 8 to 32 then one
+    // codeword per lane from the counts on where 64 codewords a wave fill the chip and three launches
+    // pay (us, lane / best other: RSi16(64,8) 16,384 codewords 18 / 17, 24,576 18 / 20; (256,8) 8,192
+    // 22 / 27; (1024,16) 16,384 80 / 71, 24,576 79 / 87; (2608,16) 16,384 125 / 134; (256,32) 8,192
+    // 61 / 47, 16,384 64 / 74; 65,536 100 / 161; (32,16) 24,576 29 / 25).
+    const bool lanes = rs->repair_synd == 2 ||
+                       (count * rs->n > ((size_t)1 << 20) &&
+                        (E == 8 || (rs->n >= 2048 ? count > 32 * cus : count >= (E == 16 ? 80 : 64) * cus)));
+    // Else the general kernel, given the syndromes where the block has chunks enough for that to pay
+    // (us, given / not: (2608,16) 8,192 codewords 120 / 163, (512,32) 8,192 43 / 48, (1024,32) 16,384
+    // 88 / 113; (256,32) 4,096 39 / 36, (64,16) 4,096 19 / 17).
+    const bool given = E <= 32 && !lanes && rs->n >= 16 * E;
+    const bool msyn = rs->synd.dev.nq && rs->repair_synd != 1 && (E >= 64 || lanes || given) &&
                       (((uintptr_t)d_msg | (uintptr_t)d_ecc) & 15) == 0;
     if (msyn) {
         // workspace: E syndromes per codeword and the list of those left to the general kernel
@@ -4367,7 +4379,13 @@ int launch_repair_reg(ffrs_rsi16 *rs, uint16_t *d_msg, uint16_t *d_ecc, size_t c
                     return r;
                 mark_kernel(rs->ctx);
             }
-            if constexpr (E >= 8 && E <= 32) {
+            if (given) {
+                if (int r = allow_lds(rsi16_repair_reg_kernel<E, true>, lds))
+                    return r;
+                hipLaunchKernelGGL((rsi16_repair_reg_kernel<E, true>), dim3((unsigned)((c + cpw - 1) / cpw)), dim3(64),
+                                   lds, rs->ctx->stream, m, e, (uint32_t)c, d_status + b, rs->dev,
+                                   (const uint32_t *)syn);
+            } else if constexpr (E >= 8 && E <= 32) {
                 hipLaunchKernelGGL(rsi16_repair_lane_kernel<E>, dim3((unsigned)((c + 63) / 64)), dim3(64), 0,
                                    rs->ctx->stream, m, e, (uint32_t)c, d_status + b, rs->dev, rs->roots.dev, syn, list);
                 FFRS_HIP(hipGetLastError());
