@@ -2586,7 +2586,9 @@ __global__ __launch_bounds__(64, 4) void rsi16_repair_lane_kernel(uint16_t *__re
     }
 }
 
-constexpr uint8_t ODD = 254, ODD_SOLVED = 253;  // transient statuses of listed codewords (ecc_len >= 64)
+// Transient statuses for ecc_len >= 64: listed codewords, and those with a record for the root search.
+// The last is no final status: the list is worked off while later workgroups of the search still pick theirs.
+constexpr uint8_t ODD = 254, ODD_SOLVED = 253, SEARCH = 252;
 
 // The codewords list[1 .. list[0]] through the general register repair, one per wave (worker
 // `first` of `step`): a few in a launch of many, so what counts is the time of one.
@@ -2641,7 +2643,7 @@ __global__ __launch_bounds__(64) void rsi16_repair_list_kernel(uint16_t *__restr
 //   bytes   a_i 3^i, i = 1 .. T, as low and high int8 limbs (T bytes each; RootTab)
 //   int16   evaluator coefficients 0 .. T - 1, then i a_i (the locator's derivative), i = 1 .. T
 //   word    a_0 + 65536 * steps
-// and status set to 2 (to be searched). Codewords that took irregular steps can have longer evaluators;
+// and status set to SEARCH. Codewords that took irregular steps can have longer evaluators;
 // they are listed for the general root search with status ODD_SOLVED and a row of 3 T / 2 + 2 words:
 //   u16     evaluator coefficients 0 .. E - 1, then a_0 .. a_T; a last word with the locator's length
 // Those left unsolved keep their syndromes and are listed with status ODD.
@@ -2983,7 +2985,7 @@ __global__ __launch_bounds__(64) void rsi16_solve_wave_kernel(uint32_t count, ui
             ev[C * lane + h] = (int16_t)r[h];
     if (lane == 0) {
         row[3 * T / 2] = bal_canon(a0) | (steps << 16);
-        status[cw] = FFRS_RSI16_REPAIR_OK;
+        status[cw] = SEARCH;
     }
 }
 
@@ -3018,9 +3020,10 @@ __global__ __launch_bounds__(512) void rsi16_roots_wave_kernel(uint16_t *__restr
         const uint32_t w = i / T, j = i % T;
         s_co[w * WORDS + j] = rec[(size_t)min(cw0 + w, count - 1) * E + T / 2 + j];
     }
+    bool on = false;  // lane w < CW: codeword w is searched here
     if (threadIdx.x < CW) {
         const uint32_t cw = min(cw0 + threadIdx.x, count - 1);
-        const bool on = cw0 + threadIdx.x < count && status[cw] == FFRS_RSI16_REPAIR_OK;
+        on = cw0 + threadIdx.x < count && status[cw] == SEARCH;
         s_last[threadIdx.x] = on ? rec[(size_t)cw * E + 3 * T / 2] : 1u;  // the constant 1: no roots
         s_found[threadIdx.x] = on ? 0u : 1u;
     }
@@ -3032,13 +3035,13 @@ __global__ __launch_bounds__(512) void rsi16_roots_wave_kernel(uint16_t *__restr
 #pragma unroll
     for (int g = 0; g < CG; ++g) {
         const uint32_t w = 16 * g + c, cw = min(cw0 + w, count - 1);
-        const bool on = (s_found[w] & 1) == 0;
+        const bool live = (s_found[w] & 1) == 0;
         const uint4 *lim = reinterpret_cast<const uint4 *>(rec + (size_t)cw * E);
 #pragma unroll
         for (int f = 0; f < KF; ++f) {
-            lo[g][f] = as_v4i(lim[4 * f + h]) & (on ? -1 : 0);
+            lo[g][f] = as_v4i(lim[4 * f + h]) & (live ? -1 : 0);
             if constexpr (KF == 1)
-                alt[g][f] = as_v4i(lim[h ^ 2]) & (on ? -1 : 0);
+                alt[g][f] = as_v4i(lim[h ^ 2]) & (live ? -1 : 0);
         }
         loc0[g] = (int32_t)(s_last[w] & 0xffffu);
     }
@@ -3158,8 +3161,8 @@ __global__ __launch_bounds__(512) void rsi16_roots_wave_kernel(uint16_t *__restr
         const uint32_t err = F::mul(nc ? F::mul(nc, scale) : 0u, r.x);
         *r.at = (uint16_t)(F::add(r.sym, err) & 0xffff);
     }
-    if (threadIdx.x < CW && s_found[threadIdx.x] == 0)
-        status[cw0 + threadIdx.x] = FFRS_RSI16_ERROR_LOCATION_FAIL;
+    if (on)
+        status[cw0 + threadIdx.x] = s_found[threadIdx.x] ? FFRS_RSI16_REPAIR_OK : FFRS_RSI16_ERROR_LOCATION_FAIL;
 }
 
 // ---------------------------------------------------------------- interleaved repair, SIMD words
