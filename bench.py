@@ -317,17 +317,22 @@ def run_plain(name, args):
     value = msg_bytes / (ms_step * 1e-3) / 1e9
     if rs256:
         enc_names = ["rs256_encode_kernel"]
-        # ecc 2, 4, 8, 16, 32 run BM inside the Chien kernel; other ecc <= 32 launch it on its own
-        rep_names = (["rs256_synd_kernel", "rs256_chien16_kernel"] if ecc in (2, 4, 8, 16, 32)
-                     else ["rs256_synd_kernel", "rs256_bm_kernel", "rs256_chien16_kernel"] if ecc <= 32
-                     else ["rs256_repair_kernel"])
+        # up to 12,288 codewords and above ecc 32 one wave per codeword
+        rep_names = (["rs256_synd_kernel", "rs256_chien16_kernel"] if ecc <= 32 and N > 12288
+                     else ["rs256_repair_wave_kernel"])
     else:
-        # the int8 MFMA contraction where it applies (these shapes have no mix constant of 65536)
-        enc_names = ["rsi16_encode_mfma_kernel" if ecc % 16 == 0 and ecc <= 256 and k <= 16384 else
+        # the int8 MFMA contraction where it applies (these shapes have no mix constant of 65536), ahead of
+        # the key equation and the root search too
+        mfma = ecc in (8, 16, 32, 64, 128, 256) and k <= 16384
+        contract = "rsi16_contract_wave_kernel" if ecc <= 32 else "rsi16_contract_kernel"
+        enc_names = [contract + " (parity)" if mfma else
                      "rsi16_encode_lane_kernel" if ecc <= 32 else
                      ("rsi16_encode_reg_kernel" if ecc <= 256 else "rsi16_encode_kernel")]
-        # syndromes as an int8 MFMA contraction ahead of the register repair where its tables exist
-        rep_names = ((["rsi16_synd_mfma_kernel"] if ecc in (16, 32, 64) and k <= 16384 else []) +
+        nk = len(krs[0])  # the launcher picks by count and block length
+        rep_names = ([contract + " (syndromes)", "rsi16_repair_lane_kernel", "rsi16_repair_list_kernel"]
+                     if nk == 3 and ecc <= 32 else
+                     [contract + " (syndromes)", "rsi16_solve_wave_kernel", "rsi16_roots_wave_kernel"] if nk == 3 else
+                     [contract + " (syndromes)", "rsi16_repair_reg_kernel"] if nk == 2 else
                      ["rsi16_repair_reg_kernel" if ecc <= 256 else "rsi16_repair_kernel"])
     ke_ms = np.mean(np.array(kes), axis=0)
     kr_ms = np.mean(np.array(krs), axis=0)

@@ -1570,8 +1570,9 @@ __device__ inline void wave_lds_sync()
 
 
 // The BM records come from bm_fixed_one<EB> run per tile, one pending codeword per lane, on the
-// syndromes `synd` (its LDS lookups overlap the Chien loops of other waves); ecc_len is at most EB. A BM kernel of its own, with records in HBM, took 56 us and this kernel 34 for 100,003
-// codewords of ecc 21; together 43. G lanes per codeword in the Chien passes: 16 (sixteen positions each, four
+// syndromes `synd` (its LDS lookups overlap the Chien loops of other waves); ecc_len is at most EB. A BM
+// kernel of its own, with records in HBM, took 56 us and this kernel 34 for 100,003 codewords of
+// ecc 21; together 43. G lanes per codeword in the Chien passes: 16 (sixteen positions each, four
 // codewords per pass) or 8 (thirty-two each, eight per pass: half the per-pass work per
 // codeword, for small ecc where that work dominates).
 template <int WG, int EB, int G = 8>
@@ -1990,7 +1991,7 @@ struct ffrs_rs256 {
     uint16_t *d_log2 = nullptr;
     uint32_t *d_stab = nullptr;  // syndrome nibble tables (ecc <= 32)
     uint32_t *d_ctab = nullptr;  // Chien nibble tables (ecc <= 32)
-    void *d_work = nullptr;      // syndromes + BM records of the last repair
+    void *d_work = nullptr;      // syndromes of the last repair
     size_t work_size = 0;
     int repair_mode = 0;         // 0 automatic, 1 pipeline (ecc <= 32), 2 one kernel, lane per codeword
 };

@@ -3016,15 +3016,17 @@ __global__ __launch_bounds__(512) void rsi16_roots_wave_kernel(uint16_t *__restr
         return;
     }
     const uint32_t cw0 = (blockIdx.x - list_blocks) * CW;
+    bool on = false;  // lane w < CW: codeword w is searched here
+    if (threadIdx.x < CW)
+        on = cw0 + threadIdx.x < count && status[cw0 + threadIdx.x] == SEARCH;
+    if (!__syncthreads_or(on))  // clean, listed: nothing to search
+        return;
     for (uint32_t i = threadIdx.x; i < (uint32_t)CW * T; i += 64 * NW) {
         const uint32_t w = i / T, j = i % T;
         s_co[w * WORDS + j] = rec[(size_t)min(cw0 + w, count - 1) * E + T / 2 + j];
     }
-    bool on = false;  // lane w < CW: codeword w is searched here
     if (threadIdx.x < CW) {
-        const uint32_t cw = min(cw0 + threadIdx.x, count - 1);
-        on = cw0 + threadIdx.x < count && status[cw] == SEARCH;
-        s_last[threadIdx.x] = on ? rec[(size_t)cw * E + 3 * T / 2] : 1u;  // the constant 1: no roots
+        s_last[threadIdx.x] = on ? rec[(size_t)(cw0 + threadIdx.x) * E + 3 * T / 2] : 1u;  // the constant 1: no roots
         s_found[threadIdx.x] = on ? 0u : 1u;
     }
     if (threadIdx.x == 0)
@@ -4280,8 +4282,13 @@ int launch_encode(ffrs_rsi16 *rs, const uint16_t *d_msg, size_t count, uint16_t 
     marks_begin(rs->ctx);
     if (count == 0)
         return FFRS_OK;
-    // the linear map on the matrix cores where it is the encode of the words asked for
-    if (rs->enc.dev.nq && I == 1 && rs->encode_mode != 1 &&
+    // the linear map on the matrix cores where it is the encode of the words asked for; but not for a few
+    // codewords of ecc_len 128 or 256, whose matrix (2 bytes an entry) one workgroup takes longer to go through
+    // (us, contraction / butterflies: RSi16(4096,256) 64 codewords 32 / 28, 1,024 33 / 29, 4,096
+    // 37 / 59; (16384,256) 256 codewords 120 / 98; (896,128) 1,024 10 / 10, one 9 / 9 with warm caches;
+    // (4096,128) 512 codewords 26 / 29).
+    const size_t few = rs->E == 256 ? 4 * (size_t)rs->ctx->cu_count : rs->E == 128 ? 16 : 0;
+    if (rs->enc.dev.nq && I == 1 && rs->encode_mode != 1 && (rs->encode_mode == 2 || count > few) &&
         !(vec && rs->mix_minus_one) && (((uintptr_t)d_msg | (uintptr_t)d_ecc) & 15) == 0)
         return launch_encode_mfma(rs, d_msg, count, d_ecc);
     // one lane per codeword (g = 1): the register kernel for ecc_len <= 32, plain layout
@@ -4357,7 +4364,12 @@ int launch_repair_reg(ffrs_rsi16 *rs, uint16_t *d_msg, uint16_t *d_ecc, size_t c
     // (us, given / not: (2608,16) 8,192 codewords 120 / 163, (512,32) 8,192 43 / 48, (1024,32) 16,384
     // 88 / 113; (256,32) 4,096 39 / 36, (64,16) 4,096 19 / 17).
     const bool given = E <= 32 && !lanes && rs->n >= 16 * E;
-    const bool msyn = rs->synd.dev.nq && rs->repair_synd != 1 && (E >= 64 || lanes || given) &&
+    // ecc_len 128, a few codewords: one launch instead of three, each about 10 us in a call with nothing
+    // queued behind it (one RSi16(896,128) encode and repair through the host, one launch / three: clean
+    // 86 / 105 us, 56 errors 137 / 126). At ecc_len 256 the solver's gain is worth them (RSi16(4096,256):
+    // 100 errors 274 / 183, clean 128 / 149).
+    const bool single = E == 128 && rs->repair_synd == 0 && count <= 16;
+    const bool msyn = rs->synd.dev.nq && rs->repair_synd != 1 && ((E >= 64 && !single) || lanes || given) &&
                       (((uintptr_t)d_msg | (uintptr_t)d_ecc) & 15) == 0;
     if (msyn) {
         // workspace: E syndromes per codeword and the list of those left to the general kernel

@@ -11,7 +11,7 @@ pytestmark = pytest.mark.gpu
 
 SHAPES = [(16, 2, 1025), (64, 8, 1025), (64, 8, 16385), (128, 8, 8193), (64, 16, 513), (256, 16, 2049), (512, 16, 4097),
           (512, 16, 20479), (2048, 16, 8193), (256, 32, 1025), (512, 32, 2049), (512, 32, 16383), (512, 32, 16384),
-          (2048, 32, 4097)]
+          (2048, 32, 4097), (896, 128, 16), (896, 128, 17)]
 
 
 @pytest.mark.parametrize("n,ecc,count", SHAPES)
