@@ -937,8 +937,10 @@ struct alignas(16) WaveRows {
     uint16_t lo[128];   // logs of Omega_0..L-1
 };
 
-// NC Lambda coefficients and NS syndromes per lane (E/2 + 1 <= 64 NC, E <= 64 NS).
-template <int NC, int NS>
+// NC Lambda coefficients and NS syndromes per lane (E/2 + 1 <= 64 NC, E <= 64 NS). SEG, for E <= 32:
+// the lanes left over by the syndromes share the positions; as a run-time choice this cost the longer
+// codes 6 % (12,896 codewords of ecc 44 90 -> 96 us).
+template <int NC, int NS, bool SEG = false>
 __device__ inline uint8_t repair_wave(uint8_t *pm, uint8_t *pe, uint32_t k, uint32_t E, const GfLds &gf, WaveRows &w)
 {
     const uint32_t lane = threadIdx.x & 63, n = k + E, H = E / 2;
@@ -951,9 +953,9 @@ __device__ inline uint8_t repair_wave(uint8_t *pm, uint8_t *pe, uint32_t k, uint
         w.lc[j] = (uint16_t)gf.log2[c];
     }
     __builtin_amdgcn_wave_barrier();
-    // ---- syndromes: lane l sums S_(l + 64 q) over the positions; for E <= 32 the lanes are SG
+    // ---- syndromes: lane l sums S_(l + 64 q) over the positions; with SEG the lanes are SG
     // groups of 64 / SG, each over every SG-th run of eight positions, XORed together afterwards
-    const uint32_t SG = NS > 1 || E > 32 ? 1 : E > 16 ? 2 : E > 8 ? 4 : 8, EP = 64 / SG, seg = lane / EP;
+    const uint32_t SG = !SEG ? 1 : E > 16 ? 2 : E > 8 ? 4 : 8, EP = 64 / SG, seg = lane / EP;
     uint32_t sy[NS], e[NS], st[NS], skip[NS];
 #pragma unroll
     for (int q = 0; q < NS; ++q) {
@@ -976,14 +978,16 @@ __device__ inline uint8_t repair_wave(uint8_t *pm, uint8_t *pe, uint32_t k, uint
                 t[u] = gf.exp2[((lw[u >> 1] >> (16 * (u & 1))) & 0xffffu) + e[q]];
                 e[q] = e[q] >= st[q] ? e[q] - st[q] : e[q] + 255 - st[q];
             }
-            e[q] = e[q] >= skip[q] ? e[q] - skip[q] : e[q] + 255 - skip[q];
+            if constexpr (SEG)
+                e[q] = e[q] >= skip[q] ? e[q] - skip[q] : e[q] + 255 - skip[q];
 #pragma unroll
             for (int u = 0; u < 8; ++u)
                 sy[q] ^= t[u];
         }
     }
-    for (uint32_t s = EP; s < 64; s <<= 1)
-        sy[0] ^= (uint32_t)__shfl_xor((int)sy[0], (int)s);
+    if constexpr (SEG)
+        for (uint32_t s = EP; s < 64; s <<= 1)
+            sy[0] ^= (uint32_t)__shfl_xor((int)sy[0], (int)s);
     uint32_t any = 0;
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
@@ -1156,7 +1160,7 @@ __device__ inline uint8_t repair_wave(uint8_t *pm, uint8_t *pe, uint32_t k, uint
 }
 
 // One codeword per wave over `count` codewords of message length k (rows of k and E bytes).
-template <int NC, int NS, int WG>
+template <int NC, int NS, int WG, bool SEG = false>
 __global__ __launch_bounds__(WG) void rs256_repair_wave_kernel(uint8_t *__restrict__ msgs, uint8_t *__restrict__ eccs,
                                                                 uint32_t count, uint32_t k, uint32_t E,
                                                                 uint8_t *__restrict__ status, Rs256Tables tab)
@@ -1173,7 +1177,7 @@ __global__ __launch_bounds__(WG) void rs256_repair_wave_kernel(uint8_t *__restri
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     WaveRows &w = s_rows[wave];
     for (uint32_t cw = blockIdx.x * (WG / 64) + wave; cw < count; cw += gridDim.x * (WG / 64)) {
-        const uint8_t st = repair_wave<NC, NS>(msgs + (size_t)cw * k, eccs + (size_t)cw * E, k, E, gf, w);
+        const uint8_t st = repair_wave<NC, NS, SEG>(msgs + (size_t)cw * k, eccs + (size_t)cw * E, k, E, gf, w);
         if ((threadIdx.x & 63) == 0)
             status[cw] = st;
         __builtin_amdgcn_wave_barrier();
@@ -2152,6 +2156,8 @@ int launch_repair_wave(ffrs_rs256 *rs, uint8_t *d_msg, uint8_t *d_ecc, size_t co
         mark_kernel(ctx);
         return FFRS_OK;
     };
+    if (E <= 32)
+        return go(rs256_repair_wave_kernel<1, 1, WG, true>);
     if (E <= 64)
         return go(rs256_repair_wave_kernel<1, 1, WG>);
     if (E <= 124)
