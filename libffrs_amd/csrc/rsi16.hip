@@ -2642,7 +2642,8 @@ __global__ __launch_bounds__(64) void rsi16_repair_list_kernel(uint16_t *__restr
 // words) is replaced by what the root search needs, a record of 3 T / 2 + 1 words:
 //   bytes   a_i 3^i, i = 1 .. T, as low and high int8 limbs (T bytes each; RootTab)
 //   int16   evaluator coefficients 0 .. T - 1, then i a_i (the locator's derivative), i = 1 .. T
-//   word    a_0 + 65536 * steps
+//   word    a_0 + 65536 * the coefficients either sum may have: the steps, or the evaluator's length where
+//           that is more (a remainder can drop to any length below T beyond the radius)
 // and status set to SEARCH. Codewords that took irregular steps can have longer evaluators;
 // they are listed for the general root search with status ODD_SOLVED and a row of 3 T / 2 + 2 words:
 //   u16     evaluator coefficients 0 .. E - 1, then a_0 .. a_T; a last word with the locator's length
@@ -2881,6 +2882,7 @@ __global__ __launch_bounds__(64) void rsi16_solve_wave_kernel(uint32_t count, ui
         return;
     }
     uint32_t steps = S.solve(D.inv_tab);
+    uint32_t terms = steps;
     bool solved = steps != 0, odd = false;
     if (steps & 1) {  // the results in R[1], A[1]
     } else {
@@ -2907,6 +2909,7 @@ __global__ __launch_bounds__(64) void rsi16_solve_wave_kernel(uint32_t count, ui
             solved = S.irregular(steps, E + 1 - steps, len, D.inv_tab);
         else
             solved = len != 0;
+        terms = max(steps, len);
     }
     int32_t a0 = S.A0[1] - RBIAS, a[CA], r[C], v[CA], d[CA];
 #pragma unroll
@@ -2984,7 +2987,7 @@ __global__ __launch_bounds__(64) void rsi16_solve_wave_kernel(uint32_t count, ui
         for (int h = 0; h < C; ++h)
             ev[C * lane + h] = (int16_t)r[h];
     if (lane == 0) {
-        row[3 * T / 2] = bal_canon(a0) | (steps << 16);
+        row[3 * T / 2] = bal_canon(a0) | (terms << 16);
         status[cw] = SEARCH;
     }
 }
@@ -3005,7 +3008,7 @@ __global__ __launch_bounds__(512) void rsi16_roots_wave_kernel(uint16_t *__restr
     constexpr uint32_t NW = 8;
     constexpr int T = E / 2, KF = 2 * T / 64, CW = 16 * CG, WORDS = T + 1;  // T / 2 words of either, odd stride
     __shared__ uint32_t s_co[CW * WORDS];
-    __shared__ uint32_t s_last[CW];        // a_0 + 65536 * steps
+    __shared__ uint32_t s_last[CW];        // a_0 + 65536 * coefficients of the sums
     __shared__ uint32_t s_found[CW];
     __shared__ uint32_t s_list[CW * T < REG_WORDS * E ? REG_WORDS * E : CW * T];
     __shared__ uint32_t s_total;
@@ -3130,7 +3133,7 @@ __global__ __launch_bounds__(512) void rsi16_roots_wave_kernel(uint16_t *__restr
         const int32_t xb = (int32_t)r.xi > 32768 ? (int32_t)r.xi - (int32_t)P16 : (int32_t)r.xi;
         const int32_t x2 = bal_mul(xb, xb);
         const uint32_t *co = s_co + r.w * WORDS;
-        // both have degree below steps; in blocks of four pairs, whose coefficients are read at once
+        // in blocks of four pairs, whose coefficients are read at once
         const int32_t pairs = (int32_t)(((s_last[r.w] >> 16) + 7) / 8) * 4;
         int32_t nb = RBIAS, db = RBIAS;
         if (__any(max(abs(xb), abs(x2)) > 32766)) {

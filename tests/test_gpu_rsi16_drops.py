@@ -1,0 +1,50 @@
+"""RSi16 repair of words whose remainders drop by more than one degree (built from their syndromes), one,
+17 and many to a launch, in every mode, against the oracle: Forney's numerator has all coefficients of an
+evaluator that is longer than the number of steps."""
+import numpy as np
+import pytest
+
+from oracle import oracle as O
+from rsi16_words import Words
+
+pytestmark = pytest.mark.gpu
+
+
+def _check(n, ecc, counts, extra=()):
+    from libffrs_amd import capi
+    k = n - ecc
+    print(f"drops ({n},{ecc})", flush=True)
+    o = O.RSi16(n, ecc)
+    base = np.array([w for _, _, w in Words(o).drops(np.random.default_rng(3 * n + ecc), extra)])
+    wm, we = np.ascontiguousarray(base[:, :k]), np.ascontiguousarray(base[:, k:])
+    wst = o.repair_batch(wm, we)
+    # the general kernels give 4 or 255 where the reference's lengths run past ecc symbols and it raises
+    keep = wst != 255
+    base, wm, we, wst = base[keep], wm[keep], we[keep], wst[keep]
+    ctx = capi.Context(0)
+    codec = capi.RSi16Codec(ctx, n, ecc)
+    top = max(counts)
+    d_m, d_p, d_s = ctx.alloc(top * k * 2), ctx.alloc(top * ecc * 2), ctx.alloc(top)
+    for count in counts:
+        for first in range(0, len(base), count):
+            idx = (first + np.arange(count)) % len(base)
+            for mode in (0, 1, 2):
+                codec.set_repair_syndromes(mode)
+                d_m.upload(np.ascontiguousarray(base[idx, :k]))
+                d_p.upload(np.ascontiguousarray(base[idx, k:]))
+                codec.repair_device(d_m, d_p, count, d_s)
+                m, e, st = np.empty((count, k), np.uint16), np.empty((count, ecc), np.uint16), np.empty(count, np.uint8)
+                d_m.download(m)
+                d_p.download(e)
+                d_s.download(st)
+                bad = np.nonzero((st != wst[idx]) | (m != wm[idx]).any(1) | (e != we[idx]).any(1))[0]
+                assert bad.size == 0, (count, mode, idx[bad[:8]], st[bad[:8]], wst[idx[bad[:8]]])
+    for b in (d_m, d_p, d_s):
+        b.free()
+    codec.close()
+    ctx.close()
+
+
+@pytest.mark.parametrize("n,ecc,counts", [(128, 64, (1, 17, 3000)), (384, 128, (1, 17, 20000)), (512, 256, (1, 17, 1100))])
+def test_evaluator_longer_than_the_steps(n, ecc, counts):
+    _check(n, ecc, counts)
