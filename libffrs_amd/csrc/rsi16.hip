@@ -2229,10 +2229,10 @@ __global__ __launch_bounds__(NW * 64) void rsi16_contract_kernel(const uint16_t 
 // The key equation for ecc_len <= 32 with one codeword per lane. pr_sugiyama's usual step (the
 // quotient has two terms, every remainder one degree below the last) needs no data-dependent
 // index: after s steps the remainder has degree E - 1 - s and the locator degree s, so the steps
-// are unrolled with every polynomial in registers, and lanes whose remainder has dropped below
-// E / 2 keep what they hold. A codeword whose remainder drops by more than one degree and stays at
-// E / 2 or above, or that meets one of the other cases listed at lane_solve, goes to the general
-// kernel (rsi16_repair_list_kernel): about 17 in 65,537 damaged codewords.
+// are unrolled with every polynomial in registers, and lanes whose remainder has fewer than E / 2
+// coefficients keep what they hold. A codeword whose remainder drops by more than one degree and still
+// has E / 2 or more, or that meets one of the other cases listed at check() and solve(), goes to the
+// general kernel (rsi16_repair_list_kernel): about 17 in 65,537 damaged codewords.
 // 262,144 RSi16(256,32) repairs with 0-16 errors: 38 us of syndromes, 96 here and 24 for the 60 odd
 // ones, against 402 + 52 with a codeword per sixteen lanes. Bound by the vector units (a wave's
 // 9,000 instructions, 80 % of the issue slots): a third of them the key equation's steps, the rest
@@ -2310,7 +2310,8 @@ struct LaneSolve {
             A[y][i] = lane_update<SAFE>(A[y][i], A[x][i], i ? A[x][i - 1] : RBIAS, n0, n1, k0, k1);
     }
 
-    // After step s: stop where the remainder fell below degree E / 2.
+    // After step s: stop where the remainder dropped to fewer than E / 2 coefficients; the reference goes on
+    // dividing from E / 2 of them on.
     template <int S_>
     __device__ void check(bool &active)
     {
@@ -2321,7 +2322,7 @@ struct LaneSolve {
         } else if (active && R[y][E - 1 - S_] == RBIAS) {
             uint32_t high = 0, low = 0;
 #pragma unroll
-            for (int i = T; i < E - 1 - S_; ++i)
+            for (int i = T - 1; i < E - 1 - S_; ++i)
                 high |= (uint32_t)(R[y][i] ^ RBIAS);
 #pragma unroll
             for (int i = 0; i < T; ++i)

@@ -1,6 +1,7 @@
 """RSi16 repair of words whose remainders drop by more than one degree (built from their syndromes), one,
-17 and many to a launch, in every mode, against the oracle: Forney's numerator has all coefficients of an
-evaluator that is longer than the number of steps."""
+17 and many to a launch, in every mode, against the oracle: the regular steps must not finish a word whose
+remainder is exactly ecc / 2 long, and Forney's numerator has all coefficients of an evaluator that is longer
+than the number of steps."""
 import numpy as np
 import pytest
 
@@ -48,3 +49,38 @@ def _check(n, ecc, counts, extra=()):
 @pytest.mark.parametrize("n,ecc,counts", [(128, 64, (1, 17, 3000)), (384, 128, (1, 17, 20000)), (512, 256, (1, 17, 1100))])
 def test_evaluator_longer_than_the_steps(n, ecc, counts):
     _check(n, ecc, counts)
+
+
+@pytest.mark.parametrize("n,ecc,counts", [(16, 8, (1, 70000)), (1024, 8, (17, 2000)), (64, 16, (1, 30000)),
+                                          (96, 32, (17, 20000)), (256, 32, (1, 17000))])
+def test_remainder_of_half_the_parity(n, ecc, counts):
+    _check(n, ecc, counts, extra=range(1, ecc // 2))
+
+
+def test_remainder_of_half_the_parity_found_word():
+    """A word beyond the radius of RSi16(1024,8) whose remainder is 4 long after three steps: the oracle finds
+    no location."""
+    from libffrs_amd import capi
+    n, ecc, count = 1024, 8, 2048
+    k = n - ecc
+    cw = np.zeros(n, np.uint16)
+    cw[:8] = (7139, 55613, 11942, 57933, 12862, 37347, 12777, 45739)
+    m, e = cw[:k].copy(), cw[k:].copy()
+    assert O.RSi16(n, ecc).repair(m, e) == 4 and np.array_equal(np.r_[m, e], cw)
+    ctx = capi.Context(0)
+    codec = capi.RSi16Codec(ctx, n, ecc)
+    d_m, d_p, d_s = ctx.alloc(count * k * 2), ctx.alloc(count * ecc * 2), ctx.alloc(count)
+    for mode in (0, 1, 2):
+        codec.set_repair_syndromes(mode)
+        d_m.upload(np.tile(cw[:k], (count, 1)))
+        d_p.upload(np.tile(cw[k:], (count, 1)))
+        codec.repair_device(d_m, d_p, count, d_s)
+        m, e, st = np.empty((count, k), np.uint16), np.empty((count, ecc), np.uint16), np.empty(count, np.uint8)
+        d_m.download(m)
+        d_p.download(e)
+        d_s.download(st)
+        assert (st == 4).all() and (m == cw[:k]).all() and (e == cw[k:]).all(), mode
+    for b in (d_m, d_p, d_s):
+        b.free()
+    codec.close()
+    ctx.close()
