@@ -166,7 +166,10 @@ int ffrs_rsi16_set_encode_kernel(ffrs_rsi16 *rs, int kernel);
  * depend on it): 0 automatic, 1 inside the general repair kernel, 2 as an int8 MFMA contraction of
  * the codewords with the matrix w^(j rbo(m)) ahead of it, where its tables exist (ecc_len 8 or a
  * multiple of 16 up to 256, message_len <= 16384, 16-byte aligned buffers); for ecc_len 8 to 32 that
- * is followed by the one-codeword-per-lane kernel. Automatic picks by ecc_len and count. */
+ * is followed by the one-codeword-per-lane kernel. Automatic picks by ecc_len and count. The
+ * syndromes take 4 (ecc_len + 1) bytes a codeword of device memory, at most 256 MiB (larger batches go in
+ * pieces), kept by the codec; where they can't be had, or a capture runs before they are large enough,
+ * the general kernel takes the batch. Threads may call the repair of one codec at the same time. */
 int ffrs_rsi16_set_repair_syndromes(ffrs_rsi16 *rs, int mode);
 uint32_t ffrs_rsi16_root(const ffrs_rsi16 *rs);
 size_t ffrs_rsi16_ntt_len(const ffrs_rsi16 *rs);

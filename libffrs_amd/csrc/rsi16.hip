@@ -4156,8 +4156,10 @@ struct ffrs_rsi16 {
     int32_t *d_rows_enc = nullptr, *d_rows_syn = nullptr;  // balanced rows of the same maps (ecc_len 2 to 8)
     bool mix_minus_one = false;      // a mix constant is 65536: the SIMD words are not the linear map
     int encode_mode = 0;             // 0 automatic, 1 butterflies, 2 MFMA wherever it applies
-    uint32_t *d_syn = nullptr;       // syndromes of the last repair launch
+    uint32_t *d_syn = nullptr;       // syndromes and list of a repair's launches
     size_t syn_size = 0;
+    std::vector<void *> syn_old;     // outgrown ones: a captured graph may still write there
+    std::mutex syn_mu;               // held while the launches that share the workspace are queued
     int repair_synd = 0;             // 0 automatic, 1 in the repair kernel, 2 MFMA ahead of it
 };
 
@@ -4338,6 +4340,33 @@ int launch_encode(ffrs_rsi16 *rs, const uint16_t *d_msg, size_t count, uint16_t 
     return FFRS_OK;
 }
 
+// Syndromes a repair launch may keep on the device: larger batches go in pieces of this many bytes
+// (261,000 codewords of ecc_len 256, 2,000,000 of 32).
+constexpr size_t SYN_BYTES = (size_t)256 << 20;
+
+// A workspace of `need` bytes (at most SYN_BYTES + 4), or nullptr where it is not there and can't be had: no
+// memory, or the stream is being captured. It grows to twice its size, so that the outgrown ones, kept until
+// the codec is destroyed, never hold more than the last. The caller holds syn_mu.
+uint32_t *syn_workspace(ffrs_rsi16 *rs, size_t need)
+{
+    if (rs->syn_size >= need)
+        return rs->d_syn;
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(rs->ctx->stream, &st) != hipSuccess || st != hipStreamCaptureStatusNone)
+        return nullptr;
+    const size_t size = std::max(need, std::min(2 * rs->syn_size, SYN_BYTES + 4));
+    uint32_t *d = nullptr;
+    if (hipMalloc(&d, size) != hipSuccess) {
+        (void)hipGetLastError();  // not the next launch's error
+        return nullptr;
+    }
+    if (rs->d_syn)
+        rs->syn_old.push_back(rs->d_syn);
+    rs->d_syn = d;
+    rs->syn_size = size;
+    return d;
+}
+
 template <int E>
 int launch_repair_reg(ffrs_rsi16 *rs, uint16_t *d_msg, uint16_t *d_ecc, size_t count, uint8_t *d_status)
 {
@@ -4375,21 +4404,18 @@ int launch_repair_reg(ffrs_rsi16 *rs, uint16_t *d_msg, uint16_t *d_ecc, size_t c
     const bool single = E == 128 && rs->repair_synd == 0 && count <= 16;
     const bool msyn = rs->synd.dev.nq && rs->repair_synd != 1 && ((E >= 64 && !single) || lanes || given) &&
                       (((uintptr_t)d_msg | (uintptr_t)d_ecc) & 15) == 0;
+    // workspace: E syndromes per codeword and the list of those left to the general kernel, which takes the
+    // whole batch where there is no workspace
+    const size_t step = std::min(contract_step_count(rs), (SYN_BYTES / (4 * (E + 1))) & ~(size_t)63);
+    const size_t chunk = std::min(count, step);
+    std::unique_lock<std::mutex> lk(rs->syn_mu, std::defer_lock);
+    uint32_t *syn = nullptr;
     if (msyn) {
-        // workspace: E syndromes per codeword and the list of those left to the general kernel
-        const size_t step = contract_step_count(rs), chunk = std::min(count, step);
-        const size_t need = chunk * E * 4 + (chunk + 1) * 4;
-        if (rs->syn_size < need) {
-            if (rs->d_syn)
-                FFRS_HIP(hipFree(rs->d_syn));
-            rs->d_syn = nullptr;
-            rs->syn_size = 0;
-            hipError_t e = hipMalloc(&rs->d_syn, need);
-            if (e != hipSuccess)
-                return fail(FFRS_ERR_NOMEM, "syndrome workspace of %zu bytes: %s", need, hipGetErrorString(e));
-            rs->syn_size = need;
-        }
-        uint32_t *syn = rs->d_syn, *list = syn + chunk * E;
+        lk.lock();
+        syn = syn_workspace(rs, chunk * E * 4 + (chunk + 1) * 4);
+    }
+    if (syn) {
+        uint32_t *list = syn + chunk * E;
         for (size_t b = 0; b < count; b += step) {
             const size_t c = std::min(step, count - b);
             uint16_t *m = d_msg + b * rs->k, *e = d_ecc + b * E;
@@ -4860,6 +4886,8 @@ void ffrs_rsi16_destroy(ffrs_rsi16 *rs)
             (void)hipFree(d);
     if (rs->d_syn)
         (void)hipFree(rs->d_syn);
+    for (void *d : rs->syn_old)
+        (void)hipFree(d);
     delete rs;
 }
 
