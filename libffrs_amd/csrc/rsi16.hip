@@ -3891,9 +3891,9 @@ __global__ __launch_bounds__(64) void circ16_outer_known_kernel(const Rsi16Dev T
 constexpr uint32_t KNOWN_E = 256;
 
 // W of interleave block blockIdx.y, rows blockIdx.x * 256 + thread: balanced words at
-// (kk n + m) E + i, i < cnt[kk].
+// (kk n + m) stride + i, i < cnt[kk] <= stride.
 __global__ __launch_bounds__(256) void circ16_known_map_kernel(const Rsi16Dev T, const uint32_t *__restrict__ pos,
-                                                               const uint32_t *__restrict__ cnt,
+                                                               const uint32_t *__restrict__ cnt, uint32_t stride,
                                                                int32_t *__restrict__ W)
 {
     __shared__ uint32_t s_x[KNOWN_E], s_y[KNOWN_E], s_b[KNOWN_E];
@@ -3921,7 +3921,7 @@ __global__ __launch_bounds__(256) void circ16_known_map_kernel(const Rsi16Dev T,
     uint32_t a = s_pow(X, E);
     for (uint32_t j = 0; j < r; ++j)
         a = F::mul(a, F::sub(1, F::mul(s_x[j], Xi)));
-    int32_t *w = W + ((size_t)kk * T.n + m) * E;
+    int32_t *w = W + ((size_t)kk * T.n + m) * stride;
     for (uint32_t i = 0; i < r; ++i) {
         const uint32_t den = F::sub(F::mul(X, s_y[i]), 1);
         const uint32_t v = den ? F::mul(F::mul(a, s_b[i]), T.inv_tab[den]) : P16 - 1;
@@ -3929,13 +3929,14 @@ __global__ __launch_bounds__(256) void circ16_known_map_kernel(const Rsi16Dev T,
     }
 }
 
-// The corrections of 64 columns (of one interleave block: col0 counts within block blockIdx.y) per
-// workgroup of 16 waves: each wave sums every 16th symbol, KNOWN_I error rows at a time.
+// The corrections of 64 columns of interleave block blockIdx.y (msg and rso32 at the first block's) per
+// workgroup of 16 waves: each wave sums every 16th symbol, KNOWN_I error rows at a time (stride is a
+// multiple of KNOWN_I).
 constexpr int KNOWN_I = 8;
 __global__ __launch_bounds__(1024) void circ16_known_apply_kernel(const Rsi16Dev T, uint16_t *__restrict__ msg,
                                                                   uint32_t *__restrict__ rso32, uint32_t il,
                                                                   uint32_t ik, const uint32_t *__restrict__ pos,
-                                                                  const uint32_t *__restrict__ cnt,
+                                                                  const uint32_t *__restrict__ cnt, uint32_t stride,
                                                                   const int32_t *__restrict__ W)
 {
     __shared__ int32_t s_part[16][KNOWN_I][64];
@@ -3952,10 +3953,10 @@ __global__ __launch_bounds__(1024) void circ16_known_apply_kernel(const Rsi16Dev
         for (uint32_t m = wave; m < n; m += 16) {
             int32_t c = m < k ? (int32_t)msg[(size_t)m * il + col] : (int32_t)rso32[(size_t)(m - k) * il + col];
             c = c > 32768 ? c - (int32_t)P16 : c;
-            const int32_t *w = W + ((size_t)kk * n + m) * E + i0;
+            const int32_t *w = W + ((size_t)kk * n + m) * stride + i0;
 #pragma unroll
             for (int u = 0; u < KNOWN_I; ++u)  // past r: words of the row that no error uses
-                acc[u] += fold16(c * (i0 + u < E ? w[u] : 0));
+                acc[u] += fold16(c * w[u]);
         }
 #pragma unroll
         for (int u = 0; u < KNOWN_I; ++u)
@@ -5698,6 +5699,8 @@ struct ffrs_circ16 {
     size_t msg_len = 0, rso_len = 0, rsi_len = 0, rsio_len = 0, ecc_len = 0;
     void *d_buf = nullptr;
     size_t buf_size = 0;
+    int32_t *d_map = nullptr;                  // the known-position repair's matrices
+    size_t map_size = 0;
 };
 
 namespace {
@@ -5769,7 +5772,6 @@ struct CircWs {
     uint16_t *msg, *ecc;
     uint32_t *rso32, *rsi32, *syn, *pos, *cnt;
     uint8_t *flag, *gst;
-    int32_t *map;  // outer ecc_len <= KNOWN_E: the known-position repair's matrix per interleave block
     uint32_t *work;
     size_t work_lanes;
 };
@@ -5796,10 +5798,81 @@ size_t circ_repair_layout(const ffrs_circ16 *c, CircWs *w, char *base)
     w->pos = (uint32_t *)take((size_t)c->I * c->oE * 4);
     w->cnt = (uint32_t *)take((size_t)c->I * 4);
     w->gst = (uint8_t *)take(ngr);
-    w->map = (int32_t *)take(c->oE <= KNOWN_E ? (size_t)c->I * c->on * c->oE * 4 : 0);
     w->work = (uint32_t *)take(lanes * wrows * 4);
     w->work_lanes = lanes;
     return o;
+}
+
+// Device memory for the matrices of the known-position repair: more interleave blocks go in turns.
+constexpr size_t MAP_BYTES = (size_t)256 << 20;
+
+// The repair of interleave blocks at known rows (w.pos, w.cnt; cnt: the host's copy), as a matrix per block
+// or, where that takes longer or has no memory, column by column. Of both the times were measured over inner
+// message_len 8 to 2048, 1 to 8,191 blocks and outer codes from (16,8) to (4096,256) and fitted (us, n and E
+// of the outer code, r rows, C columns): 8 + the larger of 0.03 n ceil(r / 8) and 0.036 n (sum of ceil(r / 8)
+// over the workgroups / CUs) + 1.2e-5 n r a block, against the larger of 10 + 0.031 n + 0.18 E + 0.065 r^2 and
+// C (0.0015 + 7e-6 n + 4e-5 E + 3.9e-5 r^2). Matrix / columns: (512,256), 1,024 columns a block, 16 blocks:
+// one row 26 / 346, 64 rows
+// 171 / 2,827; (4096,64), one block of 64 columns: 1 row 124 / 137, 64 rows 905 / 404; (1024,64), 8,191 blocks of
+// 8 columns: one row 1,744 / 659.
+int circ_repair_known(ffrs_circ16 *c, const CircWs &w, const std::vector<uint32_t> &cnt)
+{
+    hipStream_t st = c->ri->ctx->stream;
+    const uint32_t wgs = (c->ik + 63) / 64;
+    const double n = c->on, E = c->oE;
+    double rounds = 0, deepest = 0, rows = 0, columns = 0, longest = 0;
+    uint32_t most = 0;
+    for (uint32_t r : cnt) {
+        if (r == 0)
+            continue;
+        most = std::max(most, r);
+        rounds += (double)wgs * ((r + 7) / 8);
+        deepest = std::max(deepest, (double)((r + 7) / 8));
+        rows += r;
+        columns += c->ik * (0.0015 + 7e-6 * n + 4e-5 * E + 3.9e-5 * r * r);
+        longest = std::max(longest, 10 + 0.031 * n + 0.18 * E + 0.065 * r * r);
+    }
+    const double map_us = 8 + n * std::max(0.03 * deepest, 0.036 * rounds / c->ri->ctx->cu_count) + 1.2e-5 * n * rows;
+    const uint32_t stride = (most + KNOWN_I - 1) / KNOWN_I * KNOWN_I;
+    const size_t block = (size_t)c->on * stride * 4;  // at most 64 MiB
+    const uint32_t turn = c->oE <= KNOWN_E ? (uint32_t)std::min<size_t>(c->I, MAP_BYTES / block) : 0;
+    bool map = turn != 0 && map_us < std::max(columns, longest);
+    if (map && c->map_size < turn * block) {
+        if (c->d_map)
+            FFRS_HIP(hipFree(c->d_map));
+        c->d_map = nullptr;
+        c->map_size = 0;
+        if (hipMalloc(&c->d_map, turn * block) == hipSuccess) {
+            c->map_size = turn * block;
+        } else {
+            (void)hipGetLastError();  // not the next launch's error
+            c->d_map = nullptr;
+            map = false;
+        }
+    }
+    if (!map) {
+        const size_t lds = (size_t)7 * c->oE * 4;
+        if (int r = allow_lds(circ16_outer_known_kernel, lds))
+            return r;
+        hipLaunchKernelGGL(circ16_outer_known_kernel, dim3(c->rI), dim3(64), lds, st, c->ro->dev, w.msg, w.rso32, c->rI,
+                           c->ik, (const uint32_t *)w.pos, (const uint32_t *)w.cnt);
+        FFRS_HIP(hipGetLastError());
+        return FFRS_OK;
+    }
+    for (uint32_t b = 0; b < c->I; b += turn) {
+        const uint32_t nb = std::min(turn, c->I - b);
+        if (std::all_of(cnt.begin() + b, cnt.begin() + b + nb, [](uint32_t v) { return v == 0; }))
+            continue;
+        const uint32_t *pos = w.pos + (size_t)b * c->oE, *num = w.cnt + b;
+        hipLaunchKernelGGL(circ16_known_map_kernel, dim3((c->on + 255) / 256, nb), dim3(256), 0, st, c->ro->dev, pos, num,
+                           stride, c->d_map);
+        FFRS_HIP(hipGetLastError());
+        hipLaunchKernelGGL(circ16_known_apply_kernel, dim3(wgs, nb), dim3(1024), 0, st, c->ro->dev,
+                           w.msg + (size_t)b * c->ik, w.rso32 + (size_t)b * c->ik, c->rI, c->ik, pos, num, stride,
+                           (const int32_t *)c->d_map);
+        FFRS_HIP(hipGetLastError());
+    }
+    return FFRS_OK;
 }
 
 // load_ecc, compute_rsi_synd, repair_outer_zeros, repair_inner_zeros and the row flags of
@@ -5902,10 +5975,11 @@ void ffrs_circ16_destroy(ffrs_circ16 *c)
 {
     if (!c)
         return;
-    if (c->d_buf) {
-        (void)hipSetDevice(c->ri->ctx->device);
+    (void)hipSetDevice(c->ri->ctx->device);
+    if (c->d_buf)
         (void)hipFree(c->d_buf);
-    }
+    if (c->d_map)
+        (void)hipFree(c->d_map);
     delete c;
 }
 
@@ -6023,22 +6097,8 @@ int ffrs_circ16_repair(ffrs_circ16 *c, uint16_t *msg, uint16_t *ecc, int *raised
     if (std::any_of(cnt.begin(), cnt.end(), [](uint32_t v) { return v != 0; })) {
         FFRS_HIP(hipMemcpyAsync(w.pos, pos.data(), pos.size() * 4, hipMemcpyHostToDevice, st));
         FFRS_HIP(hipMemcpyAsync(w.cnt, cnt.data(), cnt.size() * 4, hipMemcpyHostToDevice, st));
-        if (c->oE <= KNOWN_E) {
-            hipLaunchKernelGGL(circ16_known_map_kernel, dim3((c->on + 255) / 256, c->I), dim3(256), 0, st, c->ro->dev,
-                               (const uint32_t *)w.pos, (const uint32_t *)w.cnt, w.map);
-            FFRS_HIP(hipGetLastError());
-            hipLaunchKernelGGL(circ16_known_apply_kernel, dim3((c->ik + 63) / 64, c->I), dim3(1024), 0, st, c->ro->dev,
-                               w.msg, w.rso32, c->rI, c->ik, (const uint32_t *)w.pos, (const uint32_t *)w.cnt,
-                               (const int32_t *)w.map);
-            FFRS_HIP(hipGetLastError());
-        } else {
-            const size_t lds = (size_t)7 * c->oE * 4;
-            if (int r = allow_lds(circ16_outer_known_kernel, lds))
-                return r;
-            hipLaunchKernelGGL(circ16_outer_known_kernel, dim3(c->rI), dim3(64), lds, st, c->ro->dev, w.msg, w.rso32,
-                               c->rI, c->ik, (const uint32_t *)w.pos, (const uint32_t *)w.cnt);
-            FFRS_HIP(hipGetLastError());
-        }
+        if (int r = circ_repair_known(c, w, cnt))
+            return r;
     }
     // without positions: the reference's SIMD groups of W columns from the block's first column
     // (pyrsi16.hpp:391-456), in block order; a group that raises stops the repair there
