@@ -3634,8 +3634,8 @@ __global__ __launch_bounds__(256) void rsi16_simd_writeback_kernel(const Rsi16De
 
 // For ecc_len 2, 4 and 8 the syndromes and (with the conditions of the contraction, above) the parity
 // are a few sums over a long row: a wave takes a codeword, each lane every 64th symbol, with the map's
-// matrix as balanced words (row m: E of them). Where there are few codewords (a CIRC16 file has
-// hundreds to thousands of inner rows) a lane group or lane per codeword leaves the chip idle:
+// matrix as balanced words (row m: E of them). Where there are few codewords for their length (a CIRC16 file
+// has hundreds to thousands of inner rows; rows_pay) a lane group or lane per codeword leaves the chip idle:
 // 1,024 rows of RSi16(2052,4) took 475 us (syndromes 516) with two lanes each, 6 here.
 template <int E, class TM>
 __device__ inline void row_accumulate(const TM *__restrict__ m, uint32_t count, const int32_t *__restrict__ tab,
@@ -5722,6 +5722,21 @@ int circ_reserve(ffrs_circ16 *c, size_t bytes)
 
 size_t al256(size_t x) { return (x + 255) & ~(size_t)255; }
 
+// Whether rsi16_rows_kernel's wave a row is faster than the lane groups or lanes a row of the others, for
+// ecc_len 2, 4, 8: it costs 0.2, 0.3, 0.55 ns a row whatever the length up to 256 symbols, and the others wait
+// for about 0.8 us a chunk of ecc_len symbols but then fit 64, 32, 16 codewords in a wave. per: rows per message
+// symbol up to which the wave a row measured faster (us, rows / others: syndromes of (10,2) 16,384 rows 6 / 8,
+// 131,072 32 / 8; (66,2) 131,072 34 / 45; (20,4) 4,096 5 / 9, 16,384 10 / 8; (24,8) 2,048 5 / 9, 16,384 13 / 7;
+// parity of the message rows of (18,2) 4,096 3 / 5, 16,384 9 / 7; of the outer parity rows 32,768 7 / 8).
+struct RowsPer {
+    uint32_t e2, e4, e8;
+};
+constexpr RowsPer ROWS_SYND{2000, 800, 280}, ROWS_ENC16{600, 300, 0}, ROWS_ENC32{3000, 900, 180};
+bool rows_pay(const ffrs_rsi16 *rs, const int32_t *tab, size_t rows, const RowsPer &per)
+{
+    return tab && rows <= (size_t)rs->k * (rs->E == 2 ? per.e2 : rs->E == 4 ? per.e4 : per.e8);
+}
+
 // rsi16_rows_kernel on `rows` codewords: syndromes where e is given, else the parity.
 template <class TM, class TO>
 int launch_rows(ffrs_rsi16 *rs, const TM *m, const uint32_t *e, size_t rows, TO *out)
@@ -5735,14 +5750,14 @@ int launch_rows(ffrs_rsi16 *rs, const TM *m, const uint32_t *e, size_t rows, TO 
     return FFRS_OK;
 }
 
-// The generic lane-group encode of `count` codewords (interleave stride I), u16 or u32 symbols in
-// and out, in the SIMD or scalar words.
+// The encode of `count` codewords (interleave stride I), u16 or u32 symbols in and out, in the SIMD or scalar
+// words.
 template <class TI, class TO>
 int circ_encode(ffrs_rsi16 *rs, const TI *d_in, size_t count, TO *d_out, bool vec, uint32_t I)
 {
     if (count == 0)
         return FFRS_OK;
-    if (I == 1 && rs->d_rows_enc && !(vec && rs->mix_minus_one))
+    if (I == 1 && rows_pay(rs, rs->d_rows_enc, count, ROWS_ENC32) && !(vec && rs->mix_minus_one))
         return launch_rows<TI, TO>(rs, d_in, nullptr, count, d_out);
     const uint32_t g = rs->g_enc == 1 && rs->E <= 32 ? group_size(rs->E) : rs->g_enc, cpw = 64 / g;
     const size_t lds = (size_t)cpw * 2 * rs->E * 4;
@@ -5761,7 +5776,7 @@ int circ_encode(ffrs_rsi16 *rs, const TI *d_in, size_t count, TO *d_out, bool ve
 int circ_encode_rows(ffrs_circ16 *c, const uint16_t *d_msg, size_t rows, uint16_t *d_rsi)
 {
     ffrs_rsi16 *rs = c->ri;
-    if (rs->d_rows_enc && rs->E <= 4 && !(c->W > 1 && rs->mix_minus_one))
+    if (rows_pay(rs, rs->d_rows_enc, rows, ROWS_ENC16) && !(c->W > 1 && rs->mix_minus_one))
         return launch_rows<uint16_t, uint16_t>(rs, d_msg, nullptr, rows, d_rsi);
     return launch_encode(rs, d_msg, rows, d_rsi, c->W > 1 ? 1 : 0);
 }
@@ -5886,25 +5901,23 @@ int circ_prepare(ffrs_circ16 *c, const CircWs &w)
                        (uint32_t)c->rso_len, w.rsi32, (uint32_t)rsi_all);
     FFRS_HIP(hipGetLastError());
     uint32_t *esyn = w.syn + (size_t)mrows * iE, *ersi = w.rsi32 + (size_t)mrows * iE;
-    if (c->ri->d_rows_syn) {
-        if (int r = launch_rows<uint16_t, uint32_t>(c->ri, w.msg, w.rsi32, mrows, w.syn))
-            return r;
-        if (int r = launch_rows<uint32_t, uint32_t>(c->ri, w.rso32, ersi, erows, esyn))
-            return r;
-    } else {
+    auto synd = [&](const auto *m, const uint32_t *e, uint32_t q, uint32_t *out) -> int {
+        using TM = std::decay_t<decltype(*m)>;
+        if (rows_pay(c->ri, c->ri->d_rows_syn, q, ROWS_SYND))
+            return launch_rows<TM, uint32_t>(c->ri, m, e, q, out);
         const uint32_t g = group_size(iE), cpw = 64 / g;
         const size_t lds = (size_t)cpw * 2 * iE * 4;
-        if (int r = allow_lds(circ16_synd_kernel<uint16_t>, lds))
+        if (int r = allow_lds(circ16_synd_kernel<TM>, lds))
             return r;
-        if (int r = allow_lds(circ16_synd_kernel<uint32_t>, lds))
-            return r;
-        hipLaunchKernelGGL(circ16_synd_kernel<uint16_t>, dim3((mrows + cpw - 1) / cpw), dim3(64), lds, st, c->ri->dev,
-                           (const uint16_t *)w.msg, (const uint32_t *)w.rsi32, mrows, w.syn, g);
+        hipLaunchKernelGGL(circ16_synd_kernel<TM>, dim3((q + cpw - 1) / cpw), dim3(64), lds, st, c->ri->dev, m, e, q, out,
+                           g);
         FFRS_HIP(hipGetLastError());
-        hipLaunchKernelGGL(circ16_synd_kernel<uint32_t>, dim3((erows + cpw - 1) / cpw), dim3(64), lds, st, c->ri->dev,
-                           (const uint32_t *)w.rso32, (const uint32_t *)ersi, erows, esyn, g);
-        FFRS_HIP(hipGetLastError());
-    }
+        return FFRS_OK;
+    };
+    if (int r = synd((const uint16_t *)w.msg, w.rsi32, mrows, w.syn))
+        return r;
+    if (int r = synd((const uint32_t *)w.rso32, ersi, erows, esyn))
+        return r;
     const size_t lz = (size_t)9 * iE * 4;
     auto *zk = !c->ri->d_rows_syn ? circ16_outer_zeros_kernel<0>
                : iE == 2          ? circ16_outer_zeros_kernel<2>

@@ -12,7 +12,9 @@ SHAPES = [(10, 2, 1024, 64, 2048, 16),   # column by column
           (10, 2, 512, 256, 2048, 72),   # matrices, in two turns
           (68, 4, 512, 256, 64, 9),      # matrices of 16 words a row
           (68, 4, 4096, 64, 1, 64),      # column by column, one block
-          (2052, 4, 512, 256, 4, 255)]   # matrices
+          (2052, 4, 512, 256, 4, 255),   # matrices
+          (20, 4, 64, 32, 1024, 9),      # 32,768 short inner rows: lane groups, not a wave a row
+          (16, 8, 64, 32, 2048, 9)]
 
 
 def _case(L, shape, rng):
