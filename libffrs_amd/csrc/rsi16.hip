@@ -4154,7 +4154,7 @@ struct ffrs_rsi16 {
         void *d = nullptr;
         RootTab dev{};
     } roots;                         // the locator's values at the n positions
-    int32_t *d_rows_enc = nullptr, *d_rows_syn = nullptr;  // balanced rows of the same maps (ecc_len 2 to 8)
+    int32_t *d_rows_enc = nullptr, *d_rows_syn = nullptr;  // balanced rows of the same maps (inner codecs of CIRC16)
     bool mix_minus_one = false;      // a mix constant is 65536: the SIMD words are not the linear map
     int encode_mode = 0;             // 0 automatic, 1 butterflies, 2 MFMA wherever it applies
     uint32_t *d_syn = nullptr;       // syndromes and list of a repair's launches
@@ -4508,16 +4508,61 @@ int launch_repair(ffrs_rsi16 *rs, uint16_t *d_msg, uint16_t *d_ecc, size_t count
 
 namespace {
 
-// NTT::gs_butterfly, ntt.hpp:280-302 (natural in, RBO out), scalar words
+// The tables' loops take HB rows side by side, so that they vectorise (S::mul without its branch).
+constexpr uint32_t HB = 16;
+
+inline uint32_t host_mul(uint32_t a, uint32_t b)
+{
+    const uint32_t r = a * b, d = (r & 0xffff) - (r >> 16);
+    return ((r == 0) & (a != 0) & (b != 0)) ? 1u : d + (d >> 31) * P16;
+}
+
+// NTT::gs_butterfly, ntt.hpp:280-302 (natural in, RBO out), scalar words, of HB vectors: element i of vector u
+// at HB i + u
 void gs_host(const std::vector<uint32_t> &roots, uint32_t *x, uint32_t len)
 {
     for (uint32_t st = len / 2, ef = 0; st > 0; st /= 2, ++ef)
         for (uint32_t b = 0; b < len; b += 2 * st)
             for (uint32_t i = b; i < b + st; ++i) {
-                const uint32_t a = x[i], c = x[i + st];
-                x[i] = S::add(a, c);
-                x[i + st] = i == b ? S::sub(a, c) : S::mul(S::sub(a, c), roots[(i - b) << ef]);
+                const uint32_t w = i == b ? 1u : roots[(i - b) << ef];
+                uint32_t *p = x + (size_t)i * HB, *q = p + (size_t)st * HB;
+                for (uint32_t u = 0; u < HB; ++u) {
+                    const uint32_t a = p[u], c = q[u];
+                    p[u] = S::add(a, c);
+                    q[u] = host_mul(S::sub(a, c), w);
+                }
             }
+}
+
+// The powers X_m^i, i < E, X_m = w^rbo(m), of rows m < `rows` into dst(m); with mix those of mix_i X_m^i
+// through the GS butterfly.
+template <class Dst>
+void power_rows(const ffrs_rsi16 *rs, uint32_t rows, const std::vector<uint32_t> &roots_ntt,
+                const std::vector<uint32_t> *mix, const std::vector<uint32_t> *roots_i_ecc, Dst dst)
+{
+    const uint32_t E = rs->E;
+    std::vector<uint32_t> buf((size_t)E * HB);
+    for (uint32_t m0 = 0; m0 < rows; m0 += HB) {
+        uint32_t x[HB], pw[HB];
+        for (uint32_t u = 0; u < HB; ++u) {
+            x[u] = roots_ntt[rbo_bits(std::min(m0 + u, rows - 1), rs->nbits)];
+            pw[u] = 1;
+        }
+        for (uint32_t i = 0; i < E; ++i) {
+            const uint32_t f = mix ? (*mix)[i] : 1;
+            for (uint32_t u = 0; u < HB; ++u) {
+                buf[(size_t)i * HB + u] = host_mul(f, pw[u]);
+                pw[u] = host_mul(pw[u], x[u]);
+            }
+        }
+        if (mix)
+            gs_host(*roots_i_ecc, buf.data(), E);
+        for (uint32_t u = 0; u < HB && m0 + u < rows; ++u) {
+            uint32_t *row = dst(m0 + u);
+            for (uint32_t i = 0; i < E; ++i)
+                row[i] = buf[(size_t)i * HB + u];
+        }
+    }
 }
 
 // Uploads a contraction's tables: `mat` holds its nq * 64 rows of E canonical entries (zero rows
@@ -4527,33 +4572,51 @@ int build_contract(ContractTab *tab, const std::vector<uint32_t> &mat, uint32_t 
     const uint32_t T = (E + 15) / 16, rows = nq * 64;
     std::vector<uint8_t> pack((size_t)T * nq * 2 * 64 * 16);
     std::vector<int32_t> row((size_t)T * 16 * 2);
-    std::vector<uint8_t> seen(P16);
+    // per column the first power of 3 that moves no entry onto 32640 and whose inverse is not +-32768: passes over
+    // the matrix with the entry that each column must not hold, until all columns are settled (one pass for 1,
+    // which suits 4 of 5 columns of 16,384 rows; a table of the values per column took 90 ms there)
+    std::vector<uint32_t> scale(E, 1), sinv(E, 1), want(E, 32640), bad(E);
     const uint32_t third = s_pow(3, 65535);
-    for (uint32_t j = 0; j < E; ++j) {
-        std::fill(seen.begin(), seen.end(), 0);
+    for (uint32_t tries = 0, open = E; open; ++tries) {
+        if (tries == 65536)
+            return FFRS_OK;  // no such scale: the butterflies stay
+        std::fill(bad.begin(), bad.end(), 0);
         for (uint32_t m = 0; m < rows; ++m)
-            seen[mat[(size_t)m * E + j]] = 1;
-        // the first power of 3 that moves no entry onto 32640 and whose inverse is not +-32768
-        uint32_t s = 1, si = 1, tries = 0;
-        while (seen[S::mul(32640, si)] || si == 32768 || si == P16 - 32768) {
-            if (++tries == 65536)
-                return FFRS_OK;  // no such scale: the butterflies stay
-            s = S::mul(s, 3);
-            si = S::mul(si, third);
+            for (uint32_t j = 0; j < E; ++j)
+                bad[j] |= mat[(size_t)m * E + j] == want[j];
+        for (uint32_t j = 0; j < E; ++j) {
+            if (want[j] == ~0u)
+                continue;
+            if (bad[j] || sinv[j] == 32768 || sinv[j] == P16 - 32768) {
+                scale[j] = S::mul(scale[j], 3);
+                sinv[j] = S::mul(sinv[j], third);
+                want[j] = S::mul(32640, sinv[j]);
+            } else {
+                want[j] = ~0u;
+                --open;
+            }
         }
-        uint64_t K = 0;
-        for (uint32_t m = 0; m < rows; ++m) {
-            const uint32_t g = S::mul(s, mat[(size_t)m * E + j]);
-            const int32_t v = g > 32639 ? (int32_t)g - (int32_t)P16 : (int32_t)g;
-            const int32_t lo = ((v + 128) & 255) - 128, hi = (v - lo) >> 8;
-            K += (uint64_t)((int64_t)g * 32896 + hi + (int64_t)P16);
-            const uint32_t q = m / 64, lane = j % 16 + 16 * (m % 64 / 16), bt = m % 16;
-            uint8_t *p = &pack[((((size_t)(j / 16) * nq + q) * 2) * 64 + lane) * 16 + bt];
-            p[0] = (uint8_t)lo;
-            p[64 * 16] = (uint8_t)hi;
+    }
+    std::vector<uint64_t> K(E);
+    for (uint32_t m0 = 0; m0 < rows; m0 += 16)  // in blocks of 16 x 16 entries, 256 bytes of either limb
+        for (uint32_t t = 0; t < T; ++t) {
+            uint8_t *p = &pack[(((size_t)t * nq + m0 / 64) * 2 * 64 + m0 % 64) * 16];
+            const uint32_t cols = std::min<uint32_t>(16, E - 16 * t);
+            for (uint32_t bt = 0; bt < 16; ++bt) {
+                const uint32_t *src = &mat[(size_t)(m0 + bt) * E + 16 * t];
+                for (uint32_t c = 0; c < cols; ++c) {
+                    const uint32_t g = host_mul(scale[16 * t + c], src[c]);
+                    const int32_t v = g > 32639 ? (int32_t)g - (int32_t)P16 : (int32_t)g;
+                    const int32_t lo = ((v + 128) & 255) - 128, hi = (v - lo) >> 8;
+                    K[16 * t + c] += (uint64_t)((int64_t)g * 32896 + hi + (int64_t)P16);
+                    p[c * 16 + bt] = (uint8_t)lo;
+                    p[64 * 16 + c * 16 + bt] = (uint8_t)hi;
+                }
+            }
         }
-        row[2 * j] = (int32_t)(K % P16);
-        row[2 * j + 1] = si > 32768 ? (int32_t)si - (int32_t)P16 : (int32_t)si;
+    for (uint32_t j = 0; j < E; ++j) {
+        row[2 * j] = (int32_t)(K[j] % P16);
+        row[2 * j + 1] = sinv[j] > 32768 ? (int32_t)sinv[j] - (int32_t)P16 : (int32_t)sinv[j];
     }
     char *d = nullptr;
     hipError_t e = hipMalloc(&d, pack.size() + row.size() * 4);
@@ -4575,46 +4638,44 @@ int build_contract(ContractTab *tab, const std::vector<uint32_t> &mat, uint32_t 
 void encode_matrix(const ffrs_rsi16 *rs, const std::vector<uint32_t> &mix, const std::vector<uint32_t> &roots_i_ecc,
                    const std::vector<uint32_t> &roots_ntt, std::vector<uint32_t> &mat)
 {
-    for (uint32_t m = 0; m < rs->k; ++m) {
-        const uint32_t x = roots_ntt[rbo_bits(m, rs->nbits)];
-        uint32_t *row = &mat[(size_t)m * rs->E];
-        uint32_t pw = 1;
-        for (uint32_t i = 0; i < rs->E; ++i) {
-            row[i] = S::mul(mix[i], pw);
-            pw = S::mul(pw, x);
-        }
-        gs_host(roots_i_ecc, row, rs->E);
-    }
+    power_rows(rs, rs->k, roots_ntt, &mix, &roots_i_ecc, [&](uint32_t m) { return &mat[(size_t)m * rs->E]; });
 }
 
 // The same matrix and the syndromes' w^(j rbo(m)) (NTT::pntt, ntt.hpp:133-152) as balanced words, for
-// rsi16_rows_kernel.
-int build_rows(ffrs_rsi16 *rs, const std::vector<uint32_t> &mix, const std::vector<uint32_t> &roots_i_ecc,
-               const std::vector<uint32_t> &roots_ntt)
+// rsi16_rows_kernel, from the codec's device tables; without the memory for them its callers' other kernels
+// take the rows.
+void build_rows(ffrs_rsi16 *rs)
 {
     const uint32_t E = rs->E, n = rs->n, k = rs->k;
-    if (E < 2 || E > 8 || k > 16384)
-        return FFRS_OK;
-    std::vector<uint32_t> enc((size_t)k * E), syn((size_t)n * E);
-    encode_matrix(rs, mix, roots_i_ecc, roots_ntt, enc);
-    for (uint32_t m = 0; m < n; ++m)
-        for (uint32_t j = 0, pw = 1; j < E; ++j) {
-            syn[(size_t)m * E + j] = pw;
-            pw = S::mul(pw, roots_ntt[rbo_bits(m, rs->nbits)]);
-        }
+    if (E < 2 || E > 8 || k > 16384 || rs->d_rows_enc)
+        return;
+    std::vector<uint32_t> mix(E), roots_i_ecc(E), roots_ntt(rs->N), enc((size_t)k * E), syn((size_t)n * E);
+    auto get = [](std::vector<uint32_t> &v, const uint32_t *d) {
+        return hipMemcpy(v.data(), d, v.size() * 4, hipMemcpyDeviceToHost) == hipSuccess;
+    };
+    bool ok = get(mix, rs->dev.mix) && get(roots_i_ecc, rs->dev.roots_i_ecc) && get(roots_ntt, rs->dev.roots_ntt);
+    if (ok) {
+        encode_matrix(rs, mix, roots_i_ecc, roots_ntt, enc);
+        power_rows(rs, n, roots_ntt, nullptr, nullptr, [&](uint32_t m) { return &syn[(size_t)m * E]; });
+    }
     for (auto *v : {&enc, &syn}) {
         for (uint32_t &x : *v)
             x = x > 32768 ? x - P16 : x;
         int32_t *d = nullptr;
-        hipError_t e = hipMalloc(&d, v->size() * 4);
-        if (e == hipSuccess) {
+        ok = ok && hipMalloc(&d, v->size() * 4) == hipSuccess;
+        if (ok) {
             (v == &enc ? rs->d_rows_enc : rs->d_rows_syn) = d;
-            e = hipMemcpy(d, v->data(), v->size() * 4, hipMemcpyHostToDevice);
+            ok = hipMemcpy(d, v->data(), v->size() * 4, hipMemcpyHostToDevice) == hipSuccess;
         }
-        if (e != hipSuccess)
-            return fail(FFRS_ERR_DEVICE, "row tables: %s", hipGetErrorString(e));
     }
-    return FFRS_OK;
+    if (!ok) {
+        for (int32_t **d : {&rs->d_rows_enc, &rs->d_rows_syn}) {
+            if (*d)
+                (void)hipFree(*d);
+            *d = nullptr;
+        }
+        (void)hipGetLastError();  // not the next launch's error
+    }
 }
 
 // Shapes with ecc_len below 8, above 256, or message_len above 16384 have no contraction tables.
@@ -4640,25 +4701,34 @@ int build_roots(ffrs_rsi16 *rs, const std::vector<uint32_t> &roots_ntt, bool *ok
     const uint32_t kb = T <= 16 ? 32 : 64, bl = kb / 4;       // bytes of a product, of a lane's share
     std::vector<uint8_t> pack((size_t)tiles * 16 * 2 * half, 0);
     std::vector<int32_t> row((size_t)tiles * 16, 0), pow3(T + 1);
-    auto slot = [&](uint32_t m, uint32_t kpos) -> uint8_t & {  // byte kpos of position m
-        const uint32_t f = kpos / kb, lane = m % 16 + 16 * (kpos % kb / bl);
-        return pack[(((size_t)(m / 16) * (2 * half / kb) + f) * 64 + lane) * bl + kpos % bl];
-    };
-    for (uint32_t m = 0; m < n; ++m) {
-        const uint32_t ri = rbo_bits(m, rs->nbits);
-        const uint32_t x = S::mul(roots_ntt[(rs->N - ri) & (rs->N - 1)], third);
-        uint32_t pw = 1;
+    bool missed = false;
+    for (uint32_t t = 0; t < tiles; ++t) {
+        uint32_t x[HB], pw[HB];
+        uint8_t *tile = &pack[(size_t)t * 16 * 2 * half];
+        for (uint32_t u = 0; u < 16; ++u) {
+            const uint32_t ri = rbo_bits(std::min(16 * t + u, n - 1), rs->nbits);
+            x[u] = host_mul(roots_ntt[(rs->N - ri) & (rs->N - 1)], third);
+            pw[u] = 1;
+        }
+        const uint32_t live = std::min<uint32_t>(16, n - 16 * t);
+        auto at = [&](uint32_t kpos) {  // byte kpos of the tile's first position; the next bl further on
+            return tile + ((size_t)(kpos / kb) * 64 + 16 * (kpos % kb / bl)) * bl + kpos % bl;
+        };
         for (uint32_t i = 0; i < T; ++i) {
-            pw = S::mul(pw, x);
-            if (pw == 32640)
-                return FFRS_OK;
-            const int32_t v = pw > 32639 ? (int32_t)pw - (int32_t)P16 : (int32_t)pw;
-            const int32_t lo = ((v + 128) & 255) - 128, hi = (v - lo) >> 8;
-            slot(m, i) = (uint8_t)lo;
-            slot(m, half + i) = (uint8_t)hi;
-            row[m] += hi;
+            uint8_t *pl = at(i), *ph = at(half + i);
+            for (uint32_t u = 0; u < live; ++u) {
+                pw[u] = host_mul(pw[u], x[u]);
+                missed |= pw[u] == 32640;
+                const int32_t v = pw[u] > 32639 ? (int32_t)pw[u] - (int32_t)P16 : (int32_t)pw[u];
+                const int32_t lo = ((v + 128) & 255) - 128, hi = (v - lo) >> 8;
+                pl[u * bl] = (uint8_t)lo;
+                ph[u * bl] = (uint8_t)hi;
+                row[16 * t + u] += hi;
+            }
         }
     }
+    if (missed)
+        return FFRS_OK;
     for (uint32_t i = 0, v = 1; i <= T; ++i, v = S::mul(v, 3))
         pow3[i] = v > 32768 ? (int32_t)v - (int32_t)P16 : (int32_t)v;
     const size_t at_row = pack.size(), at_pow3 = at_row + row.size() * 4;
@@ -4688,15 +4758,8 @@ int build_mfma_synd(ffrs_rsi16 *rs, const std::vector<uint32_t> &roots_ntt)
         return FFRS_OK;
     const uint32_t nqm = (k + 63) / 64, nq = nqm + (E + 63) / 64;
     std::vector<uint32_t> mat((size_t)nq * 64 * E, 0);
-    for (uint32_t m = 0; m < k + E; ++m) {
-        const uint32_t x = roots_ntt[rbo_bits(m, rs->nbits)];
-        uint32_t *row = &mat[(size_t)(m < k ? m : nqm * 64 + (m - k)) * E];
-        uint32_t pw = 1;
-        for (uint32_t j = 0; j < E; ++j) {
-            row[j] = pw;
-            pw = S::mul(pw, x);
-        }
-    }
+    power_rows(rs, k + E, roots_ntt, nullptr, nullptr,
+               [&](uint32_t m) { return &mat[(size_t)(m < k ? m : nqm * 64 + (m - k)) * E]; });
     bool ok = false;
     if (int r = build_roots(rs, roots_ntt, &ok))
         return r;
@@ -4705,11 +4768,8 @@ int build_mfma_synd(ffrs_rsi16 *rs, const std::vector<uint32_t> &roots_ntt)
     return build_contract(&rs->synd, mat, E, nq, nqm);
 }
 
-}  // namespace
-
-extern "C" {
-
-int ffrs_rsi16_create(ffrs_ctx *ctx, size_t block_len, size_t ecc_len, uint32_t primitive, ffrs_rsi16 **out)
+// The codec; contractions: with the tables of the int8 contractions and the root search, which plans do not read.
+int rsi16_create(ffrs_ctx *ctx, size_t block_len, size_t ecc_len, uint32_t primitive, bool contractions, ffrs_rsi16 **out)
 {
     if (!ctx || !out)
         return fail(FFRS_ERR_INVALID, "NULL argument");
@@ -4835,20 +4895,26 @@ int ffrs_rsi16_create(ffrs_ctx *ctx, size_t block_len, size_t ecc_len, uint32_t 
     rs->g_rep = group_size(rs->E);
     rs->g_enc = rs->E <= 32 ? 1u : group_size(rs->E);  // register kernel, one codeword per lane
     rs->mix_minus_one = std::any_of(mix.begin(), mix.end(), [](uint32_t v) { return v == 65536; });
-    if (int r = build_mfma_encode(rs, mix, roots_i_ecc, roots_ntt)) {
-        ffrs_rsi16_destroy(rs);
-        return r;
-    }
-    if (int r = build_mfma_synd(rs, roots_ntt)) {
-        ffrs_rsi16_destroy(rs);
-        return r;
-    }
-    if (int r = build_rows(rs, mix, roots_i_ecc, roots_ntt)) {
-        ffrs_rsi16_destroy(rs);
-        return r;
+    if (contractions) {
+        int r = build_mfma_encode(rs, mix, roots_i_ecc, roots_ntt);
+        if (r == FFRS_OK)
+            r = build_mfma_synd(rs, roots_ntt);
+        if (r != FFRS_OK) {
+            ffrs_rsi16_destroy(rs);
+            return r;
+        }
     }
     *out = rs;
     return FFRS_OK;
+}
+
+}  // namespace
+
+extern "C" {
+
+int ffrs_rsi16_create(ffrs_ctx *ctx, size_t block_len, size_t ecc_len, uint32_t primitive, ffrs_rsi16 **out)
+{
+    return rsi16_create(ctx, block_len, ecc_len, primitive, true, out);
 }
 
 int ffrs_rsi16_set_repair_syndromes(ffrs_rsi16 *rs, int mode)
@@ -5584,7 +5650,7 @@ int ffrs_rsi16_plan_create(ffrs_ctx *ctx, size_t count, const uint32_t *block_le
         size_t c = std::find(keys.begin(), keys.end(), key) - keys.begin();
         if (c == keys.size()) {
             ffrs_rsi16 *codec = nullptr;
-            if (int r = ffrs_rsi16_create(ctx, block_len[i], ecc_len[i], primitive, &codec)) {
+            if (int r = rsi16_create(ctx, block_len[i], ecc_len[i], primitive, false, &codec)) {
                 rsi16_plan_free(p);
                 return r;
             }
@@ -5964,6 +6030,12 @@ int ffrs_circ16_create(ffrs_rsi16 *inner, ffrs_rsi16 *outer, size_t interleave, 
     if (interleave == 0 || (size_t)inner->k * interleave > 0xffffu)
         return fail(FFRS_ERR_INVALID, "inner message_len * interleave must be in [1, 65535], got %zu",
                     (size_t)inner->k * interleave);
+    {
+        std::lock_guard<std::mutex> lk(inner->ctx->mu);
+        if (int r = ctx_set_device(inner->ctx))
+            return r;
+        build_rows(inner);
+    }
     auto *c = new ffrs_circ16;
     c->ri = inner;
     c->ro = outer;
