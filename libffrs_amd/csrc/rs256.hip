@@ -2278,10 +2278,11 @@ int launch_repair_pipeline(ffrs_rs256 *rs, uint8_t *d_msg, uint8_t *d_ecc, size_
     mark_kernel(ctx);
 
     // BM inside the Chien kernel, unrolled for the next of 2, 4, 8, 16, 24, 32. The last two hold more
-    // registers: 768 threads where that fills the CUs, 512 below (us, 512 / 768: 1 M codewords of ecc
-    // 32 421 / 381, of ecc 24 274 / 263; 131,072 of ecc 27 53 / 65); eight lanes per codeword in its passes, faster
-    // than sixteen at every ecc measured (1 M codewords of ecc 32: 402 vs 416 us; 2 M of ecc 16: 317
-    // vs 348 us; 4 M of ecc 8: 384 vs 412 us)
+    // registers: a CU takes 768 codewords in about 1.22 times the time of 512, so 768 threads where the CUs
+    // then need at most 4 rounds for 5 of 512 (us, 512 / 768: 1 M codewords of ecc 32 421 / 381, of
+    // ecc 24 274 / 263; 131,072 of ecc 27 53 / 65; 200,000 of ecc 32 143 / 164); eight lanes per codeword
+    // in its passes, faster than sixteen at every ecc measured (1 M codewords of ecc 32: 402 vs 416 us; 2 M
+    // of ecc 16: 317 vs 348 us; 4 M of ecc 8: 384 vs 412 us)
     auto fused = [&](auto kern, int wg) -> int {
         int g = persistent_grid(ctx, 1, (count + wg - 1) / wg);
         hipLaunchKernelGGL(kern, dim3(g), dim3(wg), 0, ctx->stream, d_msg, d_ecc, (uint32_t)count, k, E, d_status,
@@ -2298,7 +2299,8 @@ int launch_repair_pipeline(ffrs_rs256 *rs, uint8_t *d_msg, uint8_t *d_ecc, size_
         return fused(rs256_chien16_kernel<1024, 8>, 1024);
     if (E <= 16)
         return fused(rs256_chien16_kernel<1024, 16>, 1024);
-    const bool wide = count >= (size_t)ctx->cu_count * 768;
+    auto rounds = [&](size_t wg) { return (count + ctx->cu_count * wg - 1) / (ctx->cu_count * wg); };
+    const bool wide = 5 * rounds(768) <= 4 * rounds(512);
     if (E <= 24)
         return wide ? fused(rs256_chien16_kernel<768, 24>, 768) : fused(rs256_chien16_kernel<512, 24>, 512);
     return wide ? fused(rs256_chien16_kernel<768, 32>, 768) : fused(rs256_chien16_kernel<512, 32>, 512);
