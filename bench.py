@@ -321,19 +321,20 @@ def run_plain(name, args):
         rep_names = (["rs256_synd_kernel", "rs256_chien16_kernel"] if ecc <= 32 and N > 12288
                      else ["rs256_repair_wave_kernel"])
     else:
-        # the int8 MFMA contraction where it applies (these shapes have no mix constant of 65536), ahead of
-        # the key equation and the root search too
-        mfma = ecc in (8, 16, 32, 64, 128, 256) and k <= 16384
+        # the int8 MFMA contraction where it applies (these shapes have no mix constant of 65536; few codewords of
+        # ecc 128 and 256 keep the butterflies), ahead of the key equation and the root search too
+        mfma = ecc in (8, 16, 32, 64, 128, 256) and k <= 16384 and N > {256: 1024, 128: 16}.get(ecc, 0)
         contract = "rsi16_contract_wave_kernel" if ecc <= 32 else "rsi16_contract_kernel"
         enc_names = [contract + " (parity)" if mfma else
                      "rsi16_encode_lane_kernel" if ecc <= 32 else
                      ("rsi16_encode_reg_kernel" if ecc <= 256 else "rsi16_encode_kernel")]
         nk = len(krs[0])  # the launcher picks by count and block length
-        rep_names = ([contract + " (syndromes)", "rsi16_repair_lane_kernel", "rsi16_repair_list_kernel"]
-                     if nk == 3 and ecc <= 32 else
-                     [contract + " (syndromes)", "rsi16_solve_wave_kernel", "rsi16_roots_wave_kernel"] if nk == 3 else
-                     [contract + " (syndromes)", "rsi16_repair_reg_kernel"] if nk == 2 else
-                     ["rsi16_repair_reg_kernel" if ecc <= 256 else "rsi16_repair_kernel"])
+        one = N <= min((16 if ecc == 32 else 24 if ecc == 16 and n <= 4096 else 32) * 256, 128 * n // ecc)
+        rep_names = ([contract + " (syndromes)", "rsi16_solve_wave_kernel", "rsi16_roots_wave_kernel"] if nk == 3 else
+                     [contract + " (syndromes)", "rsi16_repair_lane_kernel" if N > 18432 else "rsi16_repair_reg_kernel"]
+                     if nk == 2 else
+                     ["rsi16_repair_one_kernel" if ecc <= 32 and one else
+                      "rsi16_repair_reg_kernel" if ecc <= 256 else "rsi16_repair_kernel"])
     ke_ms = np.mean(np.array(kes), axis=0)
     kr_ms = np.mean(np.array(krs), axis=0)
     if len(ke_ms) != len(enc_names) or len(kr_ms) != len(rep_names):

@@ -2232,9 +2232,8 @@ __global__ __launch_bounds__(NW * 64) void rsi16_contract_kernel(const uint16_t 
 // are unrolled with every polynomial in registers, and lanes whose remainder has fewer than E / 2
 // coefficients keep what they hold. A codeword whose remainder drops by more than one degree and still
 // has E / 2 or more, or that meets one of the other cases listed at check() and solve(), goes to the
-// general kernel (rsi16_repair_list_kernel): about 17 in 65,537 damaged codewords.
-// 262,144 RSi16(256,32) repairs with 0-16 errors: 38 us of syndromes, 96 here and 24 for the 60 odd
-// ones, against 402 + 52 with a codeword per sixteen lanes. Bound by the vector units (a wave's
+// general code (lane_odd): about 17 in 65,537 damaged codewords.
+// A wave of clean codewords stops after the key equation. Bound by the vector units (a wave's
 // 9,000 instructions, 80 % of the issue slots): a third of them the key equation's steps, the rest
 // the root search's epilogues, Forney and the conversions between.
 //
@@ -2408,12 +2407,29 @@ struct RootTab {
 
 constexpr uint32_t lane_repair_words(int T) { return 64u * (T + 1) + 64u * (uint32_t)(T < 8 ? 8 : T) + 64u; }
 
+// The codewords cw0 + i, i in `odd`, through the general register repair, one at a time by the whole wave: about 25
+// us each for ecc_len 32, beside the waves of other codewords (as a kernel after this one a clean batch paid its
+// launch as well: (96,32) x 30,000 12 -> 15 us).
+template <int E>
+__device__ inline void lane_odd(uint16_t *msgs, uint16_t *eccs, uint8_t *status, const Rsi16Dev &T,
+                                                   const uint32_t *syn, uint32_t *lds, size_t cw0, uint64_t odd)
+{
+    if (odd == 0)
+        return;
+    LaneR<E, true> L;
+    L.init(T, threadIdx.x);
+    for (; odd; odd &= odd - 1) {
+        const size_t cw = cw0 + (uint32_t)__builtin_ctzll(odd);
+        repair_group_reg<E, true, true>(T, msgs + cw * T.k, eccs + cw * E, lds, L, status + cw, syn + cw * E);
+        wave_sync();
+    }
+}
+
 template <int E>
 __global__ __launch_bounds__(64, 4) void rsi16_repair_lane_kernel(uint16_t *__restrict__ msgs,
                                                                   uint16_t *__restrict__ eccs, uint32_t count,
                                                                   uint8_t *__restrict__ status, Rsi16Dev D, RootTab RT,
-                                                                  const uint32_t *__restrict__ syn,
-                                                                  uint32_t *__restrict__ list)
+                                                                  const uint32_t *__restrict__ syn)
 {
     constexpr int T = E / 2, WORDS = T + 1;  // per codeword: T evaluator and T + 1 locator coefficients, u16
     __shared__ uint32_t s_co[64 * WORDS];
@@ -2434,6 +2450,12 @@ __global__ __launch_bounds__(64, 4) void rsi16_repair_lane_kernel(uint16_t *__re
             r[i] = ((S.steps & 1) ? S.R[1][i] : S.R[0][i]) - RBIAS;
         clean = S.clean;
         odd = S.odd || (!clean && a[0] == 0);
+        if (__ballot(!clean && !odd) == 0) {  // nothing to search in the wave
+            if (valid && clean)
+                status[cw] = FFRS_RSI16_NO_ERRORS;
+            lane_odd<E>(msgs, eccs, status, D, syn, s_co, cw0, __ballot(valid && odd));
+            return;
+        }
         // 65536 does not fit the stored u16 and 32640 not the limbs: another multiple then
         int32_t v[T];
         for (int tries = 0;; ++tries) {
@@ -2578,13 +2600,11 @@ __global__ __launch_bounds__(64, 4) void rsi16_repair_lane_kernel(uint16_t *__re
         uint16_t *at = pos < D.k ? msgs + row * D.k + pos : eccs + row * E + (pos - D.k);
         *at = (uint16_t)(F::add((uint32_t)*at, err) & 0xffff);
     }
-    if (valid) {
-        if (odd)
-            list[1 + atomicAdd(list, 1u)] = cw;
-        else
-            status[cw] = clean ? FFRS_RSI16_NO_ERRORS
-                               : s_found[lane] ? FFRS_RSI16_REPAIR_OK : FFRS_RSI16_ERROR_LOCATION_FAIL;
-    }
+    if (valid && !odd)
+        status[cw] = clean ? FFRS_RSI16_NO_ERRORS
+                           : s_found[lane] ? FFRS_RSI16_REPAIR_OK : FFRS_RSI16_ERROR_LOCATION_FAIL;
+    wave_sync();
+    lane_odd<E>(msgs, eccs, status, D, syn, s_co, cw0, __ballot(valid && odd));
 }
 
 // Transient statuses for ecc_len >= 64: listed codewords, and those with a record for the root search.
@@ -2606,7 +2626,7 @@ __device__ inline void repair_listed(uint16_t *msgs, uint16_t *eccs, uint8_t *st
         const uint32_t cw = list[1 + i];
         uint16_t *m = msgs + (size_t)cw * T.k, *e = eccs + (size_t)cw * E;
         const uint32_t *row = syn + (size_t)cw * E;
-        if (E >= 64 && status[cw] == ODD_SOLVED) {  // rsi16_solve_wave_kernel left locator and evaluator
+        if (status[cw] == ODD_SOLVED) {  // rsi16_solve_wave_kernel left locator and evaluator
             const uint16_t *ev = reinterpret_cast<const uint16_t *>(row), *lo = ev + E;
             const uint32_t inv0 = T.inv_tab[lo[0]];
             PR<E> loc, syn_;
@@ -2622,16 +2642,6 @@ __device__ inline void repair_listed(uint16_t *msgs, uint16_t *eccs, uint8_t *st
         }
         wave_sync();
     }
-}
-
-template <int E>
-__global__ __launch_bounds__(64) void rsi16_repair_list_kernel(uint16_t *__restrict__ msgs, uint16_t *__restrict__ eccs,
-                                                               uint8_t *__restrict__ status, Rsi16Dev T,
-                                                               const uint32_t *__restrict__ syn,
-                                                               const uint32_t *__restrict__ list)
-{
-    __shared__ uint32_t s_mem[REG_WORDS * E];
-    repair_listed<E>(msgs, eccs, status, T, syn, list, s_mem, blockIdx.x, gridDim.x);
 }
 
 // ---------------------------------------------------------------- repair, one wave per key equation
@@ -4377,9 +4387,12 @@ int launch_repair_reg(ffrs_rsi16 *rs, uint16_t *d_msg, uint16_t *d_ecc, size_t c
     // One codeword per wave, its groups sharing the chunks, while the chip takes the waves in a few
     // rounds: the longer the block, the more of them the general kernel's serial chunks cost (us, this
     // / best other: RSi16(64,16) 512 codewords 16 / 16, 2,048 21 / 16; (256,32) 2,048 29 / 36, 4,096
-    // 46 / 36; (1024,16) 8,192 52 / 55, 16,384 92 / 71; (2048,32) 4,096 66 / 75, 8,192 108 / 93).
+    // 46 / 36; (1024,16) 4,096 33 / 46, 8,192 51 / 48 and clean 18 / 13; (4096,16) 6,000 99 / 130, 8,192
+    // 124 / 132 and clean 61 / 31; (16384,16) 8,192 418 / 590 and clean 228 / 130; (2048,32) 4,096 65 / 75,
+    // 8,192 108 / 77).
+    const size_t one = (E == 32 ? 16 : E == 16 && rs->n <= 4096 ? 24 : 32) * cus;
     if constexpr (E <= 32)
-    if (rs->repair_synd == 0 && count <= std::min<size_t>((E == 32 ? 16 : 32) * cus, cus / 2 * rs->n / E)) {
+    if (rs->repair_synd == 0 && count <= std::min<size_t>(one, cus / 2 * rs->n / E)) {
         hipLaunchKernelGGL(rsi16_repair_one_kernel<E>, dim3((unsigned)count), dim3(64), 0, rs->ctx->stream, d_msg, d_ecc,
                            d_status, rs->dev);
         FFRS_HIP(hipGetLastError());
@@ -4387,16 +4400,17 @@ int launch_repair_reg(ffrs_rsi16 *rs, uint16_t *d_msg, uint16_t *d_ecc, size_t c
         return FFRS_OK;
     }
     // The syndromes on the matrix cores first, where their tables exist. For ecc_len 8 to 32 then one
-    // codeword per lane from the counts on where 64 codewords a wave fill the chip and three launches
-    // pay (us, lane / best other: RSi16(64,8) 16,384 codewords 18 / 17, 24,576 18 / 20; (256,8) 8,192
-    // 22 / 27; (1024,16) 16,384 80 / 71, 24,576 79 / 87; (2608,16) 16,384 125 / 134; (256,32) 8,192
-    // 61 / 47, 16,384 64 / 74; 65,536 100 / 161; (32,16) 24,576 29 / 25).
-    const bool lanes = rs->repair_synd == 2 ||
-                       (count * rs->n > ((size_t)1 << 20) &&
-                        (E == 8 || (rs->n >= 2048 ? count > 32 * cus : count >= (E == 16 ? 80 : 64) * cus)));
+    // codeword per lane from the counts on where 64 codewords a wave fill the chip and a second launch
+    // pays (us, lane / best other: RSi16(64,8) 16,384 codewords 14 / 15, clean 8.2 / 6.8, 30,000 15 / 18; (256,8)
+    // 8,192 19 / 30; (64,16) 16,384 19 / 19, 20,000 19 / 23; (256,16) 6,000 23 / 24, 12,000 24 / 28; (1024,16)
+    // 12,000 49 / 55; (256,32) 8,192 39 / 34, 12,000 40 / 43; (512,32) 12,000 53 / 49, 20,000 58 / 81;
+    // (1024,32) 12,000 86 / 64, 16,384 88 / 84, 20,000 90 / 96; (2048,32) 8,192 102 / 77, 12,000 103 / 109).
+    const size_t from = E == 16 ? one + 1
+                                : (rs->n >= 2048 ? 33 : rs->n >= 512 ? 72 : rs->n >= 256 ? 44 : 64) * cus;
+    const bool lanes =
+        rs->repair_synd == 2 || (count * rs->n > ((size_t)1 << 20) && (E == 8 || count >= from));
     // Else the general kernel, given the syndromes where the block has chunks enough for that to pay
-    // (us, given / not: (2608,16) 8,192 codewords 120 / 163, (512,32) 8,192 43 / 48, (1024,32) 16,384
-    // 88 / 113; (256,32) 4,096 39 / 36, (64,16) 4,096 19 / 17).
+    // (us, given / not: (512,32) 8,192 codewords 40 / 45, (1024,32) 12,000 64 / 83; (256,32) 4,096 39 / 36).
     const bool given = E <= 32 && !lanes && rs->n >= 16 * E;
     // ecc_len 128, a few codewords: one launch instead of three, each about 10 us in a call with nothing
     // queued behind it (one RSi16(896,128) encode and repair through the host, one launch / three: clean
@@ -4433,11 +4447,8 @@ int launch_repair_reg(ffrs_rsi16 *rs, uint16_t *d_msg, uint16_t *d_ecc, size_t c
                                    (const uint32_t *)syn);
             } else if constexpr (E >= 8 && E <= 32) {
                 hipLaunchKernelGGL(rsi16_repair_lane_kernel<E>, dim3((unsigned)((c + 63) / 64)), dim3(64), 0,
-                                   rs->ctx->stream, m, e, (uint32_t)c, d_status + b, rs->dev, rs->roots.dev, syn, list);
-                FFRS_HIP(hipGetLastError());
-                mark_kernel(rs->ctx);
-                hipLaunchKernelGGL(rsi16_repair_list_kernel<E>, dim3((unsigned)std::min<size_t>(1024, c)), dim3(64), 0,
-                                   rs->ctx->stream, m, e, d_status + b, rs->dev, syn, list);
+                                   rs->ctx->stream, m, e, (uint32_t)c, d_status + b, rs->dev, rs->roots.dev,
+                                   (const uint32_t *)syn);
             } else if constexpr (E >= 64) {
                 hipLaunchKernelGGL(rsi16_solve_wave_kernel<E>, dim3((unsigned)c), dim3(64), 0, rs->ctx->stream,
                                    (uint32_t)c, d_status + b, rs->dev, rs->roots.dev.pow3, syn, list);
