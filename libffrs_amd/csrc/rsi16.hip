@@ -1305,8 +1305,10 @@ __device__ inline bool pr_poly_div(const Rsi16Dev &T, const PR<E> &f, uint32_t f
 
 // RSi16v<1>::_sugiyama (rsi16v_impl.hpp:271-440) in coefficient form, as sugiyama: r1 holds
 // the syndromes on entry and the normalised evaluator on exit. Returns the locator length,
-// or 0xFFFFFFFF where the reference raises.
-template <int E, class LR>
+// or 0xFFFFFFFF where the reference raises. COEF: zero and three-term quotients in coefficient form too; the
+// plan kernels (and ecc_len below 8, which has none) leave these rare steps to the transforms, as their
+// registers and 3 KB of code cost every codeword.
+template <int E, bool COEF, class LR>
 __device__ inline uint32_t pr_sugiyama(const Rsi16Dev &T, PR<E> &a1, PR<E> &r1, const LR &L)
 {
     constexpr uint32_t G = RegShape<E>::G, mask = E - 1;
@@ -1406,13 +1408,13 @@ __device__ inline uint32_t pr_sugiyama(const Rsi16Dev &T, PR<E> &a1, PR<E> &r1, 
                     t.v[h] = F::fold3(a2.v[h], F::part(n0, a1.v[h]), F::part(n1, pa.v[h]));
                     rn.v[h] = F::fold3(r2.v[h], F::part(n0, r1.v[h]), F::part(n1, pr.v[h]));
                 }
-            } else if (f_len < g_len) {  // a zero quotient: the pair changes places
+            } else if (COEF && f_len < g_len) {  // a zero quotient: the pair changes places
                 h1 = r1h;
                 carried = false;
                 q_len = 0;
                 t = a2;
                 rn = r2;
-            } else if (E >= 8 && f_len == g_len + 2) {
+            } else if (COEF && f_len == g_len + 2) {
                 // q_len == 3 (g_len <= E - 2): the same in coefficients. reverse_ntt gives v[j] =
                 // r1[g_len - 1 - j mod E]; the Newton loop's one round a = a0 + c1 x with
                 // c1 = -a0^2 v[1] (v[0] = r1h = 1 / a0), and the last one coefficients 0 .. 2 of
@@ -1512,7 +1514,7 @@ __device__ inline void repair_finish_reg(const Rsi16Dev &T, uint16_t *m, uint16_
 
 // WAVE: the 64 / G groups of the wave serve one codeword: they take the chunks of the syndromes and
 // of the root search in turn and the roots by lane, and solve the key equation each for itself.
-template <int E, bool SIN = false, bool WAVE = false, class LR>
+template <int E, bool SIN = false, bool WAVE = false, bool COEF = (E >= 8), class LR>
 __device__ inline void repair_group_reg(const Rsi16Dev &T, uint16_t *m, uint16_t *e, uint32_t *base, const LR &L,
                                         uint8_t *st, const uint32_t *syn_in = nullptr)
 {
@@ -1570,7 +1572,7 @@ __device__ inline void repair_group_reg(const Rsi16Dev &T, uint16_t *m, uint16_t
         return;
     }
     PR<E> loc;
-    const uint32_t Ln = pr_sugiyama<E>(T, loc, syn, L);
+    const uint32_t Ln = pr_sugiyama<E, COEF>(T, loc, syn, L);
     if (Ln == 0xffffffffu) {
         if (first == 0)
             *st = FFRS_RSI16_RAISES;
@@ -4090,8 +4092,8 @@ __global__ __launch_bounds__(64) void rsi16_plan_kernel(uint16_t *__restrict__ m
                 const Rsi16PlanItem it = items[ch.first + grp];
                 LaneR<E> L;
                 L.init(cl.T, threadIdx.x);
-                repair_group_reg<E>(cl.T, msgs + it.msg_off, eccs + it.ecc_off, s_mem + grp * REG_WORDS * E, L,
-                                    status + it.idx);
+                repair_group_reg<E, false, false, false>(cl.T, msgs + it.msg_off, eccs + it.ecc_off,
+                                                         s_mem + grp * REG_WORDS * E, L, status + it.idx);
             }
         } else if constexpr (E > 32) {  // encode, the register code of rsi16_encode_reg_kernel<E>
             using O = typename std::conditional<MODE == 0, VectorOps, ScalarOps>::type;

@@ -84,3 +84,39 @@ def test_remainder_of_half_the_parity_found_word():
         b.free()
     codec.close()
     ctx.close()
+
+
+def test_plan_with_irregular_words():
+    """The plan kernels, which leave irregular steps to the transforms, on the same words."""
+    from libffrs_amd import capi
+    codes = [(16, 8), (64, 16), (256, 32), (128, 64), (256, 128), (512, 256)]
+    ws, wants, sts, shape = [], [], [], []
+    for n, ecc in codes:
+        o = O.RSi16(n, ecc)
+        base = np.array([w for _, _, w in Words(o).drops(np.random.default_rng(7 * n + ecc))])
+        wm, we = np.ascontiguousarray(base[:, :n - ecc]), np.ascontiguousarray(base[:, n - ecc:])
+        st = o.repair_batch(wm, we)
+        for i in np.nonzero(st != 255)[0]:
+            ws.append(base[i])
+            wants.append(np.r_[wm[i], we[i]])
+            sts.append(st[i])
+            shape.append((n, ecc))
+    print(f"plan of {len(ws)} irregular words", flush=True)
+    n, ecc = np.array(shape).T
+    k = n - ecc
+    mo, eo = np.r_[0, np.cumsum(k)], np.r_[0, np.cumsum(ecc)]
+    ctx = capi.Context(0)
+    plan = capi.RSi16Plan(ctx, n, ecc, mo[:-1], eo[:-1])
+    d_m, d_e, d_s = ctx.alloc(2 * int(mo[-1])), ctx.alloc(2 * int(eo[-1])), ctx.alloc(len(ws))
+    d_m.upload(np.concatenate([w[:a] for w, a in zip(ws, k)]))
+    d_e.upload(np.concatenate([w[a:] for w, a in zip(ws, k)]))
+    plan.repair(d_m, d_e, d_s)
+    m, e, st = np.empty(int(mo[-1]), np.uint16), np.empty(int(eo[-1]), np.uint16), np.empty(len(ws), np.uint8)
+    for b, a in zip((d_m, d_e, d_s), (m, e, st)):
+        b.download(a)
+        b.free()
+    plan.close()
+    ctx.close()
+    bad = [i for i, w in enumerate(wants) if st[i] != sts[i] or
+           not np.array_equal(np.r_[m[mo[i]:mo[i + 1]], e[eo[i]:eo[i + 1]]], w)]
+    assert not bad, [(shape[i], st[i], sts[i]) for i in bad[:8]]
