@@ -323,7 +323,7 @@ def run_plain(name, args):
     else:
         # the int8 MFMA contraction where it applies (these shapes have no mix constant of 65536; few codewords of
         # ecc 128 and 256 keep the butterflies), ahead of the key equation and the root search too
-        mfma = ecc in (8, 16, 32, 64, 128, 256) and k <= 16384 and N > {256: 1024, 128: 16}.get(ecc, 0)
+        mfma = ecc in (8, 16, 32, 64, 128, 256) and 8 < k <= 16384 and N > {256: 1024, 128: 16}.get(ecc, 0)
         contract = "rsi16_contract_wave_kernel" if ecc <= 32 else "rsi16_contract_kernel"
         enc_names = [contract + " (parity)" if mfma else
                      "rsi16_encode_lane_kernel" if ecc <= 32 else

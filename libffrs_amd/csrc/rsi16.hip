@@ -4305,9 +4305,11 @@ int launch_encode(ffrs_rsi16 *rs, const uint16_t *d_msg, size_t count, uint16_t 
     // codewords of ecc_len 128 or 256, whose matrix (2 bytes an entry) one workgroup takes longer to go through
     // (us, contraction / butterflies: RSi16(4096,256) 64 codewords 32 / 28, 1,024 33 / 29, 4,096
     // 37 / 59; (16384,256) 256 codewords 120 / 98; (896,128) 1,024 10 / 10, one 9 / 9 with warm caches;
-    // (4096,128) 512 codewords 26 / 29).
+    // (4096,128) 512 codewords 26 / 29); nor for RSi16(16,8), whose 8 symbols fill an eighth of a 64-symbol
+    // chunk (1,000,000 codewords 22 / 18; (24,8) 23 / 24).
     const size_t few = rs->E == 256 ? 4 * (size_t)rs->ctx->cu_count : rs->E == 128 ? 16 : 0;
-    if (rs->enc.dev.nq && I == 1 && rs->encode_mode != 1 && (rs->encode_mode == 2 || count > few) &&
+    const bool pays = count > few && rs->k > 8;
+    if (rs->enc.dev.nq && I == 1 && rs->encode_mode != 1 && (rs->encode_mode == 2 || pays) &&
         !(vec && rs->mix_minus_one) && (((uintptr_t)d_msg | (uintptr_t)d_ecc) & 15) == 0)
         return launch_encode_mfma(rs, d_msg, count, d_ecc);
     // one lane per codeword (g = 1): the register kernel for ecc_len <= 32, plain layout
