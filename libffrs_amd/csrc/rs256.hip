@@ -1465,13 +1465,12 @@ __device__ inline void xor_byte(uint8_t *p, uint32_t v)
 }
 
 // ======================================================================
-// Chien search and Forney, G = 16 or 8 lanes per codeword (records of the BM kernels, L <= 16;
-// reed_solomon.hpp:516-538, 704-743). With G = 16, lane j of a group holds positions
-// 16j .. 16j+15 of its codeword as the sixteen bytes of four dwords; with G = 8, 32 positions
-// in eight dwords (16j .. 16j+15 and 128+16j .. 128+16j+15). For a coefficient Lambda_i
-// (i = 1..16) with nibbles v_0, v_1, a 16-byte read of row CT[i][h][v_h] per nibble and piece
-// gives (v_h << 4h) alpha^(-ip) at sixteen of the lane's positions, so a wave evaluates 64 / G
-// codewords per pass with no value read across lanes. A 64-codeword tile is taken in ascending
+// Chien search and Forney, eight lanes per codeword (L <= 16; reed_solomon.hpp:516-538, 704-743).
+// Lane j of a group holds 32 positions of its codeword in eight dwords (16j .. 16j+15 and
+// 128+16j .. 128+16j+15). For a coefficient Lambda_i (i = 1..16) with nibbles v_0, v_1, two 16-byte
+// reads of row CT[i][h][v_h] per nibble give (v_h << 4h) alpha^(-ip) at the lane's positions, so a
+// wave evaluates eight codewords per pass with no value read across lanes (sixteen lanes and four
+// codewords were slower at every ecc measured). A 64-codeword tile is taken in ascending
 // L (the codewords of a pass have nearly the same degree and the pass stops at the largest).
 // Where the zeros among positions [0, n) number exactly L, the pass's roots are listed one per
 // slot in LDS, and each lane
@@ -1500,14 +1499,12 @@ __device__ inline void record_nibbles(const uint32_t (&r)[12], uint32_t (&nib)[8
 }
 
 // acc ^= sum over coefficients i = 1..top (top <= IMAX, wave-uniform) of Lambda_i alpha^(-ip) at
-// the lane's positions, odd coefficients into acc_odd when SPLIT. D = 4: sixteen positions, one
-// 16-byte read per nibble at `off`; D = 8: thirty-two, a second read at off ^ 128 (the other
-// half of the 256-byte row).
-template <bool SPLIT, int IMAX, int D>
+// the lane's thirty-two positions, odd coefficients into acc_odd when SPLIT: per nibble a 16-byte
+// read at `off` and one at off ^ 128 (the other half of the 256-byte row).
+template <bool SPLIT, int IMAX>
 __device__ inline void chien_eval(const char *ct, const uint32_t (&nib)[8], uint32_t lo_off, uint32_t hi_off,
-                                  uint32_t top, uint32_t (&acc)[D], uint32_t (&acc_odd)[D])
+                                  uint32_t top, uint32_t (&acc)[8], uint32_t (&acc_odd)[8])
 {
-    static_assert(D == 4 || D == 8, "16 or 32 positions per lane");
 #pragma unroll
     for (int gq = 0; gq < 4; ++gq) {
         if (4 * gq + 1 > (int)top)
@@ -1518,19 +1515,18 @@ __device__ inline void chien_eval(const char *ct, const uint32_t (&nib)[8], uint
             if (i > IMAX)
                 break;
             const uint32_t word = nib[2 * gq + (jj >> 1)];
-            uint4 t[2][D / 4];
+            uint4 t[2][2];
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
                 const int tbl = (i - 1) * 2 + h;  // 4 KB table index
                 const uint32_t sel = 0x0c020000u | ((4u + (uint32_t)(2 * (jj & 1) + h)) << 8);
                 const uint32_t a = __builtin_amdgcn_perm(word, tbl >= 16 ? hi_off : lo_off, sel);
                 t[h][0] = *reinterpret_cast<const uint4 *>(ct + a + (tbl & 15) * 4096);
-                if constexpr (D == 8)
-                    t[h][1] = *reinterpret_cast<const uint4 *>(ct + (a ^ 128u) + (tbl & 15) * 4096);
+                t[h][1] = *reinterpret_cast<const uint4 *>(ct + (a ^ 128u) + (tbl & 15) * 4096);
             }
-            uint32_t(&d)[D] = (SPLIT && (i & 1)) ? acc_odd : acc;
+            uint32_t(&d)[8] = (SPLIT && (i & 1)) ? acc_odd : acc;
 #pragma unroll
-            for (int r = 0; r < D / 4; ++r) {
+            for (int r = 0; r < 2; ++r) {
                 d[4 * r + 0] = xor3(d[4 * r + 0], t[0][r].x, t[1][r].x);
                 d[4 * r + 1] = xor3(d[4 * r + 1], t[0][r].y, t[1][r].y);
                 d[4 * r + 2] = xor3(d[4 * r + 2], t[0][r].z, t[1][r].z);
@@ -1540,28 +1536,20 @@ __device__ inline void chien_eval(const char *ct, const uint32_t (&nib)[8], uint
     }
 }
 
-// Position of byte q of position dword d of lane j in codeword group grp: G = 16 lanes hold 16
-// consecutive positions each; G = 8 lanes hold two runs of 16, one in each half of the
-// codeword, the half of dwords 0-3 alternating with the group so that one read instruction of
-// the eight groups covers all 64 LDS banks.
-template <int G>
+// Position of byte q of position dword d of lane j in codeword group grp: two runs of 16, one in
+// each half of the codeword, the half of dwords 0-3 alternating with the group so that one read
+// instruction of the eight groups covers all 64 LDS banks.
 __device__ inline uint32_t chien_pos(uint32_t j, uint32_t grp, int d, int q)
 {
-    if constexpr (G == 16)
-        return 16 * j + 4 * (uint32_t)d + (uint32_t)q;
-    else
-        return 128 * (((uint32_t)d >> 2) ^ (grp & 1u)) + 16 * j + 4 * ((uint32_t)d & 3u) + (uint32_t)q;
+    return 128 * (((uint32_t)d >> 2) ^ (grp & 1u)) + 16 * j + 4 * ((uint32_t)d & 3u) + (uint32_t)q;
 }
 
-// Sum over the G lanes of this lane's codeword group (DPP butterflies), in every lane of it.
-template <int G>
+// Sum over the eight lanes of this lane's codeword group (DPP butterflies), in every lane of it.
 __device__ inline uint32_t group_sum(uint32_t x)
 {
     x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0xB1, 0xF, 0xF, false);   // quad_perm [1,0,3,2]
     x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x4E, 0xF, 0xF, false);   // quad_perm [2,3,0,1]
     x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x141, 0xF, 0xF, false);  // row_half_mirror
-    if constexpr (G == 16)
-        x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x140, 0xF, 0xF, false);  // row_mirror
     return x;
 }
 
@@ -1576,10 +1564,8 @@ __device__ inline void wave_lds_sync()
 // The BM records come from bm_fixed_one<EB> run per tile, one pending codeword per lane, on the
 // syndromes `synd` (its LDS lookups overlap the Chien loops of other waves); ecc_len is at most EB. A BM
 // kernel of its own, with records in HBM, took 56 us and this kernel 34 for 100,003 codewords of
-// ecc 21; together 43. G lanes per codeword in the Chien passes: 16 (sixteen positions each, four
-// codewords per pass) or 8 (thirty-two each, eight per pass: half the per-pass work per
-// codeword, for small ecc where that work dominates).
-template <int WG, int EB, int G = 8>
+// ecc 21; together 43.
+template <int WG, int EB>
 __global__ __launch_bounds__(WG) void rs256_chien16_kernel(uint8_t *__restrict__ msgs, uint8_t *__restrict__ eccs,
                                                             uint32_t count, uint32_t k, uint32_t E,
                                                             uint8_t *__restrict__ status,
@@ -1591,13 +1577,12 @@ __global__ __launch_bounds__(WG) void rs256_chien16_kernel(uint8_t *__restrict__
     __shared__ uint4 s_ct4[CHIEN_TABLE_BYTES / 16];
     __shared__ uint8_t s_exp2[EXP2_LEN];
     __shared__ uint16_t s_log2[256];
-    static_assert(G == 16 || G == 8, "16 or 8 lanes per codeword");
     // L <= EB / 2: only the nibble words of coefficients 1 .. EB / 2 travel between lanes and only
     // that many degrees are ranked
     constexpr int LMX = EB / 2;
     constexpr int NW = EB >= 8 ? EB / 4 : 1;
     constexpr int EWS = EB <= 4 ? 1 : EB <= 8 ? 2 : EB <= 16 ? 4 : 8;  // syndrome dwords per codeword
-    constexpr int D = 64 / G;               // position dwords per lane, and codewords per pass
+    constexpr int G = 8, D = 8;  // lanes per codeword; position dwords per lane, and codewords per pass
     constexpr int RS = D * LMX + 64;  // root slots per wave (a pass has <= D LMX roots, 63 wait)
     __shared__ uint32_t s_roots[WG / 64 * RS];
     for (uint32_t i = threadIdx.x; i < CHIEN_TABLE_BYTES / 16; i += WG)
@@ -1613,7 +1598,7 @@ __global__ __launch_bounds__(WG) void rs256_chien16_kernel(uint8_t *__restrict__
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t n = k + E;
     // byte offset of the lane's first 16-byte piece within a table row
-    const uint32_t lo_off = 16 * j + (G == 8 ? 128 * (grp & 1u) : 0u), hi_off = lo_off + 0x10000u;
+    const uint32_t lo_off = 16 * j + 128 * (grp & 1u), hi_off = lo_off + 0x10000u;
     uint32_t *s_rt = s_roots + RS * wave;
     for (uint32_t base = (blockIdx.x * (WG / 64) + wave) * 64; base < count; base += gridDim.x * WG) {
         const uint32_t cw = base + lane;
@@ -1638,7 +1623,7 @@ __global__ __launch_bounds__(WG) void rs256_chien16_kernel(uint8_t *__restrict__
             vmask[d] = 0;
 #pragma unroll
             for (int q = 0; q < 4; ++q)
-                vmask[d] |= (chien_pos<G>(j, grp, d, q) < n) ? (0x80u << (8 * q)) : 0u;
+                vmask[d] |= (chien_pos(j, grp, d, q) < n) ? (0x80u << (8 * q)) : 0u;
         }
         uint32_t lnib[8];
         record_nibbles<20>(r, lnib);  // Lambda_1..Lambda_16 (Lambda_0 = 1 at byte 20)
@@ -1729,7 +1714,7 @@ __global__ __launch_bounds__(WG) void rs256_chien16_kernel(uint8_t *__restrict__
                 ev[d] = 0x01010101u;  // Lambda_0 = 1
                 od[d] = 0;
             }
-            chien_eval<true, LMX, D>(ct, ln, lo_off, hi_off, Lmax, ev, od);
+            chien_eval<true, LMX>(ct, ln, lo_off, hi_off, Lmax, ev, od);
             uint32_t z[D], cnt = 0;
 #pragma unroll
             for (int d = 0; d < D; ++d) {
@@ -1738,7 +1723,7 @@ __global__ __launch_bounds__(WG) void rs256_chien16_kernel(uint8_t *__restrict__
                 z[d] = __builtin_amdgcn_bitop3_b32(t, v, vmask[d], 0x02);  // ~t & ~v & mask: zero bytes
                 cnt += (uint32_t)__builtin_popcount(z[d]);
             }
-            cnt = group_sum<G>(cnt);
+            cnt = group_sum(cnt);
             const bool ok = active && cnt == Lg;
             if (j == 0 && active)
                 status[base + o] = ok ? 1 : 0;
@@ -1755,7 +1740,7 @@ __global__ __launch_bounds__(WG) void rs256_chien16_kernel(uint8_t *__restrict__
             const uint32_t nr = (uint32_t)__builtin_popcount(rm);
             uint32_t slot = waiting, total = 0;  // exclusive prefix sum of nr (<= 4 D) by bit planes
 #pragma unroll
-            for (int b = 0; b < (D == 8 ? 6 : 5); ++b) {
+            for (int b = 0; b < 6; ++b) {
                 const uint64_t m = __ballot((nr >> b) & 1u);
                 slot += __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u)) << b;
                 total += (uint32_t)__builtin_popcountll(m) << b;
@@ -1764,11 +1749,11 @@ __global__ __launch_bounds__(WG) void rs256_chien16_kernel(uint8_t *__restrict__
                 const uint32_t t = (uint32_t)__builtin_ctz(rm);
                 rm &= rm - 1;
                 const uint32_t q = t >> 3, d = t & 7u;
-                uint32_t ov = od[0], p = chien_pos<G>(j, grp, 0, 0) + q;
+                uint32_t ov = od[0], p = chien_pos(j, grp, 0, 0) + q;
 #pragma unroll
                 for (int dd = 1; dd < D; ++dd) {
                     ov = d == (uint32_t)dd ? od[dd] : ov;
-                    p = d == (uint32_t)dd ? chien_pos<G>(j, grp, dd, 0) + q : p;
+                    p = d == (uint32_t)dd ? chien_pos(j, grp, dd, 0) + q : p;
                 }
                 s_rt[slot++] = o | (p << 8) | (((ov >> (8 * q)) & 0xffu) << 16);
             }
