@@ -2058,8 +2058,9 @@ __device__ inline void contract_store(const v4i_t acc[2], const MfmaTab &M, uint
 }
 
 // ecc_len 8 (half a tile of output rows), 16 and 32: a wave takes CG groups of 16 codewords and every output tile; the matrix
-// (a few KB per chunk) comes from the caches. Bound by the codewords' HBM reads (rows of a few
-// hundred bytes): 262,144 RSi16(256,32) parities in 36 us (3.7 TB/s), 39 with three 7-bit limbs.
+// (a few KB per chunk) comes from the caches. Bound by the loads in flight at 10 waves a CU: 262,144
+// RSi16(256,32) parities in 36 us, with the 134 MB they cannot do without from HBM (3.7 TB/s), twice
+// that of the matrix from L2 and the matrix cores 10 % busy; 39 us with three 7-bit limbs.
 template <int E, int CG, int D, bool SYN>
 __global__ __launch_bounds__(256) void rsi16_contract_wave_kernel(const uint16_t *__restrict__ msgs, uint32_t msg_bytes,
                                                                   const uint16_t *__restrict__ eccs, uint32_t ecc_bytes,
@@ -2235,8 +2236,10 @@ __global__ __launch_bounds__(NW * 64) void rsi16_contract_kernel(const uint16_t 
 // coefficients keep what they hold. A codeword whose remainder drops by more than one degree and still
 // has E / 2 or more, or that meets one of the other cases listed at check() and solve(), goes to the
 // general code (lane_odd): about 17 in 65,537 damaged codewords.
-// A wave of clean codewords stops after the key equation. Bound by the vector units (a wave's
-// 9,000 instructions, 80 % of the issue slots): a third of them the key equation's steps, the rest
+// A wave of clean codewords stops after the key equation. 262,144 RSi16(256,32) repairs with 0-16
+// errors: 53 us of syndromes and 104 here, against 402 + 52 with a codeword per sixteen lanes (start
+// to end 191 us, 487 then, with the restoring copies). Bound by the vector units (a wave's 9,900
+// instructions, 80 % of the issue slots): a third of them the key equation's steps, the rest
 // the root search's epilogues, Forney and the conversions between.
 //
 // Values are held as b = (v + 32768) mod p in [-1, 65536] (zero is 32768 alone), v = b - 32768 in
