@@ -2237,10 +2237,9 @@ __global__ __launch_bounds__(NW * 64) void rsi16_contract_kernel(const uint16_t 
 // has E / 2 or more, or that meets one of the other cases listed at check() and solve(), goes to the
 // general code (lane_odd): about 17 in 65,537 damaged codewords.
 // A wave of clean codewords stops after the key equation. 262,144 RSi16(256,32) repairs with 0-16
-// errors: 53 us of syndromes and 104 here, against 402 + 52 with a codeword per sixteen lanes (start
-// to end 191 us, 487 then, with the restoring copies). Bound by the vector units (a wave's 9,900
-// instructions, 80 % of the issue slots): a third of them the key equation's steps, the rest
-// the root search's epilogues, Forney and the conversions between.
+// errors: 53 us of syndromes and 104 here, against 52 + 402 with a codeword per sixteen lanes. Bound
+// by the vector units (a wave's 9,900 instructions, 80 % of the issue slots): a third of them the key
+// equation's steps, the rest the root search's epilogues, Forney and the conversions between.
 //
 // Values are held as b = (v + 32768) mod p in [-1, 65536] (zero is 32768 alone), v = b - 32768 in
 // [-32769, 32768]: a remainder coefficient c2 + n0 c1 + n1 c1' is then
