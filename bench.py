@@ -334,6 +334,7 @@ def run_plain(name, args):
                      [contract + " (syndromes)", "rsi16_repair_lane_kernel" if N > 18432 else "rsi16_repair_reg_kernel"]
                      if nk == 2 else
                      ["rsi16_repair_one_kernel" if ecc <= 32 and one else
+                      "rsi16_repair_few_kernel" if ecc in (64, 128, 256) and k <= 16384 else
                       "rsi16_repair_reg_kernel" if ecc <= 256 else "rsi16_repair_kernel"])
     ke_ms = np.mean(np.array(kes), axis=0)
     kr_ms = np.mean(np.array(krs), axis=0)

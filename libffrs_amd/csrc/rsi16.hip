@@ -1512,32 +1512,25 @@ template <int E, bool WAVE, class LR>
 __device__ inline void repair_finish_reg(const Rsi16Dev &T, uint16_t *m, uint16_t *e, uint32_t *base, const LR &L,
                                          uint8_t *st, const PR<E> &loc, const PR<E> &syn, uint32_t Ln);
 
-// WAVE: the 64 / G groups of the wave serve one codeword: they take the chunks of the syndromes and
-// of the root search in turn and the roots by lane, and solve the key equation each for itself.
-template <int E, bool SIN = false, bool WAVE = false, bool COEF = (E >= 8), class LR>
-__device__ inline void repair_group_reg(const Rsi16Dev &T, uint16_t *m, uint16_t *e, uint32_t *base, const LR &L,
-                                        uint8_t *st, const uint32_t *syn_in = nullptr)
+// WAVE, here and below: the 64 / G groups of the wave serve one codeword: they take the chunks of the syndromes
+// and of the root search in turn and the roots by lane, and solve the key equation each for itself.
+
+// NTT::pntt (ntt.hpp:133-152) of m || e, one chunk of E symbols at a time; the symbols and shifts of PF chunks
+// are loaded before any is transformed, so their latencies overlap.
+template <int E, bool WAVE, class LR>
+__device__ inline PR<E> synd_reg(const Rsi16Dev &T, const uint16_t *m, const uint16_t *e, const LR &L)
 {
     constexpr uint32_t G = RegShape<E>::G;
     constexpr int C = RegShape<E>::C;
     constexpr uint32_t NG = WAVE ? 64 / G : 1;             // groups on the codeword
-    const uint32_t gi = WAVE ? L.lane / G : 0;             // this group
-    const uint32_t first = WAVE ? L.lane : L.gl;           // this lane among theirs
-    // NTT::pntt (ntt.hpp:133-152) of m || e, one chunk of E symbols at a time; the symbols
-    // and shifts of PF chunks are loaded before any is transformed, so their latencies overlap
     constexpr uint32_t PF = C >= 4 ? 1 : 4;
+    const uint32_t gi = WAVE ? L.lane / G : 0, nb = T.n / E;
     PR<E> syn;
-    const uint32_t nb = T.n / E;
-    if constexpr (SIN) {  // syndromes computed ahead (rsi16_contract_kernel)
-#pragma unroll
-        for (int h = 0; h < C; ++h)
-            syn.v[h] = syn_in[L.gl + (uint32_t)h * G];
-    }
-    if constexpr (!SIN && WAVE)
+    if constexpr (WAVE)
 #pragma unroll
         for (int h = 0; h < C; ++h)
             syn.v[h] = 0;
-    for (uint32_t c0 = gi * PF; !SIN && c0 < nb; c0 += NG * PF) {
+    for (uint32_t c0 = gi * PF; c0 < nb; c0 += NG * PF) {
         PR<E> x[PF], sh[PF];
 #pragma unroll
         for (uint32_t u = 0; u < PF; ++u)
@@ -1560,12 +1553,28 @@ __device__ inline void repair_group_reg(const Rsi16Dev &T, uint16_t *m, uint16_t
                 }
             }
     }
-    if constexpr (!SIN && WAVE)
+    if constexpr (WAVE)
 #pragma unroll
         for (uint32_t s = G; s < 64; s <<= 1)
 #pragma unroll
             for (int h = 0; h < C; ++h)
                 syn.v[h] = F::add(syn.v[h], lane_read(syn.v[h], L.lane ^ s));
+    return syn;
+}
+
+template <int E, bool SIN = false, bool WAVE = false, bool COEF = (E >= 8), class LR>
+__device__ inline void repair_group_reg(const Rsi16Dev &T, uint16_t *m, uint16_t *e, uint32_t *base, const LR &L,
+                                        uint8_t *st, const uint32_t *syn_in = nullptr)
+{
+    const uint32_t first = WAVE ? L.lane : L.gl;           // this lane among the codeword's
+    PR<E> syn;
+    if constexpr (SIN) {  // syndromes computed ahead (rsi16_contract_kernel)
+#pragma unroll
+        for (int h = 0; h < RegShape<E>::C; ++h)
+            syn.v[h] = syn_in[L.gl + (uint32_t)h * RegShape<E>::G];
+    } else {
+        syn = synd_reg<E, WAVE>(T, m, e, L);
+    }
     if (pr_len<E>(syn, E, L) == 0) {
         if (first == 0)
             *st = FFRS_RSI16_NO_ERRORS;
@@ -1590,6 +1599,8 @@ __device__ inline void repair_finish_reg(const Rsi16Dev &T, uint16_t *m, uint16_
     constexpr uint32_t G = RegShape<E>::G;
     constexpr int C = RegShape<E>::C;
     constexpr uint32_t PF = C >= 4 ? 1 : 4, NG = WAVE ? 64 / G : 1;
+    // Forney's sums as four chains side by side: alone on its SIMD, a wave waits for each of a chain's products
+    constexpr bool PAIRS = WAVE && E >= 64;
     const uint32_t gi = WAVE ? L.lane / G : 0, first = WAVE ? L.lane : L.gl, nb = T.n / E;
     const uint32_t eval_len = E - Ln + 1;
     // _deriv (rsi16v_impl.hpp:608-616): der[i] = (i + 1) loc[i + 1]
@@ -1612,7 +1623,8 @@ __device__ inline void repair_finish_reg(const Rsi16Dev &T, uint16_t *m, uint16_
     uint32_t *ev = base, *dv = base + E, *list = base + 2 * E, *nroots = base + 3 * E;
 #pragma unroll
     for (int h = 0; h < C; ++h) {
-        ev[L.gl + (uint32_t)h * G] = syn.v[h];
+        // PAIRS reads past the evaluator's last term
+        ev[L.gl + (uint32_t)h * G] = !PAIRS || L.gl + (uint32_t)h * G < emax ? syn.v[h] : 0u;
         dv[L.gl + (uint32_t)h * G] = der.v[h];
     }
     if (first == 0)
@@ -1657,8 +1669,22 @@ __device__ inline void repair_finish_reg(const Rsi16Dev &T, uint16_t *m, uint16_
         const uint32_t ri = rbo_bits(pos, T.nbits);
         const uint32_t x = T.roots_ntt[ri];
         const uint32_t xi = T.roots_ntt[(T.N - ri) & (T.N - 1)];
-        const uint32_t num = eval_poly(ev, emax, xi);
-        const uint32_t den = eval_poly(dv, dmax, xi);
+        uint32_t num, den;
+        if constexpr (PAIRS) {
+            const uint32_t x2 = F::mul(xi, xi);
+            uint32_t n0 = 0, n1 = 0, d0 = 0, d1 = 0;
+            for (uint32_t i = ((emax > dmax ? emax : dmax) + 1) / 2; i-- > 0;) {
+                n0 = F::add(F::mul(n0, x2), ev[2 * i]);
+                n1 = F::add(F::mul(n1, x2), ev[2 * i + 1]);
+                d0 = F::add(F::mul(d0, x2), dv[2 * i]);
+                d1 = F::add(F::mul(d1, x2), dv[2 * i + 1]);
+            }
+            num = F::add(n0, F::mul(n1, xi));
+            den = F::add(d0, F::mul(d1, xi));
+        } else {
+            num = eval_poly(ev, emax, xi);
+            den = eval_poly(dv, dmax, xi);
+        }
         // _forney (rsi16v_impl.hpp:500-512) with the table conventions of g_div
         const uint32_t q = num == 0 ? 0u : (den == 0 ? num : F::mul(num, T.inv_tab[den]));
         const uint32_t err = F::mul(q, x);
@@ -2869,7 +2895,114 @@ struct WaveSolve {
         }
         return true;
     }
+
+    // The key equation of the syndromes in R[0]: evaluator, locator and its constant in R[1], A[1], A0[1]. odd: by
+    // irregular steps; terms: the coefficients that evaluator and locator's derivative may have. False where the
+    // codeword is left to the general code.
+    __device__ bool key_equation(const uint32_t *__restrict__ inv_tab, uint32_t &steps, uint32_t &terms, bool &odd)
+    {
+        steps = solve(inv_tab);
+        terms = steps;
+        bool solved = steps != 0;
+        odd = false;
+        if (steps & 1) {  // the results in R[1], A[1]
+        } else {
+#pragma unroll
+            for (int h = 0; h < C; ++h) {
+                const int32_t v = R[0][h];
+                R[0][h] = R[1][h];
+                R[1][h] = v;
+            }
+#pragma unroll
+            for (int h = 0; h < CA; ++h) {
+                const int32_t v = A[0][h];
+                A[0][h] = A[1][h];
+                A[1][h] = v;
+            }
+            const int32_t v = A0[0];
+            A0[0] = A0[1];
+            A0[1] = v;
+        }
+        if (solved && steps < (uint32_t)T) {
+            const uint32_t len = length(R[1]);
+            odd = len >= (uint32_t)T;
+            if (odd)
+                solved = irregular(steps, E + 1 - steps, len, inv_tab);
+            else
+                solved = len != 0;
+            terms = max(steps, len);
+        }
+        return solved;
+    }
 };
+
+// A few codewords of ecc_len 64 to 256, one per wave in one launch: the syndromes and the root search of the register
+// code around WaveSolve's key equation. Bound by one wave's latency: the chunks one after another, the steps, the
+// terms of Forney's sums. 64 clean RSi16(512,256) codewords 7 us and 60 with 0-128 errors; through contraction, solver
+// and search 13 and 64, with the register code's own key equation 7 and 174.
+template <int E>
+__global__ __launch_bounds__(64) void rsi16_repair_few_kernel(uint16_t *__restrict__ msgs, uint16_t *__restrict__ eccs,
+                                                              uint8_t *__restrict__ status, Rsi16Dev T)
+{
+    using W = WaveSolve<E>;
+    constexpr int C = W::C, CA = W::CA;
+    constexpr uint32_t H = W::T, G = RegShape<E>::G;
+    __shared__ uint32_t s_mem[REG_WORDS * E];
+    const uint32_t cw = blockIdx.x, lane = threadIdx.x;
+    uint16_t *m = msgs + (size_t)cw * T.k, *e = eccs + (size_t)cw * E;
+    LaneR<E, true> L;
+    L.init(T, lane);
+    PR<E> syn = synd_reg<E, true>(T, m, e, L), loc;
+    if (pr_len<E>(syn, E, L) == 0) {
+        if (lane == 0)
+            status[cw] = FFRS_RSI16_NO_ERRORS;
+        return;
+    }
+#pragma unroll
+    for (int h = 0; h < RegShape<E>::C; ++h)
+        s_mem[L.gl + (uint32_t)h * G] = syn.v[h];
+    wave_sync();
+    W S;
+#pragma unroll
+    for (int h = 0; h < C; ++h)
+        S.R[0][h] = fold16((int32_t)s_mem[C * lane + h] + RBIAS);
+    wave_sync();
+    uint32_t steps, terms, Ln;
+    bool odd;
+    const bool solved = S.key_equation(T.inv_tab, steps, terms, odd);
+    const uint32_t a0 = bal_canon(S.A0[1] - RBIAS);
+    if (solved && a0 != 0) {
+        // locator coefficients 0 .. E / 2 and evaluator back to the register code's lanes, normalised
+        for (uint32_t i = H + 1 + lane; i < (uint32_t)E; i += 64)
+            s_mem[i] = 0;
+        if (lane == 0)
+            s_mem[0] = a0;
+#pragma unroll
+        for (int h = 0; h < CA; ++h)
+            if (CA * lane + h < H)
+                s_mem[1 + CA * lane + h] = bal_canon(S.A[1][h] - RBIAS);
+#pragma unroll
+        for (int h = 0; h < C; ++h)
+            s_mem[E + C * lane + h] = bal_canon(S.R[1][h] - RBIAS);
+        wave_sync();
+        const uint32_t inv0 = T.inv_tab[a0];
+#pragma unroll
+        for (int h = 0; h < RegShape<E>::C; ++h) {
+            loc.v[h] = F::mul(s_mem[L.gl + (uint32_t)h * G], inv0);
+            syn.v[h] = F::mul(s_mem[E + L.gl + (uint32_t)h * G], inv0);
+        }
+        wave_sync();
+        Ln = pr_len<E>(loc, E, L);
+    } else {
+        Ln = pr_sugiyama<E, true>(T, loc, syn, L);
+        if (Ln == 0xffffffffu) {
+            if (lane == 0)
+                status[cw] = FFRS_RSI16_RAISES;
+            return;
+        }
+    }
+    repair_finish_reg<E, true>(T, m, e, s_mem, L, status + cw, loc, syn, Ln);
+}
 
 // 16,384 RSi16(4096,256) codewords with 0-128 errors in 190 us (E / 4 + E / 8 coefficients of five
 // vector instructions a step, about 25 more for the quotient); the shuffles, table loads and lengths of
@@ -2896,36 +3029,9 @@ __global__ __launch_bounds__(64) void rsi16_solve_wave_kernel(uint32_t count, ui
             status[cw] = FFRS_RSI16_NO_ERRORS;
         return;
     }
-    uint32_t steps = S.solve(D.inv_tab);
-    uint32_t terms = steps;
-    bool solved = steps != 0, odd = false;
-    if (steps & 1) {  // the results in R[1], A[1]
-    } else {
-#pragma unroll
-        for (int h = 0; h < C; ++h) {
-            const int32_t v = S.R[0][h];
-            S.R[0][h] = S.R[1][h];
-            S.R[1][h] = v;
-        }
-#pragma unroll
-        for (int h = 0; h < CA; ++h) {
-            const int32_t v = S.A[0][h];
-            S.A[0][h] = S.A[1][h];
-            S.A[1][h] = v;
-        }
-        const int32_t v = S.A0[0];
-        S.A0[0] = S.A0[1];
-        S.A0[1] = v;
-    }
-    if (solved && steps < (uint32_t)T) {
-        const uint32_t len = W::length(S.R[1]);
-        odd = len >= (uint32_t)T;
-        if (odd)
-            solved = S.irregular(steps, E + 1 - steps, len, D.inv_tab);
-        else
-            solved = len != 0;
-        terms = max(steps, len);
-    }
+    bool odd;
+    uint32_t steps, terms;
+    bool solved = S.key_equation(D.inv_tab, steps, terms, odd);
     int32_t a0 = S.A0[1] - RBIAS, a[CA], r[C], v[CA], d[CA];
 #pragma unroll
     for (int h = 0; h < CA; ++h)
@@ -4418,12 +4524,25 @@ int launch_repair_reg(ffrs_rsi16 *rs, uint16_t *d_msg, uint16_t *d_ecc, size_t c
     // Else the general kernel, given the syndromes where the block has chunks enough for that to pay
     // (us, given / not: (512,32) 8,192 codewords 40 / 45, (1024,32) 12,000 64 / 83; (256,32) 4,096 39 / 36).
     const bool given = E <= 32 && !lanes && rs->n >= 16 * E;
-    // ecc_len 128, a few codewords: one launch instead of three, each about 10 us in a call with nothing
-    // queued behind it (one RSi16(896,128) encode and repair through the host, one launch / three: clean
-    // 86 / 105 us, 56 errors 137 / 126). At ecc_len 256 the solver's gain is worth them (RSi16(4096,256):
-    // 100 errors 274 / 183, clean 128 / 149).
-    const bool single = E == 128 && rs->repair_synd == 0 && count <= 16;
-    const bool msyn = rs->synd.dev.nq && rs->repair_synd != 1 && ((E >= 64 && !single) || lanes || given) &&
+    // ecc_len 64 to 256, a few codewords: one per wave in one launch, up to where the three launches' kernels repair
+    // damaged ones sooner (us damaged, this / three launches, and clean: RSi16(128,64) 4,096 codewords 30 / 32, 12 /
+    // 14; (512,64) 2,048 24 / 26, 8 / 11, 4,096 35 / 31; (2048,64) 512 36 / 35, 13 / 15; (1024,128) 2,048 45 / 45,
+    // 12 / 15; (2048,128) 1,024 55 / 60, 16 / 20; (4096,128) 16 67 / 63, 25 / 30, 256 71 / 68, 48 / 40; (512,256) 1,024
+    // 72 / 75, 8 / 14, 2,048 79 / 75; (4096,256) 64 106 / 102, 26 / 37, 1,024 130 / 153; (8192,256) 256 152 / 159,
+    // 92 / 98; (16384,256) 64 248 / 242, 89 / 126). One codeword alone is repaired sooner by three launches for long
+    // blocks ((4096,256) 92 / 76), but each of them takes about 10 us in a call with nothing queued behind it.
+    const size_t few = E == 64    ? std::min<size_t>((rs->n <= 2 * E ? 32 : 8) * cus, rs->n <= 2048 ? 4096 * cus / rs->n : 0)
+                       : E == 128 ? (rs->n > 2048 ? 16 : (rs->n <= 2 * E ? 32 : 8) * cus)
+                                  : (rs->n <= 4096 ? 4 : 1) * cus;
+    if constexpr (E >= 64)
+    if (rs->repair_synd == 0 && count <= few) {
+        hipLaunchKernelGGL(rsi16_repair_few_kernel<E>, dim3((unsigned)count), dim3(64), 0, rs->ctx->stream, d_msg, d_ecc,
+                           d_status, rs->dev);
+        FFRS_HIP(hipGetLastError());
+        mark_kernel(rs->ctx);
+        return FFRS_OK;
+    }
+    const bool msyn = rs->synd.dev.nq && rs->repair_synd != 1 && (E >= 64 || lanes || given) &&
                       (((uintptr_t)d_msg | (uintptr_t)d_ecc) & 15) == 0;
     // workspace: E syndromes per codeword and the list of those left to the general kernel, which takes the
     // whole batch where there is no workspace

@@ -71,8 +71,8 @@ def _codec(ctx, n, ecc):
     return capi.RSi16Codec(ctx, n, ecc)
 
 
-@pytest.mark.parametrize("n,ecc,counts", [(64, 8, (30000, 45000)), (256, 32, (20000, 17000)), (128, 64, (700, 900)),
-                                          (256, 128, (300, 3000)), (512, 256, (40, 700))])
+@pytest.mark.parametrize("n,ecc,counts", [(64, 8, (30000, 45000)), (256, 32, (20000, 17000)), (128, 64, (9000, 10000)),
+                                          (256, 128, (8300, 9000)), (512, 256, (1100, 2000))])
 def test_two_threads_on_one_codec(ctx, n, ecc, counts):
     codec = _codec(ctx, n, ecc)
     batches = [Batch(ctx, codec, c, 7 + c) for c in counts]
@@ -105,8 +105,8 @@ def test_two_threads_on_one_codec(ctx, n, ecc, counts):
     codec.close()
 
 
-@pytest.mark.parametrize("n,ecc,small,large", [(64, 8, 30000, 100000), (256, 32, 20000, 50000), (128, 64, 500, 3000),
-                                               (256, 128, 300, 3000), (512, 256, 300, 3000)])
+@pytest.mark.parametrize("n,ecc,small,large", [(64, 8, 30000, 100000), (256, 32, 20000, 50000), (128, 64, 9000, 30000),
+                                               (256, 128, 8300, 20000), (512, 256, 1100, 4000)])
 def test_capture_and_growth(ctx, n, ecc, small, large):
     codec = _codec(ctx, n, ecc)
     first, later = Batch(ctx, codec, small, 11), Batch(ctx, codec, large, 13)
